@@ -332,7 +332,7 @@ int adj_common(sponge_nl* nl, sponge_lj* lj, sponge_pme* pme, const unsigned int
                hipStream_t s) {
     const int n = lj->n;
     const int T = lj->ntypes, P = T * (T + 1) / 2;
-    int rc = snb_lj_scratch(lj, nl);
+    int rc = snb_scratch(&lj->ps, nl);
     if (rc) return rc;
     adj_gather_kernel<<<ceil_div(nl->slot_cap, 256), 256, 0, s>>>(nl->flags, nl->s2o, uc, q, lj->d_type, lj->ps.pk,
                                                                    A->w3, loss ? A->ws : nullptr);

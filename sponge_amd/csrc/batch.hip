@@ -103,7 +103,7 @@ extern "C" int sponge_batch_create(int nsys, sponge_nl* const* nl, sponge_lj* co
     b->lds_fwd = b->lds_conv = b->lds_inv = 0;
     int rc = SPONGE_NB_OK;
     for (int s = 0; s < nsys && rc == SPONGE_NB_OK; s++) {
-        rc = snb_lj_scratch(lj[s], nl[s]);
+        rc = snb_scratch(&lj[s]->ps, nl[s]);
         b->h[s].io = io[s];
         snb_pme_plans(pme[s], &b->h[s].px, &b->h[s].py, &b->h[s].pz);
         b->max_nt = std::max(b->max_nt, lj[s]->ntypes);

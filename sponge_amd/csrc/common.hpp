@@ -391,9 +391,8 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
               int overwrite = 0, const float4* sc = nullptr, int inner = 0,
               ExclArgs ex = ExclArgs{nullptr, nullptr, nullptr});
 void snb_scratch_free(PairScratch* ps);
-// Cluster-order records (uint coordinates, charge, type) into ps->pk.
-int snb_gather(const sponge_nl* nl, const unsigned int* d_uint_crd, const float* d_charge, const int* d_type,
-               PairScratch* ps, hipStream_t s);
+// Sizes the scratch from the list (records, totals) on first use.
+int snb_scratch(PairScratch* ps, const sponge_nl* nl);
 void snb_fep_free(void* fep_scratch);
 int snb_excluded(sponge_pme* pme, const unsigned int* d_uint_crd, const float scaler[3], const float* d_charge,
                  const int* es, const int* el, const int* en, float* d_frc, float* d_atom_energy, hipStream_t s);
@@ -429,7 +428,6 @@ inline int* snb_nl_slot_counts(const sponge_nl* nl) {
 int snb_batch_prep(sponge_batch* b, int energy, int from_crd, int overwrite, hipStream_t s);
 int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s);
 int snb_batch_excluded(sponge_batch* b, hipStream_t s);
-int snb_lj_scratch(sponge_lj* lj, const sponge_nl* nl);
 void snb_adj_free(sponge_lj* lj);
 int snb_batch_reciprocal(sponge_batch* b, int energy, hipStream_t s);
 int snb_batch_gather(sponge_batch* b, hipStream_t s);

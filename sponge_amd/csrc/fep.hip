@@ -4,8 +4,8 @@
 // 13-125, :670-739) and FEP_CORE's direct-energy split (FEP_core/FEP_core.cu:
 // 12-66, :545-558).
 //
-// One walk over the cluster list (one wave per 4-atom i-cluster, lanes as in
-// the pair kernel, each unordered pair taken once from its lower-index atom)
+// One walk over the cluster list (one wave per 4-atom i-cluster, the pairs
+// inside the cutoff on full waves, each unordered pair once: dense_walk)
 // splits the pairs in two:
 //  * ordinary pairs (same mask, neither end state appearing from zero LJ):
 //    their energy is linear in lambda for LJ and quadratic for Coulomb
@@ -28,13 +28,13 @@
 
 #include "common.hpp"
 #include "pair_math.hpp"
+#include "dense_walk.hpp"
 #include "../../include/sponge_fep.h"
 
 using namespace snb;
 
 namespace {
 
-constexpr int kFepWaves = 4;
 constexpr int kSoftThreads = 256;
 constexpr int kWinParams = 8;   // lambda, 1 - lambda, a lambda^p, a (1-lambda)^p, p a lambda^(p-1), p a (1-lambda)^(p-1), t, 0
 constexpr int kSoftFields = 6;  // LJ inter, LJ intra, direct inter, direct intra, dH/dl LJ, dH/dl direct
@@ -57,108 +57,138 @@ __global__ void fep_zero_kernel(double* __restrict__ acc, int nacc, int* __restr
     if (i == 0) count[0] = 0;
 }
 
-// Walk of the cluster list. TABLE: soft-core handle records
-// fe[pt] = (AA, AB, BA, BB), fe[nt^2 + pt] = (soft, same mask, 0, 0)
-// for the pair type pt = t_i nt + t_j of combined types; without a table all
-// pairs are ordinary with zero LJ and the mask class comes from `mask`
-// (original order; NULL: one class).
+// Slot records of the walk (position, type and charge as the pair kernel's)
+// and the charge perturbation in slot order.
+__global__ void fep_gather_kernel(const int* __restrict__ flags, const int* __restrict__ s2o,
+                                  const unsigned int* __restrict__ uc, const float* __restrict__ q,
+                                  const float* __restrict__ dq, const int* __restrict__ type,
+                                  uint4* __restrict__ pk, float* __restrict__ dqs) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= flags[3]) return;
+    const int a = s2o[p];
+    uint4 r = make_uint4(0u, 0u, 0u, 0u);
+    if (a >= 0) {
+        const unsigned t = (unsigned)type[a];
+        r = make_uint4((uc[3 * a] & ~3u) | (t & 3u), (uc[3 * a + 1] & ~3u) | ((t >> 2) & 3u),
+                       (uc[3 * a + 2] & ~3u) | ((t >> 4) & 3u), __float_as_uint(q[a]));
+    }
+    pk[p] = r;
+    if (dq) dqs[p] = a >= 0 ? dq[a] : 0.f;
+}
+
+// Walk of the pair list (dense_walk: full waves of pairs inside the cutoff,
+// each unordered pair once). TABLE: soft-core handle records
+// fe[pt] = (AA, AB, BA, BB), fe[nt^2 + pt] = (soft, same mask, 0, 0) for the
+// pair type pt = t_i nt + t_j of combined types (an ordinary pair then has
+// one mask: pairs of two masks are soft); without a table all pairs are
+// ordinary with zero LJ and the mask class comes from `mask` (original order;
+// NULL: one class). The terms of perturbed charges and of end states that
+// differ are skipped by waves without such a pair.
+// Bound: FP64 issue (17M vector instructions at 23,496 atoms, 9 A: 28 us of
+// issue) and the latency of its 4 waves per SIMD. Measured 343 -> 50 us there
+// and 146 -> 22 us at 4,446 atoms against 16 lanes per cluster pair with the
+// device library's erfc, division and square root.
 template <bool TABLE>
-__global__ __launch_bounds__(kFepWaves * 64) void fep_list_kernel(
+__global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void fep_list_kernel(
     const int* __restrict__ flags, const int* __restrict__ list_n, const uint2* __restrict__ list, int list_cap,
     const uint4* __restrict__ pk, const int* __restrict__ s2o, const float4* __restrict__ fe, int nt, float cx,
-    float cy, float cz, float rc2, double beta, const float* __restrict__ dq, const int* __restrict__ mask,
+    float cy, float cz, float rc2, double beta, int rows, const float* __restrict__ dqs, const int* __restrict__ mask,
     double* __restrict__ acc, int4* __restrict__ soft, int* __restrict__ count, int soft_cap) {
-    __shared__ double red[kFepWaves][kHard];
+    __shared__ double red[kDenseWaves][kHard];
+    __shared__ DenseLds walk[kDenseWaves];
+    __shared__ unsigned long long soft_row[kMaxLjTypes];  // bit t_j: (t_i, t_j) is a soft-core pair type
+    extern __shared__ double etab[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int ic = blockIdx.x * kFepWaves + w;
+    erfc_fill(etab, rows);
+    if (TABLE)
+        for (int t = w; t < nt; t += kDenseWaves) {
+            const unsigned long long m = __ballot(lane < nt && fe[nt * nt + t * nt + min(lane, nt - 1)].x != 0.f);
+            if (lane == 0) soft_row[t] = m;
+        }
+    __syncthreads();
     double h[kHard];
 #pragma unroll
     for (int k = 0; k < kHard; k++) h[k] = 0.0;
-    if (ic < flags[4]) {
-        const int ii = lane & 3, jj = (lane >> 2) & 3, g = lane >> 4, bit = lane & 15;
-        const int islot = ic * kClusterSize + ii;
+    int pairs = 0;
+    const double beta64 = beta * kErfcPieces;
+    const DenseUnits units = dense_units(flags[4]);
+    for (int u = units.first; u < units.end; u += units.step) {
+        const int ic = u / units.parts;
+        const int islot = ic * kClusterSize + (lane >> 4);
         const uint4 a = pk[islot];
-        const unsigned ax = a.x & ~3u, ay = a.y & ~3u, az = a.z & ~3u;
         const int ti = unpack_type(a);
         const int ai = s2o[islot];
-        const double qi = (double)__uint_as_float(a.w);
-        const double dqi = (dq && ai >= 0) ? (double)dq[ai] : 0.0;
+        const float dqi = dqs ? dqs[islot] : 0.f;
         const int mi = (mask && ai >= 0) ? mask[ai] : 0;
-        const int n = list_n[ic];
-        const uint2* lst = list + (size_t)ic * list_cap;
-        for (int base = 0; base < n; base += 4) {
-            const int e = base + g;
-            const uint2 ent = e < n ? lst[e] : make_uint2((unsigned)ic, 0u);
-            const int jc = (int)ent.x;
-            const int jslot = jc * kClusterSize + jj;
+        const unsigned long long si = TABLE ? soft_row[ti] : 0ull;
+        dense_walk<true>(ic, pk, s2o, list_n, list, list_cap, cx, cy, cz, rc2, u % units.parts, units.parts,
+                         walk[w], [&](bool in, int jslot) {
             const uint4 b = pk[jslot];
-            const int ix = (int)((b.x & ~3u) - ax), iy = (int)((b.y & ~3u) - ay), iz = (int)((b.z & ~3u) - az);
-            const float r2f = dr2_exact((float)ix * cx, (float)iy * cy, (float)iz * cz);
-            const int aj = s2o[jslot];
-            const bool in = ((ent.y >> bit) & 1u) && r2f < rc2 && ai >= 0 && ai < aj;
+            const float dqj = dqs ? dqs[jslot] : 0.f;
             const int tj = unpack_type(b);
             const int pt = ti * nt + tj;
+            const int ix = (int)((b.x & ~3u) - (a.x & ~3u)), iy = (int)((b.y & ~3u) - (a.y & ~3u)),
+                      iz = (int)((b.z & ~3u) - (a.z & ~3u));
+            pairs += in ? 1 : 0;
             bool sp = false, intra = true;
             float4 f0 = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (in) {
-                if (TABLE) {
-                    const float4 f1 = fe[nt * nt + pt];
-                    sp = f1.x != 0.f;
-                    intra = f1.y != 0.f;
-                    f0 = fe[pt];
-                } else {
-                    intra = !mask || mi == mask[aj];
-                }
-            }
-            // soft-core pairs: one slot per lane, one atomic per wave
-            const unsigned long long sb = __ballot(in && sp);
-            if (sb) {
-                int basei = 0;
-                const int leader = __builtin_ctzll(sb);
-                if (lane == leader) basei = atomicAdd(count, __popcll(sb));
-                basei = __shfl(basei, leader);
-                if (in && sp) {
-                    const int k = basei + __popcll(sb & ((1ull << lane) - 1ull));
-                    if (k < soft_cap) {
-                        soft[2 * k] = make_int4(ai, aj, pt, 0);
+            if (TABLE) {
+                sp = in && ((si >> tj) & 1ull);
+                f0 = fe[pt];
+                // soft-core pairs: one slot per lane, one atomic per wave
+                const unsigned long long sb = __ballot(sp);
+                if (sb) {
+                    int basei = 0;
+                    const int leader = __builtin_ctzll(sb);
+                    if (lane == leader) basei = atomicAdd(count, __popcll(sb));
+                    basei = __shfl(basei, leader);
+                    const int k = basei + below(sb);
+                    if (sp && k < soft_cap) {
+                        soft[2 * k] = make_int4(ai, s2o[jslot], pt, 0);
                         soft[2 * k + 1] = make_int4(ix, iy, iz, 0);
                     }
                 }
+            } else if (mask) {
+                intra = mi == mask[max(s2o[jslot], 0)];
             }
-            if (in && !sp) {
+            const bool ord = in && !sp;
+            const bool charged = __any(ord && (dqi != 0.f || dqj != 0.f));
+            const bool differ = TABLE && __any(ord && (f0.x != f0.z || f0.y != f0.w));
+            if (ord) {
                 const double dx = (double)ix * (double)cx, dy = (double)iy * (double)cy, dz = (double)iz * (double)cz;
                 const double r2 = dx * dx + dy * dy + dz * dz;
-                const double r = sqrt(r2);
-                const double ec = erfc(beta * r);
-                const double gr = ec / r;
-                const double qj = (double)__uint_as_float(b.w);
-                const double dqj = dq ? (double)dq[aj] : 0.0;
-                const double q0 = qi * qj, q1 = qi * dqj + dqi * qj, q2 = dqi * dqj;
-                double vA = 0.0, vB = 0.0;
+                double rinv, r;
+                rsqrt_f64(r2, rinv, r);
+                const double ec = erfc_at(etab, rows, beta64 * r);
+                const double gr = ec * rinv;
+                const double qi = (double)__uint_as_float(a.w), qj = (double)__uint_as_float(b.w);
+                const double e0 = qi * qj * gr;
                 if (TABLE) {
-                    const double ir2 = 1.0 / r2, ir6 = ir2 * ir2 * ir2;
-                    vA = ((double)f0.x * (1.0 / 12.0) * ir6 - (double)f0.y * (1.0 / 6.0)) * ir6;
-                    vB = ((double)f0.z * (1.0 / 12.0) * ir6 - (double)f0.w * (1.0 / 6.0)) * ir6;
-                }
-                if (intra) {
+                    // 12 x the LJ energy: A r^-12 - 2 B r^-6 of the stored x12 / x6 tables
+                    const double ir2 = rinv * rinv, ir6 = ir2 * ir2 * ir2;
+                    const double vA = fma((double)f0.x, ir6, -2.0 * (double)f0.y) * ir6;
                     h[H_VA_INTRA] += vA;
-                    h[H_VB_INTRA] += vB;
-                    h[H_Q0_INTRA] += q0 * gr;
-                    h[H_Q1_INTRA] += q1 * gr;
-                    h[H_Q2_INTRA] += q2 * gr;
+                    h[H_VB_INTRA] += differ ? fma((double)f0.z, ir6, -2.0 * (double)f0.w) * ir6 : vA;
+                    h[H_Q0_INTRA] += e0;
                 } else {
-                    h[H_VA_INTER] += vA;
-                    h[H_VB_INTER] += vB;
-                    h[H_Q0_INTER] += q0 * gr;
-                    h[H_Q1_INTER] += q1 * gr;
-                    h[H_Q2_INTER] += q2 * gr;
+                    h[H_Q0_INTRA] += intra ? e0 : 0.0;
+                    h[H_Q0_INTER] += intra ? 0.0 : e0;
                 }
-                h[H_R1] += q1 * ec;
-                h[H_R2] += q2 * ec;
+                if (charged) {
+                    const double q1 = qi * (double)dqj + (double)dqi * qj, q2 = (double)dqi * (double)dqj;
+                    h[H_Q1_INTRA] += intra ? q1 * gr : 0.0;
+                    h[H_Q2_INTRA] += intra ? q2 * gr : 0.0;
+                    h[H_Q1_INTER] += intra ? 0.0 : q1 * gr;
+                    h[H_Q2_INTER] += intra ? 0.0 : q2 * gr;
+                    h[H_R1] += q1 * ec;
+                    h[H_R2] += q2 * ec;
+                }
             }
-            if (in) h[H_PAIRS] += 1.0;
-        }
+        });
     }
+    h[H_VA_INTRA] *= 1.0 / 12.0;
+    h[H_VB_INTRA] *= 1.0 / 12.0;
+    h[H_PAIRS] = (double)pairs;
 #pragma unroll
     for (int k = 0; k < kHard; k++) {
         const double v = wave_sum(h[k]);
@@ -167,7 +197,7 @@ __global__ __launch_bounds__(kFepWaves * 64) void fep_list_kernel(
     __syncthreads();
     if (threadIdx.x < kHard) {
         double s = 0.0;
-        for (int k = 0; k < kFepWaves; k++) s += red[k][threadIdx.x];
+        for (int k = 0; k < kDenseWaves; k++) s += red[k][threadIdx.x];
         if (s != 0.0) atomicAdd(acc + threadIdx.x, s);
     }
 }
@@ -291,6 +321,8 @@ struct FepScratch {
     int soft_cap = 0;
     double* win = nullptr;      // SPONGE_FEP_MAX_WINDOWS * kWinParams
     float* phi = nullptr;       // n potentials (PME)
+    float* dqs = nullptr;       // the walk's charge perturbation in slot order
+    int dqs_cap = 0;
     int* zero_type = nullptr;   // n zeros (tableless walks)
     int n = 0;
     PairScratch ps{};           // cluster-ordered records of the walk
@@ -299,7 +331,7 @@ struct FepScratch {
 void snb_fep_free(void* p) {
     FepScratch* f = static_cast<FepScratch*>(p);
     if (!f) return;
-    void* ptrs[] = {f->acc, f->count, f->soft, f->win, f->phi, f->zero_type};
+    void* ptrs[] = {f->acc, f->count, f->soft, f->win, f->phi, f->dqs, f->zero_type};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     snb_scratch_free(&f->ps);
@@ -362,18 +394,30 @@ int fep_walk(FepScratch* f, const WalkArgs& A, int nwin, const double* h_win, do
         const int nacc = kHard + nwin * kSoftFields;
         fep_zero_kernel<<<ceil_div(nacc, 256), 256, 0, s>>>(f->acc, nacc, f->count);
         SNB_CHECK_LAUNCH();
-        int rc = snb_gather(nl, A.uc, A.q, A.type ? A.type : f->zero_type, &f->ps, s);
+        int rc = snb_scratch(&f->ps, nl);
         if (rc) return rc;
-        const int nblk = ceil_div(nl->ncl_cap, kFepWaves);
+        if (f->dqs_cap < f->ps.cap) {
+            if (f->dqs) SNB_HIP(hipFree(f->dqs));
+            f->dqs = nullptr;
+            f->dqs_cap = 0;
+            SNB_HIP(hipMalloc((void**)&f->dqs, f->ps.cap * sizeof(float)));
+            f->dqs_cap = f->ps.cap;
+        }
+        float* dqs = A.dq ? f->dqs : nullptr;
+        fep_gather_kernel<<<ceil_div(f->ps.cap, 256), 256, 0, s>>>(nl->flags, nl->s2o, A.uc, A.q, A.dq,
+                                                                  A.type ? A.type : f->zero_type, f->ps.pk, dqs);
+        SNB_CHECK_LAUNCH();
+        const int nblk = std::min(kDenseBlocks, xcd_grid(ceil_div(8l * nl->ncl_cap, kDenseWaves)));
         const float rc2 = A.cutoff * A.cutoff;
+        const int rows = erfc_rows(A.beta, A.cutoff);
         if (A.fe)
-            fep_list_kernel<true><<<nblk, kFepWaves * 64, 0, s>>>(
+            fep_list_kernel<true><<<nblk, kDenseWaves * 64, erfc_lds(rows), s>>>(
                 nl->flags, nl->list_n, nl->list, nl->list_cap, f->ps.pk, nl->s2o, A.fe, A.nt, A.cof[0], A.cof[1],
-                A.cof[2], rc2, A.beta, A.dq, A.mask, f->acc, f->soft, f->count, f->soft_cap);
+                A.cof[2], rc2, A.beta, rows, dqs, A.mask, f->acc, f->soft, f->count, f->soft_cap);
         else
-            fep_list_kernel<false><<<nblk, kFepWaves * 64, 0, s>>>(
+            fep_list_kernel<false><<<nblk, kDenseWaves * 64, erfc_lds(rows), s>>>(
                 nl->flags, nl->list_n, nl->list, nl->list_cap, f->ps.pk, nl->s2o, nullptr, 1, A.cof[0], A.cof[1],
-                A.cof[2], rc2, A.beta, A.dq, A.mask, f->acc, f->soft, f->count, f->soft_cap);
+                A.cof[2], rc2, A.beta, rows, dqs, A.mask, f->acc, f->soft, f->count, f->soft_cap);
         SNB_CHECK_LAUNCH();
         if (A.fe && nwin > 0) {
             SNB_HIP(hipMemcpyAsync(f->win, h_win, nwin * kWinParams * sizeof(double), hipMemcpyHostToDevice, s));

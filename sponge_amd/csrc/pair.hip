@@ -743,16 +743,6 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
     return SPONGE_NB_OK;
 }
 
-int snb_gather(const sponge_nl* nl, const unsigned int* d_uint_crd, const float* d_charge, const int* d_type,
-               PairScratch* ps, hipStream_t s) {
-    int rc = scratch_ensure(ps, nl);
-    if (rc) return rc;
-    gather_kernel<<<ceil_div(ps->cap, 256), 256, 0, s>>>(nl->flags, nl->s2o, d_uint_crd, d_charge, d_type, ps->pk, 0,
-                                                         ps->acc);
-    SNB_CHECK_LAUNCH();
-    return SPONGE_NB_OK;
-}
-
 int snb_step_prep(const sponge_nl* nl, sponge_lj* lj, sponge_pme* pme, const float* d_crd, unsigned int* d_uint_crd,
                   const float* d_charge, int energy, float* d_frc_assigned, hipStream_t s) {
     int rc = scratch_ensure(&lj->ps, nl);
@@ -922,5 +912,5 @@ int snb_batch_excluded(sponge_batch* b, hipStream_t s) {
     return SPONGE_NB_OK;
 }
 
-int snb_lj_scratch(sponge_lj* lj, const sponge_nl* nl) { return scratch_ensure(&lj->ps, nl); }
+int snb_scratch(PairScratch* ps, const sponge_nl* nl) { return scratch_ensure(ps, nl); }
 

@@ -1,0 +1,58 @@
+"""The walk that queues the pairs inside the cutoff for full waves, where it
+can go wrong: boxes so small that the displacement from a cluster's first atom
+no longer names the nearest image (every batch takes the exact test), systems
+of fewer clusters than the launch has waves, clusters with padding slots,
+beta * cutoff past the erfc table's last row, and no perturbed charges. The
+pair sums are FP64 on both sides from the same integer displacements: 1e-9."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle
+from sponge_amd import system
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-9
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+# waters before the solute, cutoff, skin, beta (None: the PME module's)
+CASES = [
+    (216, 8.0, 1.0, None),    # 18.6 A box: cutoff + a cluster's extent passes half of it
+    (216, 9.2, 0.1, None),    # cutoff at half the box
+    (343, 5.0, 0.5, 1.7),     # beta * cutoff 8.5: past the table's end
+    (343, 5.0, 0.5, 0.02),    # one or two rows
+    (2197, 9.0, 2.0, None),
+]
+
+
+@pytest.mark.parametrize("waters,cutoff,skin,beta", CASES)
+def test_windows(waters, cutoff, skin, beta):
+    import torch
+    from sponge_amd import nb
+    fs = system.fep_mixed(system.fep_system(waters, 0.35, seed=5, cutoff=cutoff, skin=skin))
+    say(f"[case] waters {waters} n {fs.n} box {fs.box[0]:.3f} cutoff {cutoff} beta {beta}")
+    eng = nb.NonbondedEngine(fs, refresh_interval=0)
+    eng.update_neighbor_list(forced=1)
+    eng.crd_to_uint()
+    torch.cuda.synchronize()
+    eng.nl.check()
+    u = eng.uint_crd.cpu().numpy().view(np.uint32)
+    pairs = oracle.nl_brute(fs, u)
+    b = float(np.float32(beta if beta is not None else eng.pme.beta))
+    dq_h = (fs.charge_B.astype(np.float64) - fs.charge_A.astype(np.float64)).astype(np.float32)
+    lams = [0.0, 0.35, 1.0]
+    lam0 = float(np.float32(fs.lam))
+    for dq in (dq_h, None):
+        got = eng.lj.lambda_windows(eng.nl, eng.uint_crd, eng.charge,
+                                    None if dq is None else torch.as_tensor(dq, device="cuda"), b, lams)
+        ref = oracle.fep_windows(fs, u, pairs, b, lams, dq=dq, lambda0=lam0)
+        err = np.abs(got[:, :7] - ref) / np.maximum(1.0, np.abs(ref))
+        say(f"    dq {dq is not None}: worst relative error {err.max():.2e}")
+        assert err.max() <= TOL, (dq is not None, np.unravel_index(err.argmax(), err.shape))

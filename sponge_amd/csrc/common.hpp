@@ -217,24 +217,22 @@ struct sponge_nl {
     uint4* prune_ref;           // slot_cap: slot records at the last prune
     int* list_in_n;             // ncl_cap
     uint2* list_in;             // ncl_cap * list_cap
-    // the inner pairs per i slot (j slots within prune_r2) for plain LJ,
-    // which force-only fused steps read (list_in is soft-core LJ's form),
-    // each as the 16-bit offset j - i, taken modulo the slot count when that
-    // is the shorter way (the slot records carry kPkHalo copies on either
-    // side, so i + offset is always a readable record). flags[11] = 1 once a
-    // slot held more than atom_in_cap partners, or a partner out of 16-bit
-    // reach, at a prune since the last rebuild (its cluster then reads the
-    // full list); flags[12] counts the launches that read the per-slot form
+    // per-slot lists: the partners of each i slot as 16-bit offsets j - i,
+    // taken modulo the slot count when that is the shorter way (the slot
+    // records carry kPkHalo copies on either side, so i + offset is always a
+    // readable record). atom_full: every pair of the full list, written by
+    // each rebuild while the inner lists are on, or by the first fused step after a new prune setting (flags[14] holds
+    // that step's number). atom_in: the pairs of atom_full within prune_r2
+    // when the prune radius is below the list radius (two levels).
+    // flags[11] = 1 once a slot held more than atom_in_cap partners, or a
+    // partner out of 16-bit reach, since the last rebuild (its cluster then
+    // reads the full list); flags[12] counts the launches that read the
+    // per-slot form
     int atom_in_cap;
     int* atom_in_n;             // slot_cap
     unsigned short* atom_in;    // slot_cap * atom_in_cap
-    // outer per-slot lists (same form and cap), used when the prune radius
-    // is below the list radius: every pair of the full list (within
-    // rc + skin at the rebuild), written by the rebuild or by the first
-    // fused step after a new prune setting (flags[14] holds that step's
-    // number); the inner lists are then pruned from these
-    int* atom_out_n;            // slot_cap
-    unsigned short* atom_out;   // slot_cap * atom_in_cap
+    int* atom_full_n;           // slot_cap
+    unsigned short* atom_full;  // slot_cap * atom_in_cap
     // symmetric exclusion lists in original atom order (partners of atom a:
     // sym_list[sym_start[a] .. sym_start[a+1])), built on the host from the
     // exclusion CSR the first time an update passes those arrays
@@ -352,25 +350,22 @@ struct sponge_batch {
     hipEvent_t fork = nullptr, join = nullptr;
 };
 
-// Inner-list arguments of the pair kernel (interval 0: no inner list).
+// List arguments of the pair kernel (interval 0: no inner lists).
 struct PruneArgs {
     int interval = 0;
     float r2 = 0.f;
-    int* in_n = nullptr;
+    int* in_n = nullptr;        // cluster-pair inner list (soft-core LJ)
     uint2* in_list = nullptr;
-    int* atom_n = nullptr;      // per-slot inner lists (NULL: cluster form only)
-    unsigned short* atom_list = nullptr;  // 16-bit slot offsets
+    int* full_n = nullptr;      // per-slot lists of every listed pair (plain LJ):
+    unsigned short* full_list = nullptr;  // 16-bit slot offsets
+    int* atom_n = nullptr;      // per-slot inner lists, two levels only (else NULL): a prune
+    unsigned short* atom_list = nullptr;  // filters the full ones
     int atom_cap = 0;
     int* diag = nullptr;        // flags + 11: [0] per-slot overflow, [1] per-slot launches,
                                 // [2] step of the last displacement vote, [3] step whose
                                 // per-slot lists are rewritten (a new prune setting),
                                 // [4] voted prunes
     uint4* ref = nullptr;       // slot records at the last prune
-    // two-level per-slot lists (atom_olist non-NULL): the outer lists hold
-    // every pair of the full list, and a prune of the inner lists filters
-    // them instead of the cluster-pair list
-    int* atom_on = nullptr;
-    unsigned short* atom_olist = nullptr;
     const float4* ctab = nullptr;  // the Coulomb table (per-slot force loop), NULL: the formula
     float ctab_scale = 0.f;        // intervals per Angstrom
     int pk_records = 0;            // the slot records with their copies on either side
@@ -416,15 +411,6 @@ float snb_nl_rlm(const sponge_nl* nl);
 float snb_prune_vote_r2(float cutoff, float prune_radius);
 // Two-level per-slot lists: an inner prune radius below the list radius.
 inline bool snb_two_level(const sponge_nl* nl) { return nl->prune_interval > 0 && nl->prune_r2 < nl->rl2; }
-// The per-slot lists of every listed pair, which each rebuild writes after
-// the list (the outer ones of the two-level form); NULL while the inner list
-// is off.
-inline unsigned short* snb_nl_slot_lists(const sponge_nl* nl) {
-    return nl->prune_interval > 0 ? (snb_two_level(nl) ? nl->atom_out : nl->atom_in) : nullptr;
-}
-inline int* snb_nl_slot_counts(const sponge_nl* nl) {
-    return nl->prune_interval > 0 ? (snb_two_level(nl) ? nl->atom_out_n : nl->atom_in_n) : nullptr;
-}
 int snb_batch_prep(sponge_batch* b, int energy, int from_crd, int overwrite, hipStream_t s);
 int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s);
 int snb_batch_excluded(sponge_batch* b, hipStream_t s);

@@ -25,41 +25,51 @@ constexpr int kDenseQueue = 112;   // queued pairs per i atom: at most 48 left b
 constexpr int kDenseEntries = 128; // list entries staged at a time
 
 // The walk's kernels run as kDenseBlocks resident blocks whose waves stride
-// over units of work, a unit being one of `parts` shares of a cluster's list:
+// over units of work, a unit being one of 1 to 8 shares of a cluster's list:
 // the erfc rows, the final sums and their atomics are then paid once per
 // wave and not once per cluster.
 constexpr int kDenseBlocks = 512;  // 2 of 8 waves on each of 256 CUs
 
-// Shares of a cluster's list that give the waves the evenest rounds (a
-// share's own fixed cost taken as 8 % of a whole list).
-__device__ __forceinline__ int dense_parts(int clusters, int waves) {
-    int best = 1;
+// Shares of a cluster's list (as a power of two) that give the waves the
+// evenest rounds (a share's own fixed cost taken as 8 % of a whole list).
+__device__ __forceinline__ int dense_split(int clusters, int waves) {
+    int best = 0;
     float least = 1e30f;
-    for (int p = 1; p <= 8; p *= 2) {
-        const float t = (float)((clusters * p + waves - 1) / waves) * (1.0f / p + 0.08f);
+    for (int k = 0; k <= 3; k++) {
+        const float t = (float)(((clusters << k) + waves - 1) / waves) * (1.0f / (1 << k) + 0.08f);
         if (t < least) {
             least = t;
-            best = p;
+            best = k;
         }
     }
-    return best;
+    return __builtin_amdgcn_readfirstlane(best);
 }
 
-// Units of this wave: first, first + step, ... below end (each XCD a
-// contiguous range of clusters). Blocks a multiple of kNumXcd.
+// Units of a block: block-first `base` below `end`, `step` apart, wave w taking
+// unit base + w, share u % 2^split of cluster u / 2^split; each XCD a
+// contiguous range of clusters, and the shares of one cluster adjacent waves
+// of one block. Blocks a multiple of kNumXcd.
 struct DenseUnits {
-    int parts, first, end, step;
+    int split, base, end, step;
 };
 __device__ __forceinline__ DenseUnits dense_units(int clusters) {
     DenseUnits u;
-    u.parts = dense_parts(clusters, gridDim.x * kDenseWaves);
-    const int total = clusters * u.parts, x = blockIdx.x % kNumXcd;
+    u.split = dense_split(clusters, gridDim.x * kDenseWaves);
+    const int x = blockIdx.x % kNumXcd;
     u.step = gridDim.x / kNumXcd * kDenseWaves;
-    // (uniform over the wave: the walk's loops and counts then stay scalar)
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    u.first = (int)((long)total * x / kNumXcd) + (int)(blockIdx.x / kNumXcd) * kDenseWaves + w;
-    u.end = (int)((long)total * (x + 1) / kNumXcd);
+    u.base = ((int)((long)clusters * x / kNumXcd) << u.split) + (int)(blockIdx.x / kNumXcd) * kDenseWaves;
+    u.end = (int)((long)clusters * (x + 1) / kNumXcd) << u.split;
     return u;
+}
+// Resident blocks for a list of at most `clusters` clusters.
+inline int dense_blocks(int clusters) {
+    const int most = xcd_grid(ceil_div(8l * clusters, kDenseWaves));
+    return most < kDenseBlocks ? most : kDenseBlocks;
+}
+// The wave's number in its block, uniform over the wave (the walk's loops and
+// counts then stay scalar).
+__device__ __forceinline__ int wave_in_block() {
+    return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
 struct DenseLds {
@@ -140,49 +150,64 @@ __device__ __forceinline__ void rsqrt_f64(double r2, double& rinv, double& r) {
 // ---- the walk ---------------------------------------------------------------
 // Calls use(active, jslot) with all 64 lanes, lane (i, k) = (lane >> 4,
 // lane & 15) taking pairs of the cluster's slot i; every pair inside the
-// cutoff is handed over once per side (HALF: once in all, from one of its
-// clusters: the one the parity of the cluster numbers names, so that all
-// clusters keep about half of their pairs). Every lane of the wave must call.
-// `part` of `parts`: this wave's share of the cluster's list entries.
+// cutoff is handed over once per side (kEachSide), or once in all: from the
+// side of its lower-index atom (kLowerAtom: per-atom sums credited to that
+// atom), or from one of its clusters, the one that the parity of the cluster
+// numbers names (kOneCluster: totals; half of the entries are scanned, about
+// the same share of every cluster's). Every lane of the wave must call.
+// `part` of 2^split: this wave's share of the cluster's list entries. ic and
+// part uniform over the wave.
+enum DenseSide { kEachSide, kLowerAtom, kOneCluster };
 // Set bits of a wave mask below this lane.
 __device__ __forceinline__ int below(unsigned long long m) {
     return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
+// The first lane's value, in a scalar register.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// The value of lane K of this lane's quad.
+template <int K>
+__device__ __forceinline__ float quad_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), K * 0x55, 0xF, 0xF, false));
+}
+
 typedef float DenseF4 __attribute__((ext_vector_type(4)));
 
-template <bool HALF, class Use>
+template <DenseSide SIDE, class Use>
 __device__ __forceinline__ void dense_walk(int ic, const uint4* __restrict__ pk, const int* __restrict__ s2o,
                                            const int* __restrict__ list_n, const uint2* __restrict__ list,
                                            int list_cap, float cx, float cy, float cz, float rc2, int part,
-                                           int parts, DenseLds& L, Use&& use) {
+                                           int split, DenseLds& L, Use&& use) {
     const int lane = threadIdx.x & 63, jj = lane & 3;
-    uint4 a[kClusterSize];
-    float aa[kClusterSize], own[3] = {0.f, 0.f, 0.f};
-    float ext = 0.f;
-#pragma unroll
-    for (int i = 0; i < kClusterSize; i++) {
-        a[i] = pk[ic * kClusterSize + i];
-        // padding (the last slots of a column) takes the first atom's place:
-        // none of its pairs is listed
-        const bool pad = s2o[ic * kClusterSize + i] < 0;
-        const float x = pad ? 0.f : (float)(int)((a[i].x & ~3u) - (a[0].x & ~3u)) * cx;
-        const float y = pad ? 0.f : (float)(int)((a[i].y & ~3u) - (a[0].y & ~3u)) * cy;
-        const float z = pad ? 0.f : (float)(int)((a[i].z & ~3u) - (a[0].z & ~3u)) * cz;
-        aa[i] = x * x + y * y + z * z;
-        ext = fmaxf(ext, aa[i]);
-        if (jj == i) {
-            own[0] = -2.0f * x;
-            own[1] = -2.0f * y;
-            own[2] = -2.0f * z;
-        }
+    // the first atom's position (uniform), and this lane's i atom jj: -2 a for
+    // the product, |a|^2 and the atom's index spread over the lane's quad
+    const uint4 mine = pk[ic * kClusterSize + jj];
+    const int mine_at = s2o[ic * kClusterSize + jj];
+    const unsigned ox = uniform((int)(mine.x & ~3u)), oy = uniform((int)(mine.y & ~3u)),
+                   oz = uniform((int)(mine.z & ~3u));
+    // padding (the last slots of a column) takes the first atom's place: none
+    // of its pairs is listed
+    const bool pad = mine_at < 0;
+    const float px = pad ? 0.f : (float)(int)((mine.x & ~3u) - ox) * cx;
+    const float py = pad ? 0.f : (float)(int)((mine.y & ~3u) - oy) * cy;
+    const float pz = pad ? 0.f : (float)(int)((mine.z & ~3u) - oz) * cz;
+    const float own[3] = {-2.0f * px, -2.0f * py, -2.0f * pz};
+    const float paa = px * px + py * py + pz * pz;
+    const float aa[kClusterSize] = {quad_lane<0>(paa), quad_lane<1>(paa), quad_lane<2>(paa), quad_lane<3>(paa)};
+    int at[kClusterSize] = {0, 0, 0, 0};
+    if (SIDE == kLowerAtom) {
+        const float t = __int_as_float(mine_at);
+        at[0] = __float_as_int(quad_lane<0>(t));
+        at[1] = __float_as_int(quad_lane<1>(t));
+        at[2] = __float_as_int(quad_lane<2>(t));
+        at[3] = __float_as_int(quad_lane<3>(t));
     }
-    ext = sqrtf(ext);
-    const float rc = sqrtf(rc2), reach = rc + ext;
+    const float ext = __builtin_amdgcn_sqrtf(fmaxf(fmaxf(aa[0], aa[1]), fmaxf(aa[2], aa[3])));
+    const float rc = sqrtf(rc2), reach = (rc + ext) * 1.0001f;
     // the displacement from the first atom names the nearest image of every
     // pair inside the cutoff only while cutoff + extent is below half a box
     // (2^31 units); else every batch takes the exact test
-    const bool safe = reach * 1.0001f < 2147483648.0f * fminf(cx, fminf(cy, cz));
+    const bool safe = reach < 2147483648.0f * fminf(cx, fminf(cy, cz));
     // |a|, |b| <= reach near the cutoff: coordinates 8, |a|^2 and |b|^2 13,
     // the product's three steps 16, dr2_exact 7 units of 2^-24 reach^2
     const float eps = 4.0e-6f * reach * reach;
@@ -193,22 +218,23 @@ __device__ __forceinline__ void dense_walk(int ic, const uint4* __restrict__ pk,
     // hands over up to 16 pairs of each i atom, the last queued ones first
     auto drain = [&]() {
         const int ci = i4 == 0 ? c[0] : i4 == 1 ? c[1] : i4 == 2 ? c[2] : c[3];
-        const int at = max(ci - 16, 0) + k16;
-        const bool active = at < ci;
-        const int jslot = active ? L.q[i4][at] : ic * kClusterSize;
+        const int e = max(ci - 16, 0) + k16;
+        const bool active = e < ci;
+        const int jslot = active ? L.q[i4][e] : ic * kClusterSize;
         __builtin_amdgcn_wave_barrier();
         use(active, jslot);
 #pragma unroll
         for (int i = 0; i < kClusterSize; i++) c[i] = max(c[i] - 16, 0);
     };
 
-    const int n_all = list_n[ic], first = n_all * part / parts, n = n_all * (part + 1) / parts - first;
+    const int n_all = uniform(list_n[ic]), first = (n_all * part) >> split,
+              n = ((n_all * (part + 1)) >> split) - first;
     const uint2* __restrict__ lst = list + (size_t)ic * list_cap + first;
     const uint2 none = make_uint2((unsigned)ic, 0u);
     const int e0 = lane >> 2;
     int base = 0, it = 0, kept = 0;
     uint2 ent = none;
-    uint4 b = a[0];
+    uint4 b = mine;
     for (;;) {
         while (it >= kept && base < n) {
             // stage the next entries this side takes
@@ -217,7 +243,7 @@ __device__ __forceinline__ void dense_walk(int ic, const uint4* __restrict__ pk,
             for (int h = 0; h < kDenseEntries; h += 64) {
                 const int e = base + h + lane;
                 uint2 my = e < n ? lst[e] : none;
-                if (HALF) {
+                if (SIDE == kOneCluster) {
                     const int jc = (int)my.x;
                     if (jc == ic) my.y &= 0x7310u;  // the cluster's own pairs with jj > ii
                     else if ((ic < jc) != (((ic ^ jc) & 1) != 0)) my.y = 0u;
@@ -241,9 +267,10 @@ __device__ __forceinline__ void dense_walk(int ic, const uint4* __restrict__ pk,
             const uint4 bn = pk[(int)entn.x * kClusterSize + jj];
             const int jslot = (int)ent.x * kClusterSize + jj;
             const unsigned m4 = (ent.y >> (jj * 4)) & 15u;
-            const float x = (float)(int)((b.x & ~3u) - (a[0].x & ~3u)) * cx;
-            const float y = (float)(int)((b.y & ~3u) - (a[0].y & ~3u)) * cy;
-            const float z = (float)(int)((b.z & ~3u) - (a[0].z & ~3u)) * cz;
+            const int aj = SIDE == kLowerAtom ? s2o[jslot] : 0;
+            const float x = (float)(int)((b.x & ~3u) - ox) * cx;
+            const float y = (float)(int)((b.y & ~3u) - oy) * cy;
+            const float z = (float)(int)((b.z & ~3u) - oz) * cz;
             const float bb = x * x + y * y + z * z;
             DenseF4 t = {bb + aa[0], bb + aa[1], bb + aa[2], bb + aa[3]};
             t = __builtin_amdgcn_mfma_f32_4x4x1f32(own[0], x, t, 0, 0, 0);
@@ -252,17 +279,19 @@ __device__ __forceinline__ void dense_walk(int ic, const uint4* __restrict__ pk,
             unsigned long long in[kClusterSize], near = 0ull;
 #pragma unroll
             for (int i = 0; i < kClusterSize; i++) {
-                const unsigned long long listed = __ballot((m4 >> i) & 1u);
+                const unsigned long long listed = __ballot(((m4 >> i) & 1u) && (SIDE != kLowerAtom || at[i] < aj));
                 in[i] = listed & __ballot(t[i] < lo);
                 near |= listed & ~in[i] & __ballot(t[i] < hi);
             }
             if (!safe || near) {
 #pragma unroll
                 for (int i = 0; i < kClusterSize; i++) {
-                    const float dx = (float)(int)((b.x & ~3u) - (a[i].x & ~3u)) * cx;
-                    const float dy = (float)(int)((b.y & ~3u) - (a[i].y & ~3u)) * cy;
-                    const float dz = (float)(int)((b.z & ~3u) - (a[i].z & ~3u)) * cz;
-                    in[i] = __ballot(((m4 >> i) & 1u) && dr2_exact(dx, dy, dz) < rc2);
+                    const uint4 a = pk[ic * kClusterSize + i];
+                    const float dx = (float)(int)((b.x & ~3u) - (a.x & ~3u)) * cx;
+                    const float dy = (float)(int)((b.y & ~3u) - (a.y & ~3u)) * cy;
+                    const float dz = (float)(int)((b.z & ~3u) - (a.z & ~3u)) * cz;
+                    in[i] = __ballot(((m4 >> i) & 1u) && (SIDE != kLowerAtom || at[i] < aj) &&
+                                     dr2_exact(dx, dy, dz) < rc2);
                 }
             }
 #pragma unroll

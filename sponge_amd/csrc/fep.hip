@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_e
     __shared__ DenseLds walk[kDenseWaves];
     __shared__ unsigned long long soft_row[kMaxLjTypes];  // bit t_j: (t_i, t_j) is a soft-core pair type
     extern __shared__ double etab[];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = wave_in_block();
     erfc_fill(etab, rows);
     if (TABLE)
         for (int t = w; t < nt; t += kDenseWaves) {
@@ -112,8 +112,8 @@ __global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_e
     int pairs = 0;
     const double beta64 = beta * kErfcPieces;
     const DenseUnits units = dense_units(flags[4]);
-    for (int u = units.first; u < units.end; u += units.step) {
-        const int ic = u / units.parts;
+    for (int u = units.base + w; u < units.end; u += units.step) {
+        const int ic = u >> units.split;
         const int islot = ic * kClusterSize + (lane >> 4);
         const uint4 a = pk[islot];
         const int ti = unpack_type(a);
@@ -121,8 +121,8 @@ __global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_e
         const float dqi = dqs ? dqs[islot] : 0.f;
         const int mi = (mask && ai >= 0) ? mask[ai] : 0;
         const unsigned long long si = TABLE ? soft_row[ti] : 0ull;
-        dense_walk<true>(ic, pk, s2o, list_n, list, list_cap, cx, cy, cz, rc2, u % units.parts, units.parts,
-                         walk[w], [&](bool in, int jslot) {
+        dense_walk<kOneCluster>(ic, pk, s2o, list_n, list, list_cap, cx, cy, cz, rc2, u & ((1 << units.split) - 1),
+                                  units.split, walk[w], [&](bool in, int jslot) {
             const uint4 b = pk[jslot];
             const float dqj = dqs ? dqs[jslot] : 0.f;
             const int tj = unpack_type(b);
@@ -407,7 +407,7 @@ int fep_walk(FepScratch* f, const WalkArgs& A, int nwin, const double* h_win, do
         fep_gather_kernel<<<ceil_div(f->ps.cap, 256), 256, 0, s>>>(nl->flags, nl->s2o, A.uc, A.q, A.dq,
                                                                   A.type ? A.type : f->zero_type, f->ps.pk, dqs);
         SNB_CHECK_LAUNCH();
-        const int nblk = std::min(kDenseBlocks, xcd_grid(ceil_div(8l * nl->ncl_cap, kDenseWaves)));
+        const int nblk = dense_blocks(nl->ncl_cap);
         const float rc2 = A.cutoff * A.cutoff;
         const int rows = erfc_rows(A.beta, A.cutoff);
         if (A.fe)

@@ -827,8 +827,8 @@ extern "C" int sponge_nl_create(int atom_numbers, const float box_length[3], flo
     }
     A((void**)&nl->atom_in_n, nl->slot_cap * sizeof(int));
     A((void**)&nl->atom_in, (size_t)nl->slot_cap * nl->atom_in_cap * sizeof(unsigned short));
-    A((void**)&nl->atom_out_n, nl->slot_cap * sizeof(int));
-    A((void**)&nl->atom_out, (size_t)nl->slot_cap * nl->atom_in_cap * sizeof(unsigned short));
+    A((void**)&nl->atom_full_n, nl->slot_cap * sizeof(int));
+    A((void**)&nl->atom_full, (size_t)nl->slot_cap * nl->atom_in_cap * sizeof(unsigned short));
     A((void**)&nl->pack, nl->slot_cap * sizeof(uint4));
     A((void**)&nl->flags, 16 * sizeof(int));
     if (e == hipSuccess) e = hipMemset(nl->flags, 0, 16 * sizeof(int));
@@ -837,9 +837,9 @@ extern "C" int sponge_nl_create(int atom_numbers, const float box_length[3], flo
     if (e == hipSuccess) e = hipMemset(nl->atom_in_n, 0, nl->slot_cap * sizeof(int));
     if (e == hipSuccess)
         e = hipMemset(nl->atom_in, 0, (size_t)nl->slot_cap * nl->atom_in_cap * sizeof(unsigned short));
-    if (e == hipSuccess) e = hipMemset(nl->atom_out_n, 0, nl->slot_cap * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(nl->atom_full_n, 0, nl->slot_cap * sizeof(int));
     if (e == hipSuccess)
-        e = hipMemset(nl->atom_out, 0, (size_t)nl->slot_cap * nl->atom_in_cap * sizeof(unsigned short));
+        e = hipMemset(nl->atom_full, 0, (size_t)nl->slot_cap * nl->atom_in_cap * sizeof(unsigned short));
     // Inner list of the fused step (interval mode): pruned every
     // P = refresh_interval / prune_div fused steps to rc + margin * skin, and
     // at once on a step where an atom has moved more than half the margin
@@ -873,7 +873,7 @@ extern "C" void sponge_nl_destroy(sponge_nl* nl) {
     void* ptrs[] = {nl->old_crd, nl->nl_uint, nl->col_count, nl->col_start, nl->col_atoms, nl->s2o,
                     nl->o2s,     nl->cl_lo,   nl->cl_hi,     nl->list_n,    nl->list,      nl->pack,
                     nl->flags,   nl->list_in, nl->list_in_n, nl->sym_start, nl->sym_list, nl->atom_in_n,
-                    nl->atom_in, nl->dropped, nl->prune_ref, nl->atom_out_n, nl->atom_out};
+                    nl->atom_in, nl->dropped, nl->prune_ref, nl->atom_full_n, nl->atom_full};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     delete nl;
@@ -922,9 +922,10 @@ static int nl_rebuild(sponge_nl* nl, float* d_crd, const int* es, const int* el,
         rlm, nl->col_start, nl->cl_lo, nl->cl_hi, nl->pack, es, en, el, nl->list_cap, nl->list_n, nl->list,
         nl->flags, nl->sym_start, nl->sym_list);
     SNB_CHECK_LAUNCH();
-    if (unsigned short* sl = snb_nl_slot_lists(nl)) {
+    if (nl->prune_interval > 0) {
         nl_slot_lists_kernel<<<xcd_grid(ceil_div(nl->ncl_cap, 4)), 256, 0, s>>>(
-            nl->flags, nl->list_n, nl->list, nl->list_cap, sl, snb_nl_slot_counts(nl), nl->atom_in_cap, nl->flags + 11);
+            nl->flags, nl->list_n, nl->list, nl->list_cap, nl->atom_full, nl->atom_full_n, nl->atom_in_cap,
+            nl->flags + 11);
         SNB_CHECK_LAUNCH();
     }
     return SPONGE_NB_OK;

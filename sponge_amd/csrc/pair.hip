@@ -194,26 +194,82 @@ __global__ __launch_bounds__(256) void step_prep_batch(const BatchSys* __restric
 
 
 
-// W: i-clusters (waves) per block; the force-only plain-LJ launch takes the
-// handle's tuned value (2, 4 or 8), every other launch 4. The force-only
-// kernels are held to 64 VGPRs (8 waves per SIMD): the per-slot force loops
-// wait on gathered slot records, which the other waves cover; the filtering
-// loop of the two-level lists would take 66 (two registers are spilled
-// around it, outside its loop).
-template <bool ENERGY, bool SOFT, int TB, int W = kPairWaves>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(!ENERGY && !SOFT ? 8 : 1))) void pair_kernel(
+// Force-only steps. W: i-clusters (waves) per block; the plain-LJ launch
+// takes the handle's tuned value (2, 4 or 8), every other launch 4. The
+// plain kernels are held to 64 VGPRs (8 waves per SIMD): the per-slot force
+// loops wait on gathered slot records, which the other waves cover; the
+// filtering loop of the two-level lists would take 66 (two registers are
+// spilled around it, outside its loop).
+template <bool SOFT, int TB, int W = kPairWaves>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(!SOFT ? 8 : 1))) void pair_kernel(
     const int* __restrict__ flags, const int* __restrict__ list_n, const uint2* __restrict__ list, int list_cap,
     const uint4* __restrict__ pk, const float2* __restrict__ ab, int nt, float cx, float cy, float cz, float rc2,
-    float beta, const int* __restrict__ s2o, float* __restrict__ frc, float* __restrict__ atom_e,
-    float* __restrict__ atom_v, float* __restrict__ atom_d, double* __restrict__ acc, int overwrite,
-    const float4* __restrict__ sc, PruneArgs pa, ExclArgs ex) {
-    pair_body<ENERGY, SOFT, TB, W>(xcd_block(gridDim.x), flags, list_n, list, list_cap, pk, ab, nt, cx, cy, cz, rc2,
-                                   beta, s2o, frc, atom_e, atom_v, atom_d, acc, overwrite, sc, pa, ex);
+    float beta, const int* __restrict__ s2o, float* __restrict__ frc, int overwrite, const float4* __restrict__ sc,
+    PruneArgs pa, ExclArgs ex) {
+    pair_body<SOFT, TB, W>(xcd_block(gridDim.x), flags, list_n, list, list_cap, pk, ab, nt, cx, cy, cz, rc2, beta, s2o,
+                           frc, overwrite, sc, pa, ex);
+}
+
+// Energies of an energy step (energy_wave): resident blocks over shares of
+// the clusters. The shares of one cluster are waves of one block, which adds
+// their per-atom sums up in wave order, so these repeat bit for bit.
+// Bound: vector issue (scan ~130 instructions per 256 listed pairs, terms
+// ~110 per 64 pairs inside the cutoff) at 4 waves per SIMD. Energies and
+// forces measured, 23,570 / 96,120 atoms at 10 A: 89 + 27 and 306 + 168 us,
+// against 369 and 1,362 us with both on 16 lanes per listed cluster pair and
+// the device library's erfc; 10,013 atoms without per-slot lists 55 + 37
+// against 191 us.
+template <bool SOFT, int TB>
+__global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void pair_energy_kernel(
+    const int* __restrict__ flags, const int* __restrict__ list_n, const uint2* __restrict__ list, int list_cap,
+    const uint4* __restrict__ pk, const float2* __restrict__ ab, int nt, float cx, float cy, float cz, float rc2,
+    float beta, int rows, const int* __restrict__ s2o, EnergyOut out, double* __restrict__ acc,
+    const float4* __restrict__ sc) {
+    __shared__ DenseLds walk[kDenseWaves];
+    __shared__ float sums[kDenseWaves][kClusterSize][3];
+    __shared__ double red[kDenseWaves][4];
+    extern __shared__ double etab[];
+    float2* sab = reinterpret_cast<float2*>(etab + rows * kErfcRow);
+    const int lane = threadIdx.x & 63, w = wave_in_block();
+    erfc_fill(etab, rows);
+    for (int k = threadIdx.x; k < nt * nt; k += blockDim.x) sab[k] = ab[k];
+    __syncthreads();
+    EnergySums T{};
+    const DenseUnits units = dense_units(flags[4]);
+    const int parts = 1 << units.split;
+    for (int base = units.base; base < units.end; base += units.step) {
+        const int u = base + w, ic = u >> units.split, part = u & (parts - 1);
+        if (u < units.end) {
+            T.e = T.v = T.d = 0.f;
+            energy_wave<SOFT, TB>(ic, part, units.split, walk[w], etab, rows, sab, list_n, list, list_cap, pk, nt, cx, cy,
+                                  cz, rc2, beta, s2o, sc, T);
+            const float o[3] = {row_sum(T.e), row_sum(T.v), row_sum(T.d)};
+            if ((lane & 15) == 0) {
+                if (parts == 1)
+                    energy_store(s2o[ic * kClusterSize + (lane >> 4)], o, out);
+                else
+                    for (int k = 0; k < 3; k++) sums[w][lane >> 4][k] = o[k];
+            }
+        }
+        if (parts > 1) {
+            __syncthreads();
+            if (u < units.end && part == 0 && lane < kClusterSize) {
+                float o[3];
+                for (int k = 0; k < 3; k++) {
+                    o[k] = sums[w][lane][k];
+                    for (int p = 1; p < parts; p++) o[k] += sums[w + p][lane][k];
+                }
+                energy_store(s2o[ic * kClusterSize + lane], o, out);
+            }
+            __syncthreads();
+        }
+    }
+    energy_totals<kDenseWaves>(T, red, acc);
 }
 
 // Batched: logical blocks are spread over the XCDs as in the single-system
 // launch, then mapped to (system, block of 4 i-clusters).
-template <bool ENERGY, bool SOFT, int TB>
+template <bool SOFT, int TB>
 __global__ __launch_bounds__(kPairWaves * 64) void pair_batch(const BatchSys* __restrict__ bs,
                                                               const int2* __restrict__ map, int nmap,
                                                               int overwrite) {
@@ -223,10 +279,42 @@ __global__ __launch_bounds__(kPairWaves * 64) void pair_batch(const BatchSys* __
     if (m.x < 0) return;
     const BatchSys& b = bs[m.x];
     const float rc = b.lj.cutoff;
-    pair_body<ENERGY, SOFT, TB>(m.y, b.nl.flags, b.nl.list_n, b.nl.list, b.nl.list_cap, b.lj.ps.pk, b.lj.d_ab,
-                            b.lj.ntypes, b.lj.cof_dr[0], b.lj.cof_dr[1], b.lj.cof_dr[2], rc * rc, b.pme.beta,
-                            b.nl.s2o, b.io.frc, ENERGY ? b.io.atom_energy : nullptr,
-                            ENERGY ? b.io.atom_virial : nullptr, nullptr, b.lj.ps.acc, overwrite, b.lj.d_sc);
+    pair_body<SOFT, TB>(m.y, b.nl.flags, b.nl.list_n, b.nl.list, b.nl.list_cap, b.lj.ps.pk, b.lj.d_ab, b.lj.ntypes,
+                        b.lj.cof_dr[0], b.lj.cof_dr[1], b.lj.cof_dr[2], rc * rc, b.pme.beta, b.nl.s2o, b.io.frc,
+                        overwrite, b.lj.d_sc, PruneArgs{}, ExclArgs{nullptr, nullptr, nullptr});
+}
+
+// Batched energies of an energy step, one i-cluster per wave; `rows` holds the largest
+// beta * cutoff of the batch.
+template <bool SOFT, int TB>
+__global__ __launch_bounds__(kPairWaves * 64) void pair_energy_batch(const BatchSys* __restrict__ bs,
+                                                                     const int2* __restrict__ map, int nmap,
+                                                                     int rows) {
+    __shared__ DenseLds walk[kPairWaves];
+    __shared__ double red[kPairWaves][4];
+    extern __shared__ double etab[];
+    const int g = xcd_block(nmap);
+    if (g < 0) return;
+    const int2 m = map[g];
+    if (m.x < 0) return;
+    const BatchSys& b = bs[m.x];
+    const int nt = b.lj.ntypes, lane = threadIdx.x & 63, w = wave_in_block();
+    float2* sab = reinterpret_cast<float2*>(etab + rows * kErfcRow);
+    erfc_fill(etab, rows);
+    for (int k = threadIdx.x; k < nt * nt; k += blockDim.x) sab[k] = b.lj.d_ab[k];
+    __syncthreads();
+    const float rc = b.lj.cutoff;
+    const EnergyOut out{b.io.atom_energy, b.io.atom_virial, nullptr};
+    EnergySums T{};
+    const int ic = m.y * kPairWaves + w;
+    if (ic < b.nl.flags[4]) {
+        energy_wave<SOFT, TB>(ic, 0, 0, walk[w], etab, rows, sab, b.nl.list_n, b.nl.list, b.nl.list_cap, b.lj.ps.pk, nt,
+                              b.lj.cof_dr[0], b.lj.cof_dr[1], b.lj.cof_dr[2], rc * rc, b.pme.beta, b.nl.s2o,
+                              b.lj.d_sc, T);
+        const float o[3] = {row_sum(T.e), row_sum(T.v), row_sum(T.d)};
+        if ((lane & 15) == 0) energy_store(b.nl.s2o[ic * kClusterSize + (lane >> 4)], o, out);
+    }
+    energy_totals<kPairWaves>(T, red, b.lj.ps.acc);
 }
 
 __global__ void add_scalar_kernel(float* a, float va, float* b, float vb) {
@@ -648,6 +736,14 @@ void snb_scratch_free(PairScratch* ps) {
     ps->waves = waves;  // a setting, not storage
 }
 
+// A launch that records its own start and end times in two events when given.
+template <class K, class... A>
+static void launch(K kernel, int grid, int threads, size_t lds, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
+                   A... args) {
+    if (e0) hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), (std::uint32_t)lds, s, e0, e1, 0u, args...);
+    else kernel<<<grid, threads, lds, s>>>(args...);
+}
+
 // Gather + pair kernel: forces added to d_frc (original order, may be NULL),
 // per-atom energies to the given arrays, FP64 totals to ps->acc.
 int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, float cutoff, const float* cof,
@@ -664,18 +760,16 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
         pa.r2 = nl->prune_r2;
         pa.in_n = nl->list_in_n;
         pa.in_list = nl->list_in;
-        pa.atom_n = nl->atom_in_n;
-        pa.atom_list = nl->atom_in;
+        pa.full_n = nl->atom_full_n;
+        pa.full_list = nl->atom_full;
         pa.atom_cap = nl->atom_in_cap;
         pa.diag = nl->flags + 11;
         pa.ref = nl->prune_ref;
         if (!sc && snb_two_level(nl)) {
-            pa.atom_on = nl->atom_out_n;
-            pa.atom_olist = nl->atom_out;
+            pa.atom_n = nl->atom_in_n;
+            pa.atom_list = nl->atom_in;
         }
     }
-    const int* list_n = nl->list_n;
-    const uint2* list = nl->list;
     int rc = scratch_ensure(ps, nl);
     if (rc) return rc;
     const int cap = ps->cap;
@@ -685,60 +779,50 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
                                                          energy, ps->acc);
         SNB_CHECK_LAUNCH();
     }
-    const int W = (!energy && !sc && (ps->waves == 2 || ps->waves == 8)) ? ps->waves : kPairWaves;
-    const int nblk = xcd_grid(ceil_div(nl->ncl_cap, W));
     const float rc2 = cutoff * cutoff;
     size_t lds = (size_t)nt * nt * sizeof(float2);
-    // the per-slot force loop of force-only plain steps reads the Coulomb
-    // force factor from a table in LDS; every fused step makes sure it
-    // exists (built by the first one, so that a prune schedule turned on
-    // later allocates nothing inside a graph capture)
-    if (fused && !energy && !sc && ps->pk_alloc) {
-        rc = ensure_coulomb_table(ps, beta, cutoff);
-        if (rc) return rc;
-    }
-    if (inner && !energy && !sc) {
-        pa.ctab = ps->ctab;
-        pa.ctab_scale = (float)kCoulTab / (cutoff * 1.0001f);
-        lds = ((lds + 15) & ~(size_t)15) + kCoulTab * sizeof(float4);
-    }
     // With timing events set, the launch itself records them (hipExtLaunchKernel
     // takes the kernel's own start and end times; events recorded around a
     // launch add the marker packets' latency, ~8 us per launch here)
     const bool timed = ps->ev_start && ps->ev_stop;
-#define SNB_PAIR(E, S, W)                      \
-    do {                                       \
-        if (nt <= 4) SNB_PAIR_TB(E, S, 2, W);  \
-        else SNB_PAIR_TB(E, S, 6, W);          \
-    } while (0)
-#define SNB_PAIR_TB(E, S, TB, W)                                                                                     \
-    do {                                                                                                            \
-        if (timed)                                                                                                  \
-            hipExtLaunchKernelGGL(pair_kernel<E, S, TB, W>, dim3(nblk), dim3(W * 64), (std::uint32_t)lds, s,         \
-                                  ps->ev_start, ps->ev_stop, 0u, nl->flags, list_n, list, nl->list_cap,              \
-                                  (const uint4*)ps->pk, ab, nt, cof[0], cof[1], cof[2], rc2, beta, nl->s2o, d_frc,   \
-                                  E ? atom_e : nullptr, E ? atom_v : nullptr, E ? atom_d : nullptr, ps->acc,         \
-                                  overwrite, sc, pa, ex);                                                            \
-        else                                                                                                        \
-            pair_kernel<E, S, TB, W><<<nblk, W * 64, lds, s>>>(                                                     \
-                nl->flags, list_n, list, nl->list_cap, ps->pk, ab, nt, cof[0], cof[1], cof[2], rc2, beta, nl->s2o,  \
-                d_frc, E ? atom_e : nullptr, E ? atom_v : nullptr, E ? atom_d : nullptr, ps->acc, overwrite, sc,    \
-                pa, ex);                                                                                            \
-    } while (0)
+    const hipEvent_t e0 = timed ? ps->ev_start : nullptr, e1 = timed ? ps->ev_stop : nullptr;
+    const uint4* pk = ps->pk;
     if (energy) {
-        if (sc) SNB_PAIR(true, true, kPairWaves);
-        else SNB_PAIR(true, false, kPairWaves);
-    } else if (sc) {
-        SNB_PAIR(false, true, kPairWaves);
-    } else if (W == 2) {
-        SNB_PAIR(false, false, 2);
-    } else if (W == 8) {
-        SNB_PAIR(false, false, 8);
-    } else {
-        SNB_PAIR(false, false, kPairWaves);
+        const int rows = erfc_rows(beta, cutoff);
+        const EnergyOut out{atom_e, atom_v, atom_d};
+        auto go = [&](auto kernel) {
+            kernel<<<dense_blocks(nl->ncl_cap), kDenseWaves * 64, lds + erfc_lds(rows), s>>>(
+                nl->flags, nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0], cof[1], cof[2], rc2, beta, rows,
+                nl->s2o, out, ps->acc, sc);
+        };
+        if (nt <= 4) sc ? go(pair_energy_kernel<true, 2>) : go(pair_energy_kernel<false, 2>);
+        else sc ? go(pair_energy_kernel<true, 6>) : go(pair_energy_kernel<false, 6>);
+        SNB_CHECK_LAUNCH();
+        if (!d_frc) return SPONGE_NB_OK;
     }
-#undef SNB_PAIR
-#undef SNB_PAIR_TB
+    // the per-slot force loop of force-only plain steps reads the Coulomb
+    // force factor from a table in LDS; every fused step makes sure it
+    // exists (built by the first one, so that a prune schedule turned on
+    // later allocates nothing inside a graph capture)
+    if (fused && !sc && ps->pk_alloc) {
+        rc = ensure_coulomb_table(ps, beta, cutoff);
+        if (rc) return rc;
+    }
+    if (inner && !sc) {
+        pa.ctab = ps->ctab;
+        pa.ctab_scale = (float)kCoulTab / (cutoff * 1.0001f);
+        lds = ((lds + 15) & ~(size_t)15) + kCoulTab * sizeof(float4);
+    }
+    const int W = (!sc && (ps->waves == 2 || ps->waves == 8)) ? ps->waves : kPairWaves;
+    const int grid = xcd_grid(ceil_div(nl->ncl_cap, W));
+    auto go = [&](auto kernel) {
+        launch(kernel, grid, W * 64, lds, s, e0, e1, nl->flags, nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0],
+               cof[1], cof[2], rc2, beta, nl->s2o, d_frc, overwrite, sc, pa, ex);
+    };
+    if (sc) nt <= 4 ? go(pair_kernel<true, 2>) : go(pair_kernel<true, 6>);
+    else if (W == 2) nt <= 4 ? go(pair_kernel<false, 2, 2>) : go(pair_kernel<false, 6, 2>);
+    else if (W == 8) nt <= 4 ? go(pair_kernel<false, 2, 8>) : go(pair_kernel<false, 6, 8>);
+    else nt <= 4 ? go(pair_kernel<false, 2>) : go(pair_kernel<false, 6>);
     SNB_CHECK_LAUNCH();
     return SPONGE_NB_OK;
 }
@@ -885,23 +969,22 @@ int snb_batch_prep(sponge_batch* b, int energy, int from_crd, int overwrite, hip
 int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s) {
     const int nmap = b->nblk[kStPair];
     const int grid = xcd_grid(nmap);
-#define SNB_PAIRB(E, S)                                                                                          \
-    do {                                                                                                         \
-        if (b->max_nt <= 4)                                                                                      \
-            pair_batch<E, S, 2><<<grid, kPairWaves * 64, b->lds_pair, s>>>(b->d, b->map[kStPair], nmap,          \
-                                                                          overwrite);                           \
-        else                                                                                                     \
-            pair_batch<E, S, 6><<<grid, kPairWaves * 64, b->lds_pair, s>>>(b->d, b->map[kStPair], nmap,          \
-                                                                          overwrite);                           \
-    } while (0)
     if (energy) {
-        if (b->soft) SNB_PAIRB(true, true);
-        else SNB_PAIRB(true, false);
-    } else {
-        if (b->soft) SNB_PAIRB(false, true);
-        else SNB_PAIRB(false, false);
+        double x = 0.0;
+        for (int k = 0; k < b->nsys; k++) x = std::max(x, (double)b->h[k].pme.beta * b->h[k].lj.cutoff);
+        const int rows = erfc_rows(x, 1.0);
+        auto go = [&](auto kernel) {
+            kernel<<<grid, kPairWaves * 64, b->lds_pair + erfc_lds(rows), s>>>(b->d, b->map[kStPair], nmap, rows);
+        };
+        if (b->max_nt <= 4) b->soft ? go(pair_energy_batch<true, 2>) : go(pair_energy_batch<false, 2>);
+        else b->soft ? go(pair_energy_batch<true, 6>) : go(pair_energy_batch<false, 6>);
+        SNB_CHECK_LAUNCH();
     }
-#undef SNB_PAIRB
+    auto go = [&](auto kernel) {
+        kernel<<<grid, kPairWaves * 64, b->lds_pair, s>>>(b->d, b->map[kStPair], nmap, overwrite);
+    };
+    if (b->max_nt <= 4) b->soft ? go(pair_batch<true, 2>) : go(pair_batch<false, 2>);
+    else b->soft ? go(pair_batch<true, 6>) : go(pair_batch<false, 6>);
     SNB_CHECK_LAUNCH();
     return SPONGE_NB_OK;
 }

@@ -13,6 +13,7 @@
 #pragma once
 #include "common.hpp"
 #include "pair_math.hpp"
+#include "dense_walk.hpp"
 
 namespace snb {
 
@@ -147,66 +148,6 @@ __device__ __forceinline__ int slot_lists(int ic, int nsl, const int* __restrict
     return __shfl(count, lane >> 4);
 }
 
-// Inner lists of the two-level form from the outer ones, without forces
-// (energy steps, whose forces come from the full list): the partners of each
-// slot of cluster ic within pa.r2 at this step's positions, in outer-list
-// order, with their counts, as pair_atoms_filter writes them. Lane (i, k), i = lane >> 4, takes
-// outer partners 2k and 2k + 1 of every 32 of atom i (one dword of offsets;
-// two dwords in flight per lane); n = the outer count of slot i, nmax the
-// longest of the four (at most atom_cap, so every offset read lies in the
-// slot's list). A partner 2k + h of a round lands after those of the lanes
-// below k, h = 0 before h = 1. Returns the inner count of slot i; the stores
-// are complete and visible to the whole wave on return.
-__device__ __forceinline__ int filter_slots(int ic, int n, int nmax, const uint4* __restrict__ pk, float cx,
-                                            float cy, float cz, const PruneArgs& pa) {
-    const int lane = threadIdx.x & 63, ii = lane >> 4, k = lane & 15;
-    const int islot = ic * kClusterSize + ii;
-    const uint4 a = pk[islot];
-    const unsigned ax = a.x & ~3u, ay = a.y & ~3u, az = a.z & ~3u;
-    const unsigned* __restrict__ lw =
-        reinterpret_cast<const unsigned*>(pa.atom_olist + (size_t)islot * pa.atom_cap);
-    unsigned short* __restrict__ out = pa.atom_list + (size_t)islot * pa.atom_cap;
-    const unsigned below = (1u << k) - 1u;
-    const int nwords = (nmax + 1) >> 1;
-    int count = 0;
-    for (int t = 0; t < nmax; t += 64) {
-        unsigned w[2];
-        uint4 b[4];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int kw = (t >> 1) + 16 * u + k;
-            w[u] = kw < nwords ? lw[kw] : 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            b[2 * u] = pk[islot + (int)(short)(w[u] & 0xffffu)];
-            b[2 * u + 1] = pk[islot + ((int)w[u] >> 16)];
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            bool keep[2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const uint4 r = b[2 * u + h];
-                const float dx = (float)(int)((r.x & ~3u) - ax) * cx;
-                const float dy = (float)(int)((r.y & ~3u) - ay) * cy;
-                const float dz = (float)(int)((r.z & ~3u) - az) * cz;
-                keep[h] = t + 32 * u + 2 * k + h < n && dr2_exact(dx, dy, dz) < pa.r2;
-            }
-            const unsigned m0 = (unsigned)(__ballot(keep[0]) >> (16 * ii)) & 0xffffu;
-            const unsigned m1 = (unsigned)(__ballot(keep[1]) >> (16 * ii)) & 0xffffu;
-            const int pos = count + __popc(m0 & below) + __popc(m1 & below);
-            if (keep[0]) out[pos] = (unsigned short)(w[u] & 0xffffu);
-            if (keep[1]) out[pos + (keep[0] ? 1 : 0)] = (unsigned short)(w[u] >> 16);
-            count += __popc(m0) + __popc(m1);
-        }
-    }
-    if (k == 0) pa.atom_n[islot] = count;
-    // other lanes read these lists next (as in slot_lists)
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    return count;
-}
-
 // Slot records of the per-slot force loops through a structured buffer
 // resource (16-byte records) over the records and their copies on either
 // side: a partner's record is one indexed buffer load at the slot's own
@@ -242,7 +183,7 @@ __device__ __forceinline__ uint4 slot_record(const SlotRecords& r, unsigned w) {
 // factor from its cubic piece in LDS, else from the fitted erfc): the
 // displacement and r^2 to the partner record b, and the factor f of the
 // pair force f (dx, dy, dz) on atom i; 0 unless listed and r < rc. The pair
-// terms are pair_body's, in FP32.
+// terms are pair_wave's, in FP32.
 template <int TB, bool TABLE>
 __device__ __forceinline__ float slot_pair(const uint4 b, unsigned ax, unsigned ay, unsigned az, float qi,
                                            const float2* srow, const float4* stab, float cx, float cy, float cz,
@@ -320,10 +261,11 @@ __device__ __forceinline__ void slot_finish(int islot, int k, const uint4* __res
 // too (offsets left from earlier prunes, or zero: always inside the records
 // and their copies) and are masked out.
 template <int TB, bool TABLE>
-__device__ __forceinline__ void pair_atoms(int ic, int n, int nmax, const uint4* __restrict__ pk, const float2* sab,
-                                           const float4* stab, int nt, float cx, float cy, float cz, float rc2,
-                                           float beta, const int* __restrict__ s2o, float* __restrict__ frc,
-                                           int overwrite, const PruneArgs& pa, const ExclArgs& ex) {
+__device__ __forceinline__ void pair_atoms(int ic, const unsigned short* __restrict__ lists, int n, int nmax,
+                                           const uint4* __restrict__ pk, const float2* sab, const float4* stab,
+                                           int nt, float cx, float cy, float cz, float rc2, float beta,
+                                           const int* __restrict__ s2o, float* __restrict__ frc, int overwrite,
+                                           const PruneArgs& pa, const ExclArgs& ex) {
     const int lane = threadIdx.x & 63, ii = lane >> 4, k = lane & 15;
     const int islot = ic * kClusterSize + ii;
     const uint4 a = pk[islot];
@@ -332,8 +274,7 @@ __device__ __forceinline__ void pair_atoms(int ic, int n, int nmax, const uint4*
     const int ti = TB == 2 ? (int)(a.x & 3u) : unpack_type(a);
     const float2* srow = sab + ti * nt;
     const float mlog2e_b2 = -1.4426950408889634f * (beta * beta);
-    const unsigned* __restrict__ lw =
-        reinterpret_cast<const unsigned*>(pa.atom_list + (size_t)islot * pa.atom_cap);
+    const unsigned* __restrict__ lw = reinterpret_cast<const unsigned*>(lists + (size_t)islot * pa.atom_cap);
     const int nwords = (nmax + 1) >> 1;  // atom_cap is even: the dword stays inside the slot's list
     float fix = 0.f, fiy = 0.f, fiz = 0.f;
     const SlotRecords rec = slot_records(pk, islot, pa);
@@ -396,7 +337,7 @@ __device__ __forceinline__ void pair_atoms_filter(int ic, int n, int nmax, const
     const float2* srow = sab + ti * nt;
     const float mlog2e_b2 = -1.4426950408889634f * (beta * beta);
     const unsigned lo = (unsigned)islot * (unsigned)pa.atom_cap;  // below 2^32: the lists' allocation
-    const unsigned* __restrict__ lw = reinterpret_cast<const unsigned*>(pa.atom_olist) + (lo >> 1);
+    const unsigned* __restrict__ lw = reinterpret_cast<const unsigned*>(pa.full_list) + (lo >> 1);
     const int nwords = (nmax + 1) >> 1;
     float fix = 0.f, fiy = 0.f, fiz = 0.f;
     const SlotRecords rec = slot_records(pk, islot, pa);
@@ -429,6 +370,45 @@ __device__ __forceinline__ void pair_atoms_filter(int ic, int n, int nmax, const
     slot_finish(islot, k, pk, ax, ay, az, qi, cx, cy, cz, beta, s2o, frc, overwrite, ex, fix, fiy, fiz);
 }
 
+// Which lists this step writes, from the count of steps since the rebuild
+// (flags[10], advanced by the step's gather after this kernel). Plain LJ
+// keeps per-slot lists: the full ones (every pair of the list, written by each
+// rebuild and on renewing steps, the first after a new prune setting) and, with
+// a prune radius below rc + skin ("two levels"), the inner ones (the full
+// lists' pairs within pa.r2), written on scheduled steps (every pa.interval-th
+// and the first after a rebuild), on voted ones (the prep kernel found an atom
+// that moved more than half the prune margin since the last prune) and on
+// renewing ones. Soft-core LJ prunes the cluster-pair list to pa.r2 on
+// scheduled and voted steps. A step that prunes by distance keeps the slot
+// records it pruned at.
+struct ListStep {
+    bool slots, two, write_full, write_inner;
+};
+template <bool SOFT>
+__device__ __forceinline__ ListStep list_step(int ic, const int* __restrict__ flags, const uint4* __restrict__ pk,
+                                              const PruneArgs& pa) {
+    ListStep t{false, false, false, false};
+    if (pa.interval <= 0) return t;
+    const int lane = threadIdx.x & 63;
+    t.slots = !SOFT;
+    t.two = !SOFT && pa.atom_list != nullptr;
+    const int c = flags[10] + 1;
+    const bool renew = pa.diag[3] == c;
+    const bool scheduled = c <= 1 || (c - 1) % pa.interval == 0;
+    const bool voted = pa.diag[2] == c;
+    t.write_full = !SOFT && renew;
+    t.write_inner = SOFT ? scheduled || voted : t.two && (renew || scheduled || voted);
+    if (t.write_inner && lane < kClusterSize) pa.ref[ic * kClusterSize + lane] = pk[ic * kClusterSize + lane];
+    if (voted && !scheduled && (SOFT || t.two) && ic == 0 && lane == 0) atomicAdd(pa.diag + 4, 1);
+    return t;
+}
+
+// Largest of the four slots' counts (n: the count of slot lane >> 4).
+__device__ __forceinline__ int longest(int n) {
+    return max(max(__shfl(n, 0), __shfl(n, 16)), max(__shfl(n, 32), __shfl(n, 48)));
+}
+
+// Force-only steps: one i-cluster per wave.
 // Cutoff test shared with the oracle: FP32 dr2 = (dx*dx + dy*dy) + dz*dz with
 // every operation rounded (the neighbor list's expression) against rc*rc in
 // FP32, so both sides agree on every pair, including those within one ulp of
@@ -440,96 +420,47 @@ __device__ __forceinline__ void pair_atoms_filter(int ic, int n, int nmax, const
 // waves that meet such a pair.
 // TB = 2: every type index is below 4 and sits in the x coordinate's low bits
 // alone (two instructions fewer per pair); TB = 6: the general 6-bit index.
-template <bool ENERGY, bool SOFT, int TB>
+template <bool SOFT, int TB>
 __device__ __forceinline__ void pair_wave(
     int ic, const float2* sab, const float4* stab, const int* __restrict__ flags, const int* __restrict__ list_n,
     const uint2* __restrict__ list, int list_cap, const uint4* __restrict__ pk, int nt, float cx, float cy, float cz,
-    float rc2, float beta, const int* __restrict__ s2o, float* __restrict__ frc, float* __restrict__ atom_e,
-    float* __restrict__ atom_v, float* __restrict__ atom_d, double* __restrict__ acc, int overwrite,
+    float rc2, float beta, const int* __restrict__ s2o, float* __restrict__ frc, int overwrite,
     const float4* __restrict__ sc, const PruneArgs& pa, const ExclArgs& ex) {
     const int lane = threadIdx.x & 63;
-    // Inner lists (pa.interval > 0). c = this step's number since the
-    // rebuild (the count of completed steps is advanced by the step's
-    // gather, after this kernel); a step is scheduled every pa.interval-th
-    // step and on the first after a rebuild, voted when its prep kernel
-    // found an atom that moved more than half the prune margin since the
-    // last prune, and renewing when it is the first after a new prune
-    // setting.
-    // Plain LJ keeps per-slot lists (pa.atom_list; force-only steps read
-    // them, energy steps the full list). One level (a prune radius at or
-    // beyond rc + skin): the lists hold every pair of the full list, written
-    // by each rebuild (nl_slot_lists_kernel) and on renewing steps; no other
-    // step prunes and nothing is voted (the pairs are those of the list's
-    // own radius at the rebuild). Two levels
-    // (pa.atom_olist set): those lists are the outer ones, and the inner
-    // lists, the outer pairs within pa.r2, are written on scheduled, voted
-    // and renewing steps. Soft-core LJ prunes the cluster-pair list to pa.r2
-    // on scheduled and voted steps and reads the pruned one in between. A
-    // step that prunes by distance keeps the slot records it pruned at.
-    const bool two = pa.atom_olist != nullptr;
-    const bool slots = !SOFT && pa.atom_list != nullptr && pa.interval > 0;
-    bool use_inner = false, write_inner = false, write_outer = false;
-    if (pa.interval > 0) {
-        const int c = flags[10] + 1;
-        // the rebuild writes the lists of a new period; a new prune setting
-        // has the next step write them
-        const bool renew = pa.diag[3] == c;
-        const bool scheduled = c <= 1 || (c - 1) % pa.interval == 0;
-        const bool voted = pa.diag[2] == c;
-        if (slots) {
-            write_outer = two && renew;
-            write_inner = two ? renew || scheduled || voted : renew;
-        } else {
-            write_inner = scheduled || voted;
-        }
-        use_inner = !write_inner;
-        if (write_inner && lane < kClusterSize) pa.ref[ic * kClusterSize + lane] = pk[ic * kClusterSize + lane];
-        if (voted && !scheduled && (!slots || two) && ic == 0 && lane == 0) atomicAdd(pa.diag + 4, 1);
-    }
-    if (slots && !ENERGY) {
+    const ListStep step = list_step<SOFT>(ic, flags, pk, pa);
+    if (step.slots) {
         if (ic == 0 && lane == 0) atomicAdd(pa.diag + 1, 1);
-        if (two && write_inner) {
-            const int n = write_outer ? slot_lists(ic, flags[3], list_n, list, list_cap, pa, pa.atom_olist, pa.atom_on)
-                                      : pa.atom_on[ic * kClusterSize + (lane >> 4)];
-            const int nmax = max(max(__shfl(n, 0), __shfl(n, 16)), max(__shfl(n, 32), __shfl(n, 48)));
-            if (nmax <= pa.atom_cap) {
+        const bool filter = step.write_inner;
+        const bool inner = step.two && !filter;
+        int n;
+        if (step.write_full) n = slot_lists(ic, flags[3], list_n, list, list_cap, pa, pa.full_list, pa.full_n);
+        else n = (inner ? pa.atom_n : pa.full_n)[ic * kClusterSize + (lane >> 4)];
+        const int nmax = longest(n);
+        if (nmax <= pa.atom_cap) {
+            if (filter) {
                 if (stab)
                     pair_atoms_filter<TB, true>(ic, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
                                                 overwrite, pa, ex);
                 else
                     pair_atoms_filter<TB, false>(ic, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
                                                  overwrite, pa, ex);
-                return;
-            }
-            // an outer list overflowed: the inner lists follow it to the
-            // full list until the outer ones are written again
-            if (lane < kClusterSize) pa.atom_n[ic * kClusterSize + lane] = pa.atom_cap + 1;
-        } else {
-            const int n = write_inner ? slot_lists(ic, flags[3], list_n, list, list_cap, pa, pa.atom_list, pa.atom_n)
-                                      : pa.atom_n[ic * kClusterSize + (lane >> 4)];
-            const int nmax = max(max(__shfl(n, 0), __shfl(n, 16)), max(__shfl(n, 32), __shfl(n, 48)));
-            if (nmax <= pa.atom_cap) {
+            } else {
+                const unsigned short* lists = inner ? pa.atom_list : pa.full_list;
                 if (stab)
-                    pair_atoms<TB, true>(ic, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc, overwrite,
-                                         pa, ex);
+                    pair_atoms<TB, true>(ic, lists, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
+                                         overwrite, pa, ex);
                 else
-                    pair_atoms<TB, false>(ic, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc, overwrite,
-                                          pa, ex);
-                return;
+                    pair_atoms<TB, false>(ic, lists, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
+                                          overwrite, pa, ex);
             }
+            return;
         }
-        write_inner = false;  // a slot overflowed: this cluster's forces from the full list
-        write_outer = false;
+        // a list overflowed: this cluster's forces come from the full list,
+        // and its inner lists follow until the full ones are written again
+        if (filter && lane < kClusterSize) pa.atom_n[ic * kClusterSize + lane] = pa.atom_cap + 1;
     }
-    // energy steps that write the per-slot lists take every listed pair from
-    // the full list (the outer ones in the two-level form, which then writes
-    // the inner ones from them below)
-    const bool write_atoms = slots && (two ? write_outer : write_inner);
-    const bool write_cluster = !slots && write_inner;
-    unsigned short* const wl = two ? pa.atom_olist : pa.atom_list;
-    int* const wn = two ? pa.atom_on : pa.atom_n;
-    const float wr2 = slots ? __builtin_huge_valf() : pa.r2;
-    if (slots) use_inner = false;
+    const bool write_cluster = SOFT && step.write_inner;
+    const bool use_inner = SOFT && pa.interval > 0 && !write_cluster;
     const int ii = lane & 3, jj = (lane >> 2) & 3, g = lane >> 4, bit = lane & 15;
     const int islot = ic * kClusterSize + ii;
     const uint4 a = pk[islot];
@@ -538,17 +469,11 @@ __device__ __forceinline__ void pair_wave(
     const int ti = TB == 2 ? (int)(a.x & 3u) : unpack_type(a);
     const float2* srow = sab + ti * nt;
     const float mlog2e_b2 = -1.4426950408889634f * (beta * beta);
-    int ai = 0;
-    if (ENERGY) ai = s2o[islot];
     float fix = 0.f, fiy = 0.f, fiz = 0.f;
-    float eie = 0.f, eiv = 0.f, eid = 0.f;
-    double tlj = 0.0, tdir = 0.0, tvir = 0.0, tcnt = 0.0;
     const int n = use_inner ? pa.in_n[ic] : list_n[ic];
     const uint2* lst = (use_inner ? pa.in_list : list) + (size_t)ic * list_cap;
     uint2* inner_out = write_cluster ? pa.in_list + (size_t)ic * list_cap : nullptr;
-    int inner_count = 0, atom_count = 0;
-    bool atom_far = false;
-    const int nsl = flags[3];
+    int inner_count = 0;
     for (int base = 0; base < n; base += 64) {
         // 64 list entries (16 iterations of 4 j-clusters) held one per lane.
         const uint2 my = base + lane < n ? lst[base + lane] : make_uint2((unsigned)ic, 0u);
@@ -567,110 +492,40 @@ __device__ __forceinline__ void pair_wave(
             const float dz = (float)(int)((b.z & ~3u) - az) * cz;
             const float r2 = dr2_exact(dx, dy, dz);
             const bool in = ((m >> bit) & 1u) && r2 < rc2;
-            if (write_inner) {
-                const bool keep = ((m >> bit) & 1u) && r2 < wr2;
-                const unsigned long long kb = __ballot(keep);
-                if (write_cluster) {
-                    const unsigned mk = (unsigned)(kb >> (g * 16)) & 0xffffu;
-                    const bool leader = (lane & 15) == 0 && mk != 0u;
-                    const unsigned long long lb2 = __ballot(leader);
-                    if (leader)
-                        inner_out[inner_count + __popcll(lb2 & ((1ull << lane) - 1ull))] =
-                            make_uint2((unsigned)jc, mk);
-                    inner_count += __popcll(lb2);
-                } else {
-                    // lanes ii, ii + 4, ... append to slot ii's list in lane order
-                    const unsigned long long mi = kb & (0x1111111111111111ull << ii);
-                    const int pos = atom_count + __popcll(mi & ((1ull << lane) - 1ull));
-                    int off = 0;
-                    const bool reach = slot_offset(islot, jc * kClusterSize + jj, nsl, off);
-                    atom_far = atom_far || (keep && !reach);
-                    if (keep && pos < pa.atom_cap) wl[(size_t)islot * pa.atom_cap + pos] = (unsigned short)off;
-                    atom_count += __popcll(mi);
-                }
+            if (write_cluster) {
+                const unsigned long long kb = __ballot(((m >> bit) & 1u) && r2 < pa.r2);
+                const unsigned mk = (unsigned)(kb >> (g * 16)) & 0xffffu;
+                const bool leader = (lane & 15) == 0 && mk != 0u;
+                const unsigned long long lb2 = __ballot(leader);
+                if (leader)
+                    inner_out[inner_count + __popcll(lb2 & ((1ull << lane) - 1ull))] = make_uint2((unsigned)jc, mk);
+                inner_count += __popcll(lb2);
             }
             // masked lanes (padding, the atom itself) may give inf / NaN
             // below; the final select discards them
-            const float r2s = r2;
-            const float rinv = __builtin_amdgcn_rsqf(r2s);
+            const float rinv = __builtin_amdgcn_rsqf(r2);
             const float rinv2 = rinv * rinv;
             const float rinv6 = rinv2 * rinv2 * rinv2;
             const int tj = TB == 2 ? (int)(b.x & 3u) : unpack_type(b);
             const float2 AB = srow[tj];
             float flj = (AB.y - AB.x * rinv6) * rinv6 * rinv2;
-            const float x = beta * (r2s * rinv);
-            const float ex = __builtin_amdgcn_exp2f(mlog2e_b2 * r2s);
+            const float x = beta * (r2 * rinv);
+            const float ex = __builtin_amdgcn_exp2f(mlog2e_b2 * r2);
             const float ecx = erfcx_poly(x);
             const float qq = qi * __uint_as_float(b.w);
             float fc = qq * ex * fmaf(kTwoOverSqrtPi, x, ecx) * rinv * rinv2;
-            bool sp = false;
-            float4 s0 = make_float4(0.f, 0.f, 0.f, 0.f), s1 = s0;
-            if (SOFT) {
-                sp = in && AB.x < 0.f;
-                if (sp) {
-                    s0 = sc[ti * nt + tj];
-                    s1 = sc[nt * nt + ti * nt + tj];
-                    soft_pair(r2s, qq, beta, mlog2e_b2, s0, s1, flj, fc);
-                }
-            }
+            if (SOFT && in && AB.x < 0.f)
+                soft_pair(r2, qq, beta, mlog2e_b2, sc[ti * nt + tj], sc[nt * nt + ti * nt + tj], flj, fc);
             const float f = in ? flj - fc : 0.f;
             fix += f * dx;
             fiy += f * dy;
             fiz += f * dz;
-            if (ENERGY) {
-                // Energy steps evaluate the pair energies in FP64 from the exact
-                // integer displacement: the totals are nets of large cancelling
-                // terms, which FP32 terms cannot hold to 1e-6. Each unordered
-                // pair is credited once, to its lower-index atom, as the
-                // reference's half list does.
-                const int aj = s2o[jc * kClusterSize + jj];
-                if (in && ai < aj) {
-                    const double ddx = (double)(int)((b.x & ~3u) - ax) * (double)cx;
-                    const double ddy = (double)(int)((b.y & ~3u) - ay) * (double)cy;
-                    const double ddz = (double)(int)((b.z & ~3u) - az) * (double)cz;
-                    const double dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
-                    double elj, edir, vlj;
-                    if (SOFT && sp) {
-                        soft_pair_energy(dr2, (double)qi * (double)__uint_as_float(b.w), (double)beta, s0, s1, elj,
-                                         edir, vlj);
-                    } else {
-                        const double dr = sqrt(dr2);
-                        const double ir2 = 1.0 / dr2, ir6 = ir2 * ir2 * ir2;
-                        elj = ((double)AB.x * (1.0 / 12.0) * ir6 - (double)AB.y * (1.0 / 6.0)) * ir6;
-                        edir = (double)qi * (double)__uint_as_float(b.w) * erfc((double)beta * dr) / dr;
-                        vlj = ((double)AB.x * ir6 - (double)AB.y) * ir6;
-                    }
-                    tlj += elj;
-                    tdir += edir;
-                    tvir += vlj;
-                    tcnt += 1.0;
-                    eie += (float)(elj + edir);
-                    eiv += (float)vlj;
-                    eid += (float)edir;
-                }
-            }
             b = bn;
             m = mn;
             jc = jcn;
         }
     }
     if (write_cluster && lane == 0) pa.in_n[ic] = inner_count;
-    if (write_atoms && (__ballot(atom_far) & (0x1111111111111111ull << ii))) atom_count = pa.atom_cap + 1;
-    if (write_atoms && lane < kClusterSize) {
-        wn[islot] = atom_count;
-        if (atom_count > pa.atom_cap) atomicOr(pa.diag, 1);
-    }
-    if (ENERGY && slots && two && write_inner) {
-        // the inner lists from the outer ones (no force: this step's forces
-        // come from the full list)
-        if (write_atoms) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        const int no = pa.atom_on[ic * kClusterSize + (lane >> 4)];
-        const int nomax = max(max(__shfl(no, 0), __shfl(no, 16)), max(__shfl(no, 32), __shfl(no, 48)));
-        if (nomax <= pa.atom_cap)
-            filter_slots(ic, no, nomax, pk, cx, cy, cz, pa);
-        else if (lane < kClusterSize)
-            pa.atom_n[ic * kClusterSize + lane] = pa.atom_cap + 1;
-    }
     if (ex.start) {
         // this cluster's atoms: lane (ii, k) takes the k-th exclusion partner
         // of atom ii, 16 per pass
@@ -683,72 +538,150 @@ __device__ __forceinline__ void pair_wave(
         fix += __shfl_xor(fix, o);
         fiy += __shfl_xor(fiy, o);
         fiz += __shfl_xor(fiz, o);
-        if (ENERGY) {
-            eie += __shfl_xor(eie, o);
-            eiv += __shfl_xor(eiv, o);
-            eid += __shfl_xor(eid, o);
-        }
     }
     if (lane < 4) {
         const int at = s2o[islot];
-        if (at >= 0) {
-            if (frc) {
-                // every atom has exactly one slot, so this is the only writer
-                if (overwrite) {
-                    frc[3 * at] = fix;
-                    frc[3 * at + 1] = fiy;
-                    frc[3 * at + 2] = fiz;
-                } else {
-                    frc[3 * at] += fix;
-                    frc[3 * at + 1] += fiy;
-                    frc[3 * at + 2] += fiz;
-                }
+        if (at >= 0 && frc) {
+            // every atom has exactly one slot, so this is the only writer
+            if (overwrite) {
+                frc[3 * at] = fix;
+                frc[3 * at + 1] = fiy;
+                frc[3 * at + 2] = fiz;
+            } else {
+                frc[3 * at] += fix;
+                frc[3 * at + 1] += fiy;
+                frc[3 * at + 2] += fiz;
             }
-            if (ENERGY) {
-                if (atom_e) atom_e[at] += eie;
-                if (atom_v) atom_v[at] += eiv;
-                if (atom_d) atom_d[at] = eid;
-            }
-        }
-    }
-    if (ENERGY) {
-        tlj = wave_sum(tlj);
-        tdir = wave_sum(tdir);
-        tvir = wave_sum(tvir);
-        tcnt = wave_sum(tcnt);
-        if (lane == 0) {
-            atomicAdd(acc + SPONGE_PART_LJ, tlj);
-            atomicAdd(acc + SPONGE_PART_DIRECT, tdir);
-            atomicAdd(acc + SPONGE_PART_LJ_VIRIAL, tvir);
-            atomicAdd(acc + SPONGE_PART_PAIRS_IN, tcnt);
         }
     }
 }
 
-
-// One block of the pair kernel: the LJ (A, B) table into LDS, then one
-// i-cluster per wave (logical block lb covers clusters W lb .. W lb + W - 1).
-template <bool ENERGY, bool SOFT, int TB, int W = kPairWaves>
+// One block of the force-only pair kernel: the LJ (A, B) table and, when
+// given, the Coulomb table into LDS, then one i-cluster per wave (logical
+// block lb covers clusters W lb .. W lb + W - 1).
+template <bool SOFT, int TB, int W = kPairWaves>
 __device__ __forceinline__ void pair_body(
     int lb, const int* __restrict__ flags, const int* __restrict__ list_n, const uint2* __restrict__ list,
     int list_cap, const uint4* __restrict__ pk, const float2* __restrict__ ab, int nt, float cx, float cy, float cz,
-    float rc2, float beta, const int* __restrict__ s2o, float* __restrict__ frc, float* __restrict__ atom_e,
-    float* __restrict__ atom_v, float* __restrict__ atom_d, double* __restrict__ acc, int overwrite,
-    const float4* __restrict__ sc, PruneArgs pa = PruneArgs{},
-    ExclArgs ex = ExclArgs{nullptr, nullptr, nullptr}) {
+    float rc2, float beta, const int* __restrict__ s2o, float* __restrict__ frc, int overwrite,
+    const float4* __restrict__ sc, const PruneArgs& pa, const ExclArgs& ex) {
     extern __shared__ float2 sab[];
     for (int k = threadIdx.x; k < nt * nt; k += blockDim.x) sab[k] = ab[k];
     // the Coulomb table after the LJ table (16-byte aligned), when given
     float4* stab = nullptr;
-    if (!ENERGY && !SOFT && pa.ctab) {
+    if (pa.ctab) {
         stab = reinterpret_cast<float4*>(reinterpret_cast<char*>(sab) + ((nt * nt * 8 + 15) & ~15));
         for (int k = threadIdx.x; k < kCoulTab; k += blockDim.x) stab[k] = pa.ctab[k];
     }
     __syncthreads();
     const int ic = lb * W + (int)(threadIdx.x >> 6);
     if (lb < 0 || ic >= flags[4]) return;
-    pair_wave<ENERGY, SOFT, TB>(ic, sab, stab, flags, list_n, list, list_cap, pk, nt, cx, cy, cz, rc2, beta, s2o,
-                                frc, atom_e, atom_v, atom_d, acc, overwrite, sc, pa, ex);
+    pair_wave<SOFT, TB>(ic, sab, stab, flags, list_n, list, list_cap, pk, nt, cx, cy, cz, rc2, beta, s2o, frc,
+                        overwrite, sc, pa, ex);
+}
+
+// ---- energy steps -----------------------------------------------------------
+// Forces come from the force-only kernel (with the lists it reads or writes);
+// the energies of every pair of the full list from energy_wave.
+
+// Sums of an energy step: the FP32 per-atom energies of lane (i, k)'s pairs
+// and its FP64 totals.
+struct EnergySums {
+    float e, v, d;
+    double lj, dir, vir;
+    int pairs;
+};
+
+// Pair energies of one i-cluster, or one wave's share of it (dense_walk: full
+// waves of pairs inside the cutoff), in FP64 from the exact integer
+// displacement: the totals are nets of large cancelling terms, which FP32
+// terms cannot hold to 1e-6. Each unordered pair is credited once, to its
+// lower-index atom, as the reference's half list does.
+template <bool SOFT, int TB>
+__device__ __forceinline__ void energy_wave(int ic, int part, int split, DenseLds& L, const double* etab, int rows,
+                                            const float2* sab, const int* __restrict__ list_n,
+                                            const uint2* __restrict__ list, int list_cap,
+                                            const uint4* __restrict__ pk, int nt, float cx, float cy, float cz,
+                                            float rc2, float beta, const int* __restrict__ s2o,
+                                            const float4* __restrict__ sc, EnergySums& S) {
+    const int islot = ic * kClusterSize + (int)((threadIdx.x & 63) >> 4);
+    const uint4 a = pk[islot];
+    const int ti = TB == 2 ? (int)(a.x & 3u) : unpack_type(a);
+    const float2* srow = sab + ti * nt;
+    const double beta64 = (double)beta * kErfcPieces;
+    dense_walk<kLowerAtom>(ic, pk, s2o, list_n, list, list_cap, cx, cy, cz, rc2, part, split, L,
+                           [&](bool in, int jslot) {
+        const uint4 b = pk[jslot];
+        const int tj = TB == 2 ? (int)(b.x & 3u) : unpack_type(b);
+        const float2 AB = srow[tj];
+        const double dx = (double)(int)((b.x & ~3u) - (a.x & ~3u)) * (double)cx;
+        const double dy = (double)(int)((b.y & ~3u) - (a.y & ~3u)) * (double)cy;
+        const double dz = (double)(int)((b.z & ~3u) - (a.z & ~3u)) * (double)cz;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const double qq = (double)__uint_as_float(a.w) * (double)__uint_as_float(b.w);
+        if (in) {
+            double elj, edir, vlj;
+            if (SOFT && AB.x < 0.f) {
+                soft_pair_energy(r2, qq, (double)beta, sc[ti * nt + tj], sc[nt * nt + ti * nt + tj], elj, edir, vlj);
+            } else {
+                double rinv, r;
+                rsqrt_f64(r2, rinv, r);
+                const double ir2 = rinv * rinv, ir6 = ir2 * ir2 * ir2;
+                // (A r^-6 / 12 - B / 6) r^-6 of the stored x12 / x6 tables
+                elj = fma((double)AB.x, ir6, -2.0 * (double)AB.y) * ir6 * (1.0 / 12.0);
+                vlj = ((double)AB.x * ir6 - (double)AB.y) * ir6;
+                edir = qq * erfc_at(etab, rows, beta64 * r) * rinv;
+            }
+            S.lj += elj;
+            S.dir += edir;
+            S.vir += vlj;
+            S.pairs += 1;
+            S.e += (float)(elj + edir);
+            S.v += (float)vlj;
+            S.d += (float)edir;
+        }
+    });
+}
+
+// Sum over the 16 lanes of an i atom, valid in all of them.
+__device__ __forceinline__ float row_sum(float v) {
+    v += dpp_row_ror<8>(v);
+    v += dpp_row_ror<4>(v);
+    v += dpp_row_ror<2>(v);
+    return v + dpp_row_ror<1>(v);
+}
+
+struct EnergyOut {
+    float* e;
+    float* v;
+    float* d;
+};
+
+// Adds one atom's energies (o: e, v, d) to the caller's arrays; every atom
+// has exactly one slot, so this is the only writer.
+__device__ __forceinline__ void energy_store(int at, const float* o, const EnergyOut& out) {
+    if (at < 0) return;
+    if (out.e) out.e[at] += o[0];
+    if (out.v) out.v[at] += o[1];
+    if (out.d) out.d[at] = o[2];
+}
+
+// The block's totals to acc: one atomic per total and block.
+template <int W>
+__device__ __forceinline__ void energy_totals(const EnergySums& S, double (*red)[4], double* __restrict__ acc) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double t[4] = {wave_sum(S.lj), wave_sum(S.dir), wave_sum(S.vir), wave_sum((double)S.pairs)};
+    if (lane < 4) red[w][lane] = lane == 0 ? t[0] : lane == 1 ? t[1] : lane == 2 ? t[2] : t[3];
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        double s = 0.0;
+        for (int k = 0; k < W; k++) s += red[k][threadIdx.x];
+        const int slot = threadIdx.x == 0   ? SPONGE_PART_LJ
+                         : threadIdx.x == 1 ? SPONGE_PART_DIRECT
+                         : threadIdx.x == 2 ? SPONGE_PART_LJ_VIRIAL
+                                            : SPONGE_PART_PAIRS_IN;
+        atomicAdd(acc + slot, s);
+    }
 }
 
 }  // namespace snb

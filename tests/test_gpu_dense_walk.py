@@ -56,3 +56,49 @@ def test_windows(waters, cutoff, skin, beta):
         err = np.abs(got[:, :7] - ref) / np.maximum(1.0, np.abs(ref))
         say(f"    dq {dq is not None}: worst relative error {err.max():.2e}")
         assert err.max() <= TOL, (dq is not None, np.unravel_index(err.argmax(), err.shape))
+
+
+@pytest.mark.parametrize("waters,cutoff,skin", [(27, 3.5, 0.5), (216, 9.2, 0.1), (729, 7.0, 1.0)])
+@pytest.mark.parametrize("soft", [False, True])
+def test_energies(waters, cutoff, skin, soft):
+    """Per-atom energies, totals and pair count of an energy step, and the
+    same forces bit for bit as a force-only step's. Per-atom arrays are FP32
+    sums of FP64 terms: 1e-6 of their size; totals 1e-9 of the terms' scale,
+    for soft-core handles 2^-23 of it (their pair records are FP32, the
+    oracle's FP64: half an ulp in lambda-mixed A, B and sigma^6 terms)."""
+    import torch
+    from sponge_amd import nb
+    length = (waters * system.WATER_VOLUME) ** (1.0 / 3.0)
+    if soft:
+        if waters < 100:
+            pytest.skip("no room for the solute")
+        s = system.fep_mixed(system.fep_system(waters, 0.35, seed=5, cutoff=cutoff, skin=skin))
+    else:
+        s = system.water_box(waters, round(length, 3), seed=3, cutoff=cutoff, skin=skin)
+    say(f"[case] energies waters {waters} n {s.n} box {s.box[0]:.3f} cutoff {cutoff} soft {soft}")
+    eng = nb.NonbondedEngine(s, refresh_interval=0)
+    eng.update_neighbor_list(forced=1)
+    eng.force_step(0, 0, from_crd=True, overwrite=True)
+    torch.cuda.synchronize()
+    eng.nl.check()
+    f = eng.frc.cpu().numpy()
+    eng.lj.LJ_PME_Direct_Force_With_Atom_Energy_And_Virial(
+        eng.nl, eng.uint_crd, eng.charge, eng.frc.zero_(), eng.pme.beta, 1, eng.atom_energy, 1, eng.atom_virial,
+        eng.atom_direct)
+    g = eng.frc.cpu().numpy()
+    eng.lj.LJ_PME_Direct_Force_With_Atom_Energy_And_Virial(eng.nl, eng.uint_crd, eng.charge, eng.frc.zero_(),
+                                                           eng.pme.beta)
+    assert np.array_equal(g, eng.frc.cpu().numpy()) and np.isfinite(f).all()
+    u = eng.uint_crd.cpu().numpy().view(np.uint32)
+    pairs = oracle.nl_brute(s, u)
+    ref = (oracle.direct_soft if soft else oracle.direct)(s, u, pairs, eng.pme.beta)
+    for got, want in ((eng.atom_energy, ref["atom_energy"]), (eng.atom_virial, ref["atom_virial"]),
+                      (eng.atom_direct, ref["atom_direct"])):
+        got = got.cpu().numpy().astype(np.float64)
+        assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max()
+    eng.force_step(1, 1, from_crd=True, overwrite=True)
+    p = eng.energy_parts()
+    scale = np.abs(ref["atom_energy"]).sum()
+    assert p["pairs_in"] == ref["n_in"]
+    for k, v in (("lj", ref["e_lj"]), ("direct", ref["e_direct"])):
+        assert abs(p[k] - v) <= (2.0 ** -23 if soft else 1e-9) * scale, (k, p[k], v)

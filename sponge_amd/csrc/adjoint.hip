@@ -22,12 +22,12 @@
 
 #include "common.hpp"
 #include "pair_math.hpp"
+#include "dense_walk.hpp"
 
 using namespace snb;
 
 namespace {
 
-constexpr int kAdjWaves = 4;
 constexpr int kAdjMaxTypes = 8;  // per-lane accumulators of the table gradients
 
 struct AdjScratch {
@@ -120,113 +120,127 @@ __device__ __forceinline__ int pidx(int a, int b) {
     return hi * (hi + 1) / 2 + lo;
 }
 
-// One wave per i-cluster over the full cluster-pair list (the forward
-// kernel's layout and cutoff predicate). LOSS = false: energy gradient
-// (potential of atom i; half of every ordered pair's table term, since the
-// full list holds each unordered pair twice). LOSS = true: force-matching
-// gradient. gq[atom] is assigned; the table gradients are reduced per
-// (type i, type j) over the wave and added to gA / gB in FP64.
-template <bool LOSS>
-__global__ __launch_bounds__(kAdjWaves * 64) void adj_pair_kernel(
+// Pair gradients (dense_walk: full waves of pairs inside the cutoff, each from
+// both sides; the forward cutoff predicate). LOSS = false: energy gradient
+// (potential of atom i; half of every ordered pair's table term, since each
+// unordered pair comes twice). LOSS = true: force-matching gradient.
+// gq[atom] is assigned; the table gradients are kept per partner type (NT of
+// them, types below NT) in registers, a cluster's go to the wave's bins in
+// LDS by pair type, and the blocks' to gA / gB in FP64.
+// Bound: vector issue (48M vector instructions at 23,570 atoms, 10 A: 80 us of
+// issue at 4 waves per SIMD). Measured 495 -> 106 us there, 2,001 -> 361 us at
+// 96,120 atoms and 105 -> 29 us (loss, 3,006 atoms), against 16 lanes per
+// listed cluster pair with every type's accumulators added on every pair.
+template <bool LOSS, int NT>
+__global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void adj_pair_kernel(
     const int* __restrict__ flags, const int* __restrict__ list_n, const uint2* __restrict__ list, int list_cap,
-    const uint4* __restrict__ pk, const float4* __restrict__ ws, int nt, float cx, float cy, float cz, float rc2,
-    float beta, const int* __restrict__ s2o, float* __restrict__ gq, double* __restrict__ gA,
-    double* __restrict__ gB) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int lb = xcd_block(gridDim.x);
-    const int ic = lb * kAdjWaves + w;
-    if (lb < 0 || ic >= flags[4]) return;
-    const int ii = lane & 3, jj = (lane >> 2) & 3, g = lane >> 4, bit = lane & 15;
-    const int islot = ic * kClusterSize + ii;
-    const uint4 a = pk[islot];
-    const unsigned ax = a.x & ~3u, ay = a.y & ~3u, az = a.z & ~3u;
-    const int ti = unpack_type(a);
-    float4 wi = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (LOSS) wi = ws[islot];
+    const uint4* __restrict__ pk, const float4* __restrict__ ws, float cx, float cy, float cz, float rc2, float beta,
+    const int* __restrict__ s2o, float* __restrict__ gq, double* __restrict__ gA, double* __restrict__ gB) {
+    constexpr int P = NT * (NT + 1) / 2;
+    __shared__ DenseLds walk[kDenseWaves];
+    __shared__ double sums[kDenseWaves][kClusterSize];
+    __shared__ double bins[kDenseWaves][2][P];
+    const int lane = threadIdx.x & 63, w = wave_in_block();
+    for (int k = threadIdx.x; k < kDenseWaves * 2 * P; k += blockDim.x) (&bins[0][0][0])[k] = 0.0;
+    __syncthreads();
     const float mlog2e_b2 = -1.4426950408889634f * (beta * beta);
-    // per-lane sums in FP64: single terms are FP32, but the sums over a
-    // lane's pairs cancel (d.w changes sign) and near pairs dominate
-    double sq = 0.0;
-    double ta[kAdjMaxTypes], tb[kAdjMaxTypes];
+    const DenseUnits units = dense_units(flags[4]);
+    const int parts = 1 << units.split;
+    for (int base = units.base; base < units.end; base += units.step) {
+        const int u = base + w, ic = u >> units.split, part = u & (parts - 1);
+        if (u < units.end) {
+            const int islot = ic * kClusterSize + (lane >> 4);
+            const uint4 a = pk[islot];
+            const int ti = unpack_type(a);
+            float4 wi = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (LOSS) wi = ws[islot];
+            // per-lane sums in FP64: single terms are FP32, but the sums over
+            // a lane's pairs cancel (d.w changes sign) and near pairs dominate
+            double sq = 0.0;
+            double ta[NT], tb[NT];
 #pragma unroll
-    for (int t = 0; t < kAdjMaxTypes; t++) ta[t] = tb[t] = 0.0;
-    const int n = list_n[ic];
-    const uint2* lst = list + (size_t)ic * list_cap;
-    for (int base = 0; base < n; base += 64) {
-        const uint2 my = base + lane < n ? lst[base + lane] : make_uint2((unsigned)ic, 0u);
-        const int cnt = min(64, n - base);
-        for (int it = 0; it < cnt; it += 4) {
-            const int src = min(it + g, 63);
-            const int jc = __shfl((int)my.x, src);
-            const unsigned m = (unsigned)__shfl((int)my.y, src);
-            const int jslot = jc * kClusterSize + jj;
-            const uint4 b = pk[jslot];
-            const float dx = (float)(int)((b.x & ~3u) - ax) * cx;
-            const float dy = (float)(int)((b.y & ~3u) - ay) * cy;
-            const float dz = (float)(int)((b.z & ~3u) - az) * cz;
-            const float r2 = dr2_exact(dx, dy, dz);
-            const bool in = (it + g < cnt) && ((m >> bit) & 1u) && r2 < rc2;
-            const float r2s = in ? r2 : 1.0f;
-            const float rinv = __builtin_amdgcn_rsqf(r2s);
-            const float rinv2 = rinv * rinv;
-            const float x = beta * (r2s * rinv);
-            const float ex = __builtin_amdgcn_exp2f(mlog2e_b2 * r2s);
-            const float ecx = erfcx_poly(x);
-            const float qj = __uint_as_float(b.w);
-            const int tj = unpack_type(b);
-            // table terms in FP64 from the exact integer displacement: r^-14
-            // amplifies the FP32 rounding of r^2 seven-fold
-            double cA = 0.0, cB = 0.0;
-            if (in) {
-                const double ddx = (double)(int)((b.x & ~3u) - ax) * (double)cx;
-                const double ddy = (double)(int)((b.y & ~3u) - ay) * (double)cy;
-                const double ddz = (double)(int)((b.z & ~3u) - az) * (double)cz;
-                const double ir2 = 1.0 / (ddx * ddx + ddy * ddy + ddz * ddz);
+            for (int t = 0; t < NT; t++) ta[t] = tb[t] = 0.0;
+            dense_walk<kEachSide>(ic, pk, s2o, list_n, list, list_cap, cx, cy, cz, rc2, part, units.split, walk[w],
+                                  [&](bool in, int jslot) {
+                const uint4 b = pk[jslot];
+                const int ix = (int)((b.x & ~3u) - (a.x & ~3u)), iy = (int)((b.y & ~3u) - (a.y & ~3u)),
+                          iz = (int)((b.z & ~3u) - (a.z & ~3u));
+                const int tj = unpack_type(b);
+                const float dx = (float)ix * cx, dy = (float)iy * cy, dz = (float)iz * cz;
+                const float r2 = in ? dr2_exact(dx, dy, dz) : 1.0f;
+                const float rinv = __builtin_amdgcn_rsqf(r2);
+                const float x = beta * (r2 * rinv);
+                const float ex = __builtin_amdgcn_exp2f(mlog2e_b2 * r2);
+                const float ecx = erfcx_poly(x);
+                const float qj = __uint_as_float(b.w);
+                // table terms in FP64 from the exact integer displacement:
+                // r^-14 amplifies the FP32 rounding of r^2 seven-fold
+                const double ddx = (double)ix * (double)cx, ddy = (double)iy * (double)cy,
+                             ddz = (double)iz * (double)cz;
+                const double ir2 = rcp_f64(in ? ddx * ddx + ddy * ddy + ddz * ddz : 1.0);
                 const double ir6 = ir2 * ir2 * ir2;
+                double cA, cB;
                 if (!LOSS) {
-                    sq += (double)(qj * ex * ecx * rinv);
-                    cA = ir6 * ir6 * (0.5 / 12.0);
-                    cB = ir6 * (-0.5 / 6.0);
+                    sq += in ? (double)(qj * ex * ecx * rinv) : 0.0;
+                    cA = ir6 * ir6;
+                    cB = ir6;
                 } else {
                     const float4 wj = ws[jslot];
                     const float sdi = dx * wi.x + dy * wi.y + dz * wi.z;
                     const float sdj = dx * wj.x + dy * wj.y + dz * wj.z;
-                    const float gr = ex * fmaf(kTwoOverSqrtPi, x, ecx) * rinv * rinv2;
-                    sq += (double)(-qj * gr * (sdi - sdj));
-                    const double sdid = ddx * (double)wi.x + ddy * (double)wi.y + ddz * (double)wi.z;
-                    cA = -ir6 * ir6 * ir2 * sdid;
-                    cB = ir6 * ir2 * sdid;
+                    const float gr = ex * fmaf(kTwoOverSqrtPi, x, ecx) * rinv * (rinv * rinv);
+                    sq += in ? (double)(-qj * gr * (sdi - sdj)) : 0.0;
+                    const double sd = ddx * (double)wi.x + ddy * (double)wi.y + ddz * (double)wi.z;
+                    cB = ir6 * ir2 * sd;
+                    cA = ir6 * cB;
+                }
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const bool mine = in && tj == t;
+                    if (__any(mine)) {
+                        ta[t] += mine ? cA : 0.0;
+                        tb[t] += mine ? cB : 0.0;
+                    }
+                }
+            });
+            const double q = row_sum(sq);
+            if ((lane & 15) == 0) {
+                const int at = s2o[islot];
+                if (parts > 1) sums[w][lane >> 4] = q;
+                else if (at >= 0) gq[at] = (float)q;
+            }
+            // the cluster's table terms by pair type (atoms of one type share
+            // a bin: LDS atomics of the wave's four row leaders)
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if (!__any(ta[t] != 0.0 || tb[t] != 0.0)) continue;
+                const double sa = row_sum(ta[t]), sb = row_sum(tb[t]);
+                if ((lane & 15) == 0) {
+                    const int p = pidx(min(ti, NT - 1), t);
+                    atomicAdd(&bins[w][0][p], sa);
+                    atomicAdd(&bins[w][1][p], sb);
                 }
             }
-#pragma unroll
-            for (int t = 0; t < kAdjMaxTypes; t++) {
-                ta[t] += tj == t ? cA : 0.0;
-                tb[t] += tj == t ? cB : 0.0;
+        }
+        if (parts > 1) {
+            __syncthreads();
+            if (u < units.end && part == 0 && lane < kClusterSize) {
+                double q = sums[w][lane];
+                for (int p = 1; p < parts; p++) q += sums[w + p][lane];
+                const int at = s2o[ic * kClusterSize + lane];
+                if (at >= 0) gq[at] = (float)q;
             }
+            __syncthreads();
         }
     }
-    // sum the 16 lanes sharing ii
-#pragma unroll
-    for (int o = 4; o < 64; o <<= 1) {
-        sq += __shfl_xor(sq, o);
-#pragma unroll
-        for (int t = 0; t < kAdjMaxTypes; t++) {
-            ta[t] += __shfl_xor(ta[t], o);
-            tb[t] += __shfl_xor(tb[t], o);
-        }
-    }
-    if (lane < 4) {
-        const int at = s2o[islot];
-        if (at >= 0) {
-            gq[at] = (float)sq;
-#pragma unroll
-            for (int t = 0; t < kAdjMaxTypes; t++) {
-                if (t < nt && (ta[t] != 0.0 || tb[t] != 0.0)) {
-                    atomicAdd(gA + pidx(ti, t), ta[t]);
-                    atomicAdd(gB + pidx(ti, t), tb[t]);
-                }
-            }
-        }
+    __syncthreads();
+    if (threadIdx.x < 2 * P) {
+        const int which = threadIdx.x / P, p = threadIdx.x - which * P;
+        double s = 0.0;
+        for (int k = 0; k < kDenseWaves; k++) s += bins[k][which][p];
+        // energy: half of each ordered pair's r^-12 / 12 and -r^-6 / 6
+        const double c = LOSS ? (which ? 1.0 : -1.0) : (which ? -0.5 / 6.0 : 0.5 / 12.0);
+        if (s != 0.0) atomicAdd((which ? gB : gA) + p, c * s);
     }
 }
 
@@ -331,21 +345,20 @@ int adj_common(sponge_nl* nl, sponge_lj* lj, sponge_pme* pme, const unsigned int
                const int* es, const int* el, const int* en, int loss, AdjScratch* A, double* gA, double* gB,
                hipStream_t s) {
     const int n = lj->n;
-    const int T = lj->ntypes, P = T * (T + 1) / 2;
+    const int T = lj->ntypes;
     int rc = snb_scratch(&lj->ps, nl);
     if (rc) return rc;
     adj_gather_kernel<<<ceil_div(nl->slot_cap, 256), 256, 0, s>>>(nl->flags, nl->s2o, uc, q, lj->d_type, lj->ps.pk,
                                                                    A->w3, loss ? A->ws : nullptr);
     SNB_CHECK_LAUNCH();
-    const int nblk = xcd_grid(ceil_div(nl->ncl_cap, kAdjWaves));
     const float rc2 = lj->cutoff * lj->cutoff;
-#define SNB_ADJ(L)                                                                                               \
-    adj_pair_kernel<L><<<nblk, kAdjWaves * 64, 0, s>>>(nl->flags, nl->list_n, nl->list, nl->list_cap, lj->ps.pk, \
-                                                       A->ws, T, lj->cof_dr[0], lj->cof_dr[1], lj->cof_dr[2], rc2, \
-                                                       pme->beta, nl->s2o, A->gq, gA, gB)
-    if (loss) SNB_ADJ(true);
-    else SNB_ADJ(false);
-#undef SNB_ADJ
+    auto go = [&](auto kernel) {
+        kernel<<<dense_blocks(nl->ncl_cap), kDenseWaves * 64, 0, s>>>(
+            nl->flags, nl->list_n, nl->list, nl->list_cap, lj->ps.pk, A->ws, lj->cof_dr[0], lj->cof_dr[1],
+            lj->cof_dr[2], rc2, pme->beta, nl->s2o, A->gq, gA, gB);
+    };
+    if (T <= 4) loss ? go(adj_pair_kernel<true, 4>) : go(adj_pair_kernel<false, 4>);
+    else loss ? go(adj_pair_kernel<true, kAdjMaxTypes>) : go(adj_pair_kernel<false, kAdjMaxTypes>);
     SNB_CHECK_LAUNCH();
     if (loss)
         adj_excl_kernel<true><<<ceil_div(n, 256), 256, 0, s>>>(n, uc, lj->cof_dr[0], lj->cof_dr[1], lj->cof_dr[2], q,
@@ -354,7 +367,6 @@ int adj_common(sponge_nl* nl, sponge_lj* lj, sponge_pme* pme, const unsigned int
         adj_excl_kernel<false><<<ceil_div(n, 256), 256, 0, s>>>(n, uc, lj->cof_dr[0], lj->cof_dr[1], lj->cof_dr[2],
                                                                 q, pme->beta, es, el, en, A->w3, A->gq);
     SNB_CHECK_LAUNCH();
-    (void)P;
     // reciprocal: R = theta * Q (prep, spread, FFTs, convolution; no gather)
     return snb_pme_reciprocal(pme, uc, q, nullptr, 0, 0, s);
 }

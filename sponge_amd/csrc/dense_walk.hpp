@@ -147,6 +147,35 @@ __device__ __forceinline__ void rsqrt_f64(double r2, double& rinv, double& r) {
     }
 }
 
+// 1 / v from v_rcp_f64 and two Newton steps; v = 0 gives inf, as 1.0 / 0.0.
+__device__ __forceinline__ double rcp_f64(double v) {
+    double y = __builtin_amdgcn_rcp(v);
+    y = fma(fma(-v, y, 1.0), y, y);
+    y = fma(fma(-v, y, 1.0), y, y);
+    if (__any(v == 0.0)) y = v == 0.0 ? __builtin_huge_val() : y;
+    return y;
+}
+
+// Sums over the 16 lanes of a row (one i atom's in the walk), in all of them.
+__device__ __forceinline__ float row_sum(float v) {
+    v += dpp_row_ror<8>(v);
+    v += dpp_row_ror<4>(v);
+    v += dpp_row_ror<2>(v);
+    return v + dpp_row_ror<1>(v);
+}
+template <int N>
+__device__ __forceinline__ double dpp_row_ror(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + N, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + N, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_row_ror<8>(v);
+    v += dpp_row_ror<4>(v);
+    v += dpp_row_ror<2>(v);
+    return v + dpp_row_ror<1>(v);
+}
+
 // ---- the walk ---------------------------------------------------------------
 // Calls use(active, jslot) with all 64 lanes, lane (i, k) = (lane >> 4,
 // lane & 15) taking pairs of the cluster's slot i; every pair inside the

@@ -643,14 +643,6 @@ __device__ __forceinline__ void energy_wave(int ic, int part, int split, DenseLd
     });
 }
 
-// Sum over the 16 lanes of an i atom, valid in all of them.
-__device__ __forceinline__ float row_sum(float v) {
-    v += dpp_row_ror<8>(v);
-    v += dpp_row_ror<4>(v);
-    v += dpp_row_ror<2>(v);
-    return v + dpp_row_ror<1>(v);
-}
-
 struct EnergyOut {
     float* e;
     float* v;

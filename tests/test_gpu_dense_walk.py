@@ -102,3 +102,46 @@ def test_energies(waters, cutoff, skin, soft):
     assert p["pairs_in"] == ref["n_in"]
     for k, v in (("lj", ref["e_lj"]), ("direct", ref["e_direct"])):
         assert abs(p[k] - v) <= (2.0 ** -23 if soft else 1e-9) * scale, (k, p[k], v)
+
+
+@pytest.mark.parametrize("waters,cutoff,skin,ntypes", [(27, 3.5, 0.5, 1), (216, 9.2, 0.1, 4), (343, 6.0, 1.0, 5),
+                                                       (729, 7.0, 1.0, 8)])
+def test_gradients(waters, cutoff, skin, ntypes):
+    """Both gradients at the edges of the type count (4 and 8 accumulators)
+    against the FP64 oracle. Table gradients are FP64 sums of FP64 terms, with
+    FP32 weights F - T on the loss side: 1e-9 and 1e-6 of the sum of the
+    entries' sizes; charge gradients are FP32 terms: 1e-5 of their norm."""
+    import dataclasses
+    import torch
+    from sponge_amd import nb
+    rng = np.random.default_rng(ntypes)
+    length = (waters * system.WATER_VOLUME) ** (1.0 / 3.0)
+    base = system.water_box(waters, round(length, 3), seed=3, cutoff=cutoff, skin=skin)
+    A, B = system._lb_table(rng.uniform(2.0, 3.2, ntypes), rng.uniform(0.05, 0.2, ntypes))
+    s = dataclasses.replace(base, lj_type=rng.integers(0, ntypes, base.n).astype(np.int32), lj_A=A, lj_B=B)
+    say(f"[case] gradients waters {waters} n {s.n} cutoff {cutoff} types {ntypes}")
+    eng = nb.NonbondedEngine(s, refresh_interval=0)
+    eng.update_neighbor_list(forced=1)
+    eng.force_step(0, 0, from_crd=True, overwrite=True)
+    P = len(A)
+    gq, gA, gB = (torch.zeros(k, dtype=torch.float64, device="cuda") for k in (s.n, P, P))
+    loss = torch.zeros(1, dtype=torch.float64, device="cuda")
+    target = torch.as_tensor(rng.normal(0.0, 5.0, (s.n, 3)).astype(np.float32), device="cuda")
+    u = eng.uint_crd.cpu().numpy().view(np.uint32)
+    pairs = oracle.nl_brute(s, u)
+    K = (eng.pme.fftx, eng.pme.ffty, eng.pme.fftz)
+    eng.energy_gradient(gq, gA, gB)
+    e = oracle.energy_grad(s, u, pairs, eng.pme.beta, K)
+    got = [t.cpu().numpy().copy() for t in (gq, gA, gB)]
+    eng.force_matching_gradient(eng.frc, target, loss, gq, gA, gB)
+    f = oracle.loss_grad(s, u, pairs, eng.pme.beta, K, eng.frc.cpu().numpy().astype(np.float64),
+                         target.cpu().numpy().astype(np.float64))
+    more = [t.cpu().numpy().copy() for t in (gq, gA, gB)]
+    for name, g, ref, tol in (("energy", got, e, (1e-9, 2.0 ** -23)), ("loss", more, f[1:], (1e-6, 1e-6))):
+        err = np.linalg.norm(g[0] - ref[0]) / np.linalg.norm(ref[0])
+        say(f"    {name}: charges {err:.2e}")
+        assert err <= 1e-5, name
+        for k in (1, 2):
+            d = np.abs(g[k] - ref[k]).max() / np.abs(ref[k]).sum()
+            say(f"    {name}: table {k} {d:.2e}")
+            assert d <= tol[k - 1], (name, k)

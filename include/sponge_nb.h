@@ -35,7 +35,7 @@ extern "C" {
 /* Overflow flags reported by sponge_nl_status (bit set = overflowed). */
 #define SPONGE_NL_OVERFLOW_COLUMN 1  /* too many atoms in one cell column */
 #define SPONGE_NL_OVERFLOW_LIST 2    /* too many cluster pairs for one cluster */
-#define SPONGE_NL_OVERFLOW_CANDIDATES 4
+#define SPONGE_NL_OVERFLOW_CANDIDATES 4 /* not raised: the search has no such limit */
 
 /* Energy / virial parts accumulated in FP64 on the device by the fused step
  * and by the energy queries (index into a double[SPONGE_NB_NPARTS]). */

@@ -180,12 +180,12 @@ struct sponge_nl {
     int slot_cap;               // max padded slots (multiple of 4)
     int ncl_cap;                // slot_cap / 4
     int list_cap;               // max cluster-pair entries per i-cluster
-    int cand_cap;               // max candidate j-clusters per i-cluster
     // device buffers
     float* old_crd;             // 3n
     unsigned int* nl_uint;      // 3n, uint coordinates at the last rebuild
     int* col_count;             // ncol
     int* col_start;             // ncol+1 (slots)
+    unsigned short* col_z;      // per column: atoms below each z bin's start
     int* col_atoms;             // ncol * col_cap
     int* s2o;                   // slot_cap: slot -> atom (-1 = padding)
     int* o2s;                   // n: atom -> slot (-1: left out by a column overflow)
@@ -193,12 +193,13 @@ struct sponge_nl {
     float4* cl_lo;              // ncl_cap bounding boxes (Angstrom)
     float4* cl_hi;
     int* list_n;                // ncl_cap
+    int* list_pairs;            // ncl_cap: atom pairs a cluster's entries hold
     uint2* list;                // ncl_cap * list_cap : (j cluster, 16-bit pair mask)
     uint4* pack;                // slot_cap sorted (ux, uy, uz, atom) at the last rebuild
     int* flags;                 // [0] rebuild flag, [1] overflow bits, [2] rebuild count,
                                 // [3] slot count, [4] cluster count, [5] atoms left out
                                 // (column overflow), [7] skin-check vote,
-                                // [8..9] listed pair count (64-bit), [10] fused steps
+                                // [10] fused steps
                                 // completed since the last rebuild
     int device;
     // inner list of the fused step: the entries and masks of `list` whose

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "dense_walk.hpp"
 #include "tune_table.hpp"
 
 using namespace snb;
@@ -34,8 +35,12 @@ namespace {
 constexpr int kSortThreads = 256;
 constexpr int kMaxColumn = 1024;     // bitonic sort capacity per column (LDS)
 constexpr int kPairWaves = 4;
-constexpr int kCandCap = 1024;       // candidate j-clusters per i-cluster (LDS)
-constexpr int kColCap = 128;         // cell columns of one search window held in LDS
+constexpr int kListCap = 1024;       // most cluster-pair entries per i-cluster
+// z bins of a column's table (col_z: per bin the column's atoms below its
+// start): the rebuild's search then reads the run of clusters in a z window
+// with two loads where a binary search over the boxes took 5 to 8 in turn.
+constexpr int kZBinBits = 7, kZBins = 1 << kZBinBits, kZStride = kZBins + 2;
+constexpr int kCandWindow = 512;     // candidate j-clusters held in LDS at a time 
 
 // Is_need_refresh_neighbor_list_cuda (neighbor_list.cu:336-351): FP32
 // periodic displacement against the coordinates of the last rebuild.
@@ -71,8 +76,6 @@ __device__ __forceinline__ void nl_begin_body(int forced, int* flags, int* col_c
         if (f) {
             flags[1] = 0;
             flags[5] = 0;
-            flags[8] = 0;
-            flags[9] = 0;
             flags[2] += 1;
             flags[10] = 0;  // the next fused step prunes the new list
             flags[13] = 0;  // no displacement vote on the new list yet
@@ -253,13 +256,14 @@ __global__ void nl_scan_kernel(int ncol, int col_cap, const int* __restrict__ co
 }
 
 // One block per column: sort its atoms by (uint z, atom index) -- a
-// deterministic order -- write the slot maps, the sorted uint coordinates and
-// the bounding box of every 4-atom cluster.
+// deterministic order -- write the slot maps, the sorted uint coordinates, the
+// bounding box of every 4-atom cluster and the column's z table.
 __device__ __forceinline__ void nl_sort_body(
     int c, int col_cap, const int* __restrict__ col_count, const int* __restrict__ col_start,
     const int* __restrict__ col_atoms, const unsigned int* __restrict__ nl_uint,
     float crx, float cry, float crz, int* __restrict__ s2o, int* __restrict__ o2s,
-    uint4* __restrict__ pack, float4* __restrict__ cl_lo, float4* __restrict__ cl_hi, const int* flags) {
+    uint4* __restrict__ pack, float4* __restrict__ cl_lo, float4* __restrict__ cl_hi,
+    unsigned short* __restrict__ col_z, const int* flags) {
     if (!flags[0]) return;
     __shared__ unsigned long long key[kMaxColumn];
     int cnt = min(col_count[c], col_cap);
@@ -304,7 +308,17 @@ __device__ __forceinline__ void nl_sort_body(
             pack[slot] = make_uint4(0u, 0u, 0u, 0xffffffffu);
         }
     }
-    __syncthreads();
+    // the column's atoms below each z bin's start
+    for (int b = threadIdx.x; b <= kZBins; b += blockDim.x) {
+        const unsigned long long start_z = (unsigned long long)b << (32 - kZBinBits);
+        int lo = 0, up = cnt;
+        while (lo < up) {
+            const int mid = (lo + up) >> 1;
+            if ((key[mid] >> 32) < start_z) lo = mid + 1;
+            else up = mid;
+        }
+        col_z[(size_t)c * kZStride + b] = (unsigned short)lo;
+    }
     int ncl = pad / kClusterSize;
     for (int k = threadIdx.x; k < ncl; k += blockDim.x) {
         float lo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, hi[3] = {-3.0e38f, -3.0e38f, -3.0e38f};
@@ -330,9 +344,10 @@ __global__ __launch_bounds__(kSortThreads) void nl_sort_kernel(
     int col_cap, const int* __restrict__ col_count, const int* __restrict__ col_start,
     const int* __restrict__ col_atoms, const unsigned int* __restrict__ nl_uint,
     float crx, float cry, float crz, int* __restrict__ s2o, int* __restrict__ o2s,
-    uint4* __restrict__ pack, float4* __restrict__ cl_lo, float4* __restrict__ cl_hi, const int* flags) {
+    uint4* __restrict__ pack, float4* __restrict__ cl_lo, float4* __restrict__ cl_hi,
+    unsigned short* __restrict__ col_z, const int* flags) {
     nl_sort_body(blockIdx.x, col_cap, col_count, col_start, col_atoms, nl_uint, crx, cry, crz, s2o, o2s, pack, cl_lo,
-                 cl_hi, flags);
+                 cl_hi, col_z, flags);
 }
 
 // FP32 neighbor-list distance, the reference's expression with every
@@ -354,240 +369,261 @@ __device__ __forceinline__ bool excluded_pair(int a, int b, const int* __restric
     return false;
 }
 
-// One wave per i-cluster: gather candidate j-clusters (index >= i) from the
-// columns within rc+skin, test bounding boxes, then compute the exact 16-bit
-// pair masks four cluster pairs at a time and append the non-empty ones.
+// v in [0, n) for v in [-n, 2n).
+__device__ __forceinline__ int wrap(int v, int n) { return v < 0 ? v + n : v >= n ? v - n : v; }
+
+// One wave per i-cluster: the j-clusters that can hold a listed pair, column
+// by column, then their exact 16-bit pair masks, appended where not empty.
+//
+// Candidates: of every column of the search window, the clusters whose z
+// extent (sorted, as the atoms are) comes within sqrt(rlm^2 - gap^2) of the
+// i-cluster's, gap being the xy distance of the column's rectangle: a circular
+// run, read from the column's z table (64 columns at a time, one per lane). At
+// water density 1.3 candidates a listed cluster; a box test of each cost more
+// than it saved the mask stage.
+//
+// Masks, 16 candidates at a time: lane (e, jj) = (lane >> 2, lane & 3) holds
+// one j atom against the four i atoms, r^2 = |a|^2 + |b|^2 - 2 a.b about the
+// cluster's first atom with the product from three 4x4x1 MFMAs; a batch with a
+// value closer to (rc + skin)^2 than the expansion's rounding bound, and every
+// batch of a box too small for displacements from one atom (dense_walk.hpp
+// has both conditions), takes the list's own FP32 expression nl_dr2. With
+// symmetric exclusion lists (sym_start) each partner sets its bit in a mask on
+// its cluster among the candidates; without them the CSR is searched for every
+// pair in range.
+// Bound: latency of a wave's ~30 record loads and vector issue. Measured, 648 /
+// 4,446 / 10,013 / 23,570 / 96,120 atoms: 12 / 22 / 30 / 46 / 136 us against
+// 24 / 100 / 79 / 128 / 368 us with a box test of the candidates, one pair per
+// lane in the mask stage and one pair counter for all waves.
 __device__ __forceinline__ void nl_pairs_body(
     int lb, int ncx, int ncy, float bx, float by, float bz, float crx, float cry, float crz, float rl2,
-    float rlm, const int* __restrict__ col_start, const float4* __restrict__ cl_lo,
-    const float4* __restrict__ cl_hi, const uint4* __restrict__ pack, const int* __restrict__ es,
-    const int* __restrict__ en, const int* __restrict__ el, int list_cap, int* __restrict__ list_n,
-    uint2* __restrict__ list, int* flags, const int* __restrict__ sym_start = nullptr,
-    const int* __restrict__ sym_list = nullptr) {
+    float rlm, const int* __restrict__ col_start, const unsigned short* __restrict__ col_z,
+    const float4* __restrict__ cl_lo, const float4* __restrict__ cl_hi, const uint4* __restrict__ pack,
+    const int* __restrict__ o2s,
+    const int* __restrict__ es, const int* __restrict__ en, const int* __restrict__ el, int list_cap,
+    int* __restrict__ list_n, int* __restrict__ list_pairs, uint2* __restrict__ list, int* flags,
+    const int* __restrict__ sym_start = nullptr, const int* __restrict__ sym_list = nullptr) {
     if (!flags[0]) return;
-    __shared__ int cand[kPairWaves][kCandCap];
-    __shared__ int colj0[kPairWaves][kColCap];
-    __shared__ int colpre[kPairWaves][kColCap];
-    __shared__ int colzc[kPairWaves][kColCap];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __shared__ uint2 cands[kPairWaves][kCandWindow];  // (j cluster, mask of excluded pairs)
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int ic = lb * kPairWaves + w;
-    const int ncl = flags[4];
-    if (lb < 0 || ic >= ncl) return;
+    if (lb < 0 || ic >= flags[4]) return;
+    uint2* cand = cands[w];
+    const int jj = lane & 3, e0 = lane >> 2;
+    // i atoms: this lane's is jj, for the mask stage
+    const uint4 mine = pack[ic * kClusterSize + jj];
+    const unsigned ox = uniform((int)mine.x), oy = uniform((int)mine.y), oz = uniform((int)mine.z);
+    const bool pad = (int)mine.w < 0;
+    const float px = pad ? 0.f : (float)(int)(mine.x - ox) * crx;
+    const float py = pad ? 0.f : (float)(int)(mine.y - oy) * cry;
+    const float pz = pad ? 0.f : (float)(int)(mine.z - oz) * crz;
+    const float paa = px * px + py * py + pz * pz;
+    const float aa[kClusterSize] = {quad_lane<0>(paa), quad_lane<1>(paa), quad_lane<2>(paa), quad_lane<3>(paa)};
+    const unsigned real = (unsigned)__ballot(!pad) & 15u;
+    const float rl = sqrtf(rl2);
+    const float reach = (rl + sqrtf(fmaxf(fmaxf(aa[0], aa[1]), fmaxf(aa[2], aa[3])))) * 1.0001f;
+    const bool safe = reach < 2147483648.0f * fminf(crx, fminf(cry, crz));
+    const float eps = 4.0e-6f * reach * reach;
+    const float r2lo = rl2 - eps, r2hi = rl2 + eps;
+    // exclusion partners: lane (i, k) = (lane >> 4, lane & 15) keeps the k-th
+    // of atom i, its slot and cell column
+    const int xi = lane >> 4, xk = lane & 15;
+    const int xatom = (int)pack[ic * kClusterSize + xi].w;
+    int x0 = 0, x1 = 0;
+    if (sym_start && xatom >= 0) {
+        x0 = sym_start[xatom];
+        x1 = sym_start[xatom + 1];
+    }
+    auto partner = [&](int k, int& js, int& col) {
+        js = -1;
+        if (k >= x1) return;
+        js = o2s[sym_list[k]];
+        if (js < 0) return;
+        const uint4 b = pack[js];
+        col = (int)(((unsigned long long)b.x * (unsigned)ncx) >> 32) * ncy +
+              (int)(((unsigned long long)b.y * (unsigned)ncy) >> 32);
+    };
+    int xslot, xcol = 0;
+    partner(x0 + xk, xslot, xcol);
+
     const float4 li = cl_lo[ic], hi = cl_hi[ic];
-    const float cix = 0.5f * (li.x + hi.x), ciy = 0.5f * (li.y + hi.y), ciz = 0.5f * (li.z + hi.z);
-    const float hix = 0.5f * (hi.x - li.x), hiy = 0.5f * (hi.y - li.y), hiz = 0.5f * (hi.z - li.z);
-    const float cwx = bx / ncx, cwy = by / ncy;
+    const float cix = 0.5f * (li.x + hi.x), ciy = 0.5f * (li.y + hi.y);
+    const float hix = 0.5f * (hi.x - li.x), hiy = 0.5f * (hi.y - li.y);
+    const float cwx = bx / ncx, cwy = by / ncy, zbin = kZBins / bz;
     int ax0 = (int)floorf((li.x - rlm) / cwx), ax1 = (int)floorf((hi.x + rlm) / cwx);
     int ay0 = (int)floorf((li.y - rlm) / cwy), ay1 = (int)floorf((hi.y + rlm) / cwy);
     int nxr = ax1 - ax0 + 1, nyr = ay1 - ay0 + 1;
     if (nxr >= ncx) { ax0 = 0; nxr = ncx; }
     if (nyr >= ncy) { ay0 = 0; nyr = ncy; }
-    const float rlm2 = rlm * rlm;
-    int ncand = 0;
-    bool over = false;
-    // bounding-box test of candidate j-cluster jc; appends it to cand[w]
-    auto test_box = [&](int jc, bool live) {
-        bool ok = false;
-        if (live) {
-            const float4 lj = cl_lo[jc], hj = cl_hi[jc];
-            float dx = 0.5f * (lj.x + hj.x) - cix, dy = 0.5f * (lj.y + hj.y) - ciy, dz = 0.5f * (lj.z + hj.z) - ciz;
-            dx -= bx * rintf(dx / bx);
-            dy -= by * rintf(dy / by);
-            dz -= bz * rintf(dz / bz);
-            const float gx = fmaxf(fabsf(dx) - hix - 0.5f * (hj.x - lj.x), 0.f);
-            const float gy = fmaxf(fabsf(dy) - hiy - 0.5f * (hj.y - lj.y), 0.f);
-            const float gz = fmaxf(fabsf(dz) - hiz - 0.5f * (hj.z - lj.z), 0.f);
-            ok = gx * gx + gy * gy + gz * gz < rlm2;
-        }
-        const unsigned long long bal = __ballot(ok);
-        const int pos = ncand + __popcll(bal & ((1ull << lane) - 1ull));
-        if (ok) {
-            if (pos < kCandCap) cand[w][pos] = jc;
-            else over = true;
-        }
-        ncand += __popcll(bal);
-    };
     const int ncols = nxr * nyr;
-    if (ncols <= kColCap) {
-        // The window's columns as one flat range of j-clusters: a table of
-        // each column's first cluster and running cluster count, then 64
-        // clusters per step whatever their column (instead of one column per
-        // step, most of whose lanes would idle).
-        // Within a column the clusters are sorted by z (their atoms are), so
-        // only those whose z extent meets [lo.z - rlm, hi.z + rlm] of the
-        // i-cluster (periodically: a circular run of the column's clusters,
-        // found by two binary searches) can pass the box test; a window at
-        // least a box length long takes the whole column.
-        const float zpad = rlm + 1.0e-2f;
-        const float zlo = li.z - zpad, zhi = hi.z + zpad;
-        const bool zwin = zhi - zlo < bz;
-        const float za = zlo < 0.f ? zlo + bz : zlo;   // window start in [0, bz)
-        const float zb = zhi >= bz ? zhi - bz : zhi;   // window end in [0, bz)
-        const bool zwrap = zlo < 0.f || zhi >= bz;
-        int total = 0;
-        for (int base = 0; base < ncols; base += 64) {
-            const int k = base + lane;
-            int j0 = 0, cnt = 0, zs = 0, zl = 0;
-            if (k < ncols) {
-                const int ox = k / nyr, oy = k - ox * nyr;
-                const int cx = ((ax0 + ox) % ncx + ncx) % ncx, cy = ((ay0 + oy) % ncy + ncy) % ncy;
-                const int c = cx * ncy + cy;
-                j0 = col_start[c] / kClusterSize;
-                cnt = col_start[c + 1] / kClusterSize - j0;
-                zl = cnt;
-                if (zwin && cnt > 0) {
-                    // s: the first cluster whose top reaches za; e: the first
-                    // whose bottom lies above zb
-                    int lo = 0, up = cnt;
-                    while (lo < up) {
-                        const int mid = (lo + up) >> 1;
-                        if (cl_hi[j0 + mid].z < za) lo = mid + 1;
-                        else up = mid;
-                    }
-                    const int s = lo;
-                    lo = 0;
-                    up = cnt;
-                    while (lo < up) {
-                        const int mid = (lo + up) >> 1;
-                        if (cl_lo[j0 + mid].z <= zb) lo = mid + 1;
-                        else up = mid;
-                    }
-                    const int e = lo;
-                    zs = s == cnt ? 0 : s;
-                    zl = zwrap ? min(cnt - s + e, cnt) : max(e - s, 0);
-                }
-            }
-            int incl = zl;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int t = __shfl_up(incl, o);
-                if (lane >= o) incl += t;
-            }
-            if (k < ncols) {
-                colj0[w][k] = j0;
-                colpre[w][k] = total + incl - zl;
-                colzc[w][k] = zs | (cnt << 16);
-            }
-            total += __shfl(incl, 63);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        for (int t0 = 0; t0 < total; t0 += 64) {
-            const int t = t0 + lane;
-            int jc = 0;
-            if (t < total) {
-                // last column whose run starts at or before t (empty columns
-                // share their successor's start and are skipped)
-                int lo = 0, hi = ncols - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (colpre[w][mid] <= t) lo = mid;
-                    else hi = mid - 1;
-                }
-                const int zc = colzc[w][lo], zs = zc & 0xffff, cnt = zc >> 16;
-                const int u = zs + (t - colpre[w][lo]);
-                jc = colj0[w][lo] + (u >= cnt ? u - cnt : u);
-            }
-            test_box(jc, t < total);
-        }
-    } else {
-    for (int ox = 0; ox < nxr; ox++) {
-        int cx = ((ax0 + ox) % ncx + ncx) % ncx;
-        for (int oy = 0; oy < nyr; oy++) {
-            int cy = ((ay0 + oy) % ncy + ncy) % ncy;
-            int c = cx * ncy + cy;
-            int j0 = col_start[c] / kClusterSize, j1 = col_start[c + 1] / kClusterSize;
-            for (int jb = j0; jb < j1; jb += 64) test_box(jb + lane, jb + lane < j1);
-        }
-    }
-    }
-    if (ncand > kCandCap) {
-        ncand = kCandCap;
-        over = true;
-    }
-    if (over && lane == 0) atomicOr(flags + 1, SPONGE_NL_OVERFLOW_CANDIDATES);
-    // cand[w] is private to this wave: order its LDS writes before the reads.
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-
-    const int ii = lane & 3, jj = (lane >> 2) & 3, g = lane >> 4;
-    const uint4 pi = pack[ic * kClusterSize + ii];
-    const int ai = (int)pi.w;
-    // The lane's i-atom exclusion partners, the first four in registers, from
-    // the symmetric lists when there are some (else the CSR is searched).
-    int e0 = -1, e1 = -1, e2 = -1, e3 = -1, r0 = 0, r1 = 0;
-    if (sym_start && ai >= 0) {
-        r0 = sym_start[ai];
-        r1 = sym_start[ai + 1];
-        const int len = r1 - r0;
-        if (len > 0) e0 = sym_list[r0];
-        if (len > 1) e1 = sym_list[r0 + 1];
-        if (len > 2) e2 = sym_list[r0 + 2];
-        if (len > 3) e3 = sym_list[r0 + 3];
-    }
-    auto is_excluded = [&](int aj) -> bool {
-        if (!sym_start) return excluded_pair(ai, aj, es, en, el);
-        if (aj == e0 || aj == e1 || aj == e2 || aj == e3) return true;
-        for (int k = r0 + 4; k < r1; k++)
-            if (sym_list[k] == aj) return true;
-        return false;
-    };
     int count = 0;
     long npairs = 0;
-    // four groups of 4 candidates per pass: their j records are loaded
-    // together, then tested and appended in candidate order (the loop is
-    // latency bound; the list stores of a pass no longer stall the next
-    // group's loads)
-    for (int cb = 0; cb < ncand; cb += 16) {
-        int jcs[4];
-        uint4 pjs[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int c = cb + 4 * u + g;
-            jcs[u] = c < ncand ? cand[w][c] : -1;
-            pjs[u] = jcs[u] >= 0 ? pack[jcs[u] * kClusterSize + jj] : make_uint4(0u, 0u, 0u, 0u);
+    for (int cb = 0; cb < ncols; cb += 64) {
+        // this lane's column: its first cluster j0, and the run of zl clusters
+        // from the zs-th on (circular over its cnt)
+        const int k = cb + lane;
+        int j0 = 0, cnt = 0, zs = 0, zl = 0, col = -1;
+        if (k < ncols) {
+            const int qx = k / nyr, qy = k - qx * nyr;
+            const int cx = wrap(ax0 + qx, ncx), cy = wrap(ay0 + qy, ncy);
+            col = cx * ncy + cy;
+            float dx = (cx + 0.5f) * cwx - cix, dy = (cy + 0.5f) * cwy - ciy;
+            dx -= bx * rintf(dx / bx);
+            dy -= by * rintf(dy / by);
+            const float gx = fmaxf(fabsf(dx) - hix - 0.5f * cwx, 0.f);
+            const float gy = fmaxf(fabsf(dy) - hiy - 0.5f * cwy, 0.f);
+            const float z2 = rlm * rlm - gx * gx - gy * gy;
+            if (z2 > 0.f) {
+                const float zpad = sqrtf(z2) + 1.0e-2f;
+                const float zlo = li.z - zpad, zhi = hi.z + zpad;
+                // window start and end in [0, bz), their bins
+                const bool up = zlo < 0.f, over = zhi >= bz;
+                const int ba = min((int)((up ? zlo + bz : zlo) * zbin), kZBins - 1);
+                const int bb = min((int)((over ? zhi - bz : zhi) * zbin), kZBins - 1);
+                const unsigned short* cz = col_z + (size_t)col * kZStride;
+                j0 = col_start[col] / kClusterSize;
+                cnt = col_start[col + 1] / kClusterSize - j0;
+                const int atoms = cz[kZBins], first = cz[max(ba, 0)], last = cz[max(bb, 0) + 1];
+                // the first cluster with an atom at or above the window's
+                // start, the first past those with one below its end's bin
+                const int s0 = first == atoms ? cnt : first / kClusterSize;
+                const int f0 = (last + kClusterSize - 1) / kClusterSize;
+                zs = s0 == cnt ? 0 : s0;
+                zl = zhi - zlo >= bz ? cnt : (up || over) ? min(cnt - s0 + f0, cnt) : max(f0 - s0, 0);
+            }
         }
+        int pre = zl;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int jc = jcs[u];
-            const uint4 pj = pjs[u];
-            bool bit = false;
-            if (jc >= 0) {
-                int aj = (int)pj.w;
-                bool valid = ai >= 0 && aj >= 0 && (jc != ic || jj != ii);
-                if (valid && nl_dr2(pi, pj, crx, cry, crz) < rl2) bit = !is_excluded(aj);
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(pre, o);
+            if (lane >= o) pre += t;
+        }
+        const int total = __builtin_amdgcn_readlane(pre, 63);
+        pre -= zl;
+        int longest = zl;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) longest = max(longest, __shfl_xor(longest, o));
+        longest = uniform(longest);
+        for (int w0 = 0; w0 < total; w0 += kCandWindow) {
+            // candidates w0 .. w0 + kCandWindow - 1 of these columns
+            for (int r = 0; r < longest; r++) {
+                const int pos = pre + r - w0;
+                if (r < zl && pos >= 0 && pos < kCandWindow) {
+                    const int u = zs + r;
+                    cand[pos] = make_uint2((unsigned)(j0 + (u >= cnt ? u - cnt : u)), 0u);
+                }
             }
-            unsigned long long bal = __ballot(bit);
-            unsigned m = (unsigned)(bal >> (g * 16)) & 0xffffu;
-            bool leader = (lane & 15) == 0 && m != 0;
-            unsigned long long lb2 = __ballot(leader);
-            int slot = count + __popcll(lb2 & ((1ull << lane) - 1ull));
-            if (leader) {
-                if (slot < list_cap) list[(size_t)ic * list_cap + slot] = make_uint2((unsigned)jc, m);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            // the excluded pairs of each candidate (LDS atomics: two atoms'
+            // partners may share a cluster)
+            if (sym_start) {
+                int js = xslot, pc = xcol;
+                for (int kk = x0 + xk; __any(kk < x1); kk += 16) {
+                    if (kk != x0 + xk) partner(kk, js, pc);
+                    int src = -1;
+                    if (kk < x1 && js >= 0) {
+                        const int cx = pc / ncy, qx = wrap(cx - ax0, ncx), qy = wrap(pc - cx * ncy - ay0, ncy);
+                        if (qx < nxr && qy < nyr) src = qx * nyr + qy - cb;
+                    }
+                    const bool here = src >= 0 && src < 64;
+                    const int sl = here ? src : 0;
+                    const int pj0 = __shfl(j0, sl), pcnt = __shfl(cnt, sl), pzs = __shfl(zs, sl), pzl = __shfl(zl, sl),
+                              ppre = __shfl(pre, sl);
+                    if (here && pcnt > 0) {
+                        int d = js / kClusterSize - pj0 - pzs;
+                        if (d < 0) d += pcnt;
+                        const int pos = ppre + d - w0;
+                        if (d < pzl && pos >= 0 && pos < kCandWindow)
+                            atomicOr(&cand[pos].y, 1u << ((js & (kClusterSize - 1)) * kClusterSize + xi));
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
-            count += __popcll(lb2);
-            npairs += __popcll(bal);
+            const int nc = min(total - w0, kCandWindow);
+            // (past the end: the i-cluster itself with every pair excluded)
+            const uint2 none = make_uint2((unsigned)ic, 0xffffu);
+            uint2 c = e0 < nc ? cand[e0] : none;
+            uint4 b = pack[(int)c.x * kClusterSize + jj];
+            for (int it = 0; it < nc; it += 16) {
+                const uint2 cn = it + 16 + e0 < nc ? cand[it + 16 + e0] : none;
+                const uint4 bn = pack[(int)cn.x * kClusterSize + jj];
+                const int jc = (int)c.x;
+                const int aj = (int)b.w;
+                const float x = (float)(int)(b.x - ox) * crx;
+                const float y = (float)(int)(b.y - oy) * cry;
+                const float z = (float)(int)(b.z - oz) * crz;
+                const float bb = x * x + y * y + z * z;
+                DenseF4 t = {bb + aa[0], bb + aa[1], bb + aa[2], bb + aa[3]};
+                t = __builtin_amdgcn_mfma_f32_4x4x1f32(-2.0f * px, x, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_4x4x1f32(-2.0f * py, y, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_4x4x1f32(-2.0f * pz, z, t, 0, 0, 0);
+                // this lane's j atom against the i atoms: pairs that may be
+                // listed, then those in range
+                unsigned ok = aj >= 0 ? real & ~(c.y >> (4 * jj)) : 0u;
+                if (jc == ic) ok &= ~(1u << jj);
+                unsigned in = 0u, near = 0u;
+#pragma unroll
+                for (int i = 0; i < kClusterSize; i++) {
+                    in |= t[i] < r2lo ? 1u << i : 0u;
+                    near |= t[i] < r2hi ? 1u << i : 0u;
+                }
+                if (!safe || __any((in ^ near) & ok)) {
+                    in = 0u;
+#pragma unroll
+                    for (int i = 0; i < kClusterSize; i++)
+                        in |= nl_dr2(pack[ic * kClusterSize + i], b, crx, cry, crz) < rl2 ? 1u << i : 0u;
+                }
+                in &= ok;
+                if (!sym_start) {
+#pragma unroll
+                    for (int i = 0; i < kClusterSize; i++)
+                        if ((in >> i) & 1u)
+                            if (excluded_pair((int)pack[ic * kClusterSize + i].w, aj, es, en, el)) in &= ~(1u << i);
+                }
+                // the quad's four nibbles make the entry's mask
+                unsigned m = in << (4 * jj);
+                m |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, false);
+                m |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, false);
+                const unsigned long long lead = __ballot(jj == 0 && m != 0u);
+                if (jj == 0 && m != 0u) {
+                    const int slot = count + below(lead);
+                    if (slot < list_cap) list[(size_t)ic * list_cap + slot] = make_uint2((unsigned)jc, m);
+                    npairs += __popc(m);
+                }
+                count += __popcll(lead);
+                c = cn;
+                b = bn;
+            }
         }
     }
+    int np = (int)npairs;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) np += __shfl_xor(np, o);
     if (lane == 0) {
         if (count > list_cap) {
             atomicOr(flags + 1, SPONGE_NL_OVERFLOW_LIST);
             count = list_cap;
         }
         list_n[ic] = count;
-        // every unordered pair is listed from both of its atoms
-        atomicAdd((unsigned long long*)(flags + 8), (unsigned long long)npairs);
+        // summed by the status call: one counter for all waves would take
+        // 16 ns of every wave in turn (half of this kernel's time at 23,570
+        // atoms)
+        list_pairs[ic] = np;
     }
 }
 
-__global__ __launch_bounds__(kPairWaves * 64) void nl_pairs_kernel(
+__global__ __launch_bounds__(kPairWaves * 64) __attribute__((amdgpu_waves_per_eu(6))) void nl_pairs_kernel(
     int ncx, int ncy, float bx, float by, float bz, float crx, float cry, float crz, float rl2,
-    float rlm, const int* __restrict__ col_start, const float4* __restrict__ cl_lo,
-    const float4* __restrict__ cl_hi, const uint4* __restrict__ pack, const int* __restrict__ es,
-    const int* __restrict__ en, const int* __restrict__ el, int list_cap, int* __restrict__ list_n,
-    uint2* __restrict__ list, int* flags, const int* __restrict__ sym_start, const int* __restrict__ sym_list) {
-    nl_pairs_body(xcd_block(gridDim.x), ncx, ncy, bx, by, bz, crx, cry, crz, rl2, rlm, col_start, cl_lo, cl_hi, pack,
-                  es, en, el, list_cap, list_n, list, flags, sym_start, sym_list);
+    float rlm, const int* __restrict__ col_start, const unsigned short* __restrict__ col_z,
+    const float4* __restrict__ cl_lo, const float4* __restrict__ cl_hi, const uint4* __restrict__ pack,
+    const int* __restrict__ o2s,
+    const int* __restrict__ es, const int* __restrict__ en, const int* __restrict__ el, int list_cap,
+    int* __restrict__ list_n, int* __restrict__ list_pairs, uint2* __restrict__ list, int* flags,
+    const int* __restrict__ sym_start, const int* __restrict__ sym_list) {
+    nl_pairs_body(xcd_block(gridDim.x), ncx, ncy, bx, by, bz, crx, cry, crz, rl2, rlm, col_start, col_z, cl_lo, cl_hi,
+                  pack, o2s, es, en, el, list_cap, list_n, list_pairs, list, flags, sym_start, sym_list);
 }
 
 // Per-slot lists of the fused step from the stored list (plain LJ, inner list
@@ -702,7 +738,7 @@ __global__ __launch_bounds__(kSortThreads) void nl_sort_batch(const BatchSys* __
     if (m.x < 0) return;
     const sponge_nl& L = bs[m.x].nl;
     nl_sort_body(m.y, L.col_cap, L.col_count, L.col_start, L.col_atoms, L.nl_uint, L.cof_dr[0], L.cof_dr[1],
-                 L.cof_dr[2], L.s2o, L.o2s, L.pack, L.cl_lo, L.cl_hi, L.flags);
+                 L.cof_dr[2], L.s2o, L.o2s, L.pack, L.cl_lo, L.cl_hi, L.col_z, L.flags);
 }
 
 __global__ __launch_bounds__(kPairWaves * 64) void nl_pairs_batch(const BatchSys* __restrict__ bs,
@@ -714,8 +750,8 @@ __global__ __launch_bounds__(kPairWaves * 64) void nl_pairs_batch(const BatchSys
     const BatchSys& b = bs[m.x];
     const sponge_nl& L = b.nl;
     nl_pairs_body(m.y, L.ncx, L.ncy, L.box[0], L.box[1], L.box[2], L.cof_dr[0], L.cof_dr[1], L.cof_dr[2], L.rl2,
-                  b.rlm, L.col_start, L.cl_lo, L.cl_hi, L.pack, b.io.excluded_list_start, b.io.excluded_numbers, b.io.excluded_list,
-                  L.list_cap, L.list_n, L.list, L.flags);
+                  b.rlm, L.col_start, L.col_z, L.cl_lo, L.cl_hi, L.pack, L.o2s, b.io.excluded_list_start, b.io.excluded_numbers, b.io.excluded_list,
+                  L.list_cap, L.list_n, L.list_pairs, L.list, L.flags);
 }
 
 __global__ void nl_uint_kernel(int n, const float* __restrict__ crd, float cqx, float cqy, float cqz,
@@ -794,8 +830,7 @@ extern "C" int sponge_nl_create(int atom_numbers, const float box_length[3], flo
     double rl = cws;
     double est = (4.0 / 3.0) * M_PI * std::pow(rl + 2.0 * w, 3) * dens / kClusterSize;
     int lc = (int)std::ceil(2.0 * est) + 64;
-    nl->list_cap = std::min(std::max(lc, 64), std::min(nl->ncl_cap, kCandCap));
-    nl->cand_cap = kCandCap;
+    nl->list_cap = std::min(std::max(lc, 64), std::min(nl->ncl_cap, kListCap));
 
     size_t n = atom_numbers;
     hipError_t e = hipSuccess;
@@ -806,6 +841,7 @@ extern "C" int sponge_nl_create(int atom_numbers, const float box_length[3], flo
     A((void**)&nl->nl_uint, 3 * n * sizeof(unsigned));
     A((void**)&nl->col_count, nl->ncol * sizeof(int));
     A((void**)&nl->col_start, (nl->ncol + 1) * sizeof(int));
+    A((void**)&nl->col_z, (size_t)nl->ncol * kZStride * sizeof(unsigned short));
     A((void**)&nl->col_atoms, (size_t)nl->ncol * nl->col_cap * sizeof(int));
     A((void**)&nl->s2o, nl->slot_cap * sizeof(int));
     A((void**)&nl->o2s, n * sizeof(int));
@@ -813,6 +849,7 @@ extern "C" int sponge_nl_create(int atom_numbers, const float box_length[3], flo
     A((void**)&nl->cl_lo, nl->ncl_cap * sizeof(float4));
     A((void**)&nl->cl_hi, nl->ncl_cap * sizeof(float4));
     A((void**)&nl->list_n, nl->ncl_cap * sizeof(int));
+    A((void**)&nl->list_pairs, nl->ncl_cap * sizeof(int));
     A((void**)&nl->list, (size_t)nl->ncl_cap * nl->list_cap * sizeof(uint2));
     A((void**)&nl->list_in, (size_t)nl->ncl_cap * nl->list_cap * sizeof(uint2));
     A((void**)&nl->list_in_n, nl->ncl_cap * sizeof(int));
@@ -833,6 +870,7 @@ extern "C" int sponge_nl_create(int atom_numbers, const float box_length[3], flo
     A((void**)&nl->flags, 16 * sizeof(int));
     if (e == hipSuccess) e = hipMemset(nl->flags, 0, 16 * sizeof(int));
     if (e == hipSuccess) e = hipMemset(nl->list_n, 0, nl->ncl_cap * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(nl->list_pairs, 0, nl->ncl_cap * sizeof(int));
     if (e == hipSuccess) e = hipMemset(nl->list_in_n, 0, nl->ncl_cap * sizeof(int));
     if (e == hipSuccess) e = hipMemset(nl->atom_in_n, 0, nl->slot_cap * sizeof(int));
     if (e == hipSuccess)
@@ -873,7 +911,7 @@ extern "C" void sponge_nl_destroy(sponge_nl* nl) {
     void* ptrs[] = {nl->old_crd, nl->nl_uint, nl->col_count, nl->col_start, nl->col_atoms, nl->s2o,
                     nl->o2s,     nl->cl_lo,   nl->cl_hi,     nl->list_n,    nl->list,      nl->pack,
                     nl->flags,   nl->list_in, nl->list_in_n, nl->sym_start, nl->sym_list, nl->atom_in_n,
-                    nl->atom_in, nl->dropped, nl->prune_ref, nl->atom_full_n, nl->atom_full};
+                    nl->atom_in, nl->dropped, nl->prune_ref, nl->atom_full_n, nl->atom_full, nl->col_z, nl->list_pairs};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     delete nl;
@@ -913,14 +951,15 @@ static int nl_rebuild(sponge_nl* nl, float* d_crd, const int* es, const int* el,
     SNB_CHECK_LAUNCH();
     nl_sort_kernel<<<nl->ncol, kSortThreads, 0, s>>>(nl->col_cap, nl->col_count, nl->col_start, nl->col_atoms,
                                                       nl->nl_uint, nl->cof_dr[0], nl->cof_dr[1], nl->cof_dr[2],
-                                                      nl->s2o, nl->o2s, nl->pack, nl->cl_lo, nl->cl_hi, nl->flags);
+                                                      nl->s2o, nl->o2s, nl->pack, nl->cl_lo, nl->cl_hi, nl->col_z,
+                                                      nl->flags);
     SNB_CHECK_LAUNCH();
     const float rlm = snb_nl_rlm(nl);
     int nblk = xcd_grid(ceil_div(nl->ncl_cap, kPairWaves));
     nl_pairs_kernel<<<nblk, kPairWaves * 64, 0, s>>>(
         nl->ncx, nl->ncy, nl->box[0], nl->box[1], nl->box[2], nl->cof_dr[0], nl->cof_dr[1], nl->cof_dr[2], nl->rl2,
-        rlm, nl->col_start, nl->cl_lo, nl->cl_hi, nl->pack, es, en, el, nl->list_cap, nl->list_n, nl->list,
-        nl->flags, nl->sym_start, nl->sym_list);
+        rlm, nl->col_start, nl->col_z, nl->cl_lo, nl->cl_hi, nl->pack, nl->o2s, es, en, el, nl->list_cap, nl->list_n,
+        nl->list_pairs, nl->list, nl->flags, nl->sym_start, nl->sym_list);
     SNB_CHECK_LAUNCH();
     if (nl->prune_interval > 0) {
         nl_slot_lists_kernel<<<xcd_grid(ceil_div(nl->ncl_cap, 4)), 256, 0, s>>>(
@@ -1057,9 +1096,14 @@ extern "C" int sponge_nl_status(sponge_nl* nl, long* pair_count, int* overflow_f
     int f[16];
     SNB_HIP(hipDeviceSynchronize());
     SNB_HIP(hipMemcpy(f, nl->flags, sizeof(f), hipMemcpyDeviceToHost));
-    unsigned long long pc;
-    memcpy(&pc, f + 8, sizeof(pc));
-    if (pair_count) *pair_count = (long)(pc / 2);
+    if (pair_count) {
+        // every unordered pair is listed from both of its atoms
+        std::vector<int> np(std::max(f[4], 1));
+        if (f[4] > 0) SNB_HIP(hipMemcpy(np.data(), nl->list_pairs, f[4] * sizeof(int), hipMemcpyDeviceToHost));
+        long sum = 0;
+        for (int c = 0; c < f[4]; c++) sum += np[c];
+        *pair_count = sum / 2;
+    }
     if (overflow_flags) *overflow_flags = f[1];
     if (rebuilds) *rebuilds = f[2];
     return f[1] ? SPONGE_NB_ECAPACITY : SPONGE_NB_OK;

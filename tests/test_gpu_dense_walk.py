@@ -145,3 +145,30 @@ def test_gradients(waters, cutoff, skin, ntypes):
             d = np.abs(g[k] - ref[k]).max() / np.abs(ref[k]).sum()
             say(f"    {name}: table {k} {d:.2e}")
             assert d <= tol[k - 1], (name, k)
+
+
+@pytest.mark.parametrize("waters,cutoff,skin", [(1, 0.9, 0.1), (27, 3.5, 0.5), (216, 9.2, 0.1), (700, 4.0, 0.3),
+                                                (1500, 12.0, 2.0)])
+def test_list(waters, cutoff, skin):
+    """The rebuild's z tables, runs and exclusion marks: the listed pairs are
+    the oracle's, bit for bit, with a second rebuild after every atom moved
+    across the faces of the box."""
+    import torch
+    from sponge_amd import nb
+    length = (waters * system.WATER_VOLUME) ** (1.0 / 3.0)
+    s = system.water_box(waters, round(length, 3), seed=waters, cutoff=cutoff, skin=skin, fft=(20, 20, 20))
+    say(f"[case] list waters {waters} box {s.box[0]:.3f} list radius {cutoff + skin}")
+    eng = nb.NonbondedEngine(s, refresh_interval=0)
+    x0 = eng.crd.clone()
+    for shift in (0.0, 0.37):
+        x = torch.remainder(x0 + shift * float(s.box[0]), float(s.box[0]))
+        eng.crd.copy_(torch.where(x >= float(s.box[0]), torch.zeros_like(x), x))
+        eng.update_neighbor_list(forced=1)
+        eng.crd_to_uint()
+        torch.cuda.synchronize()
+        eng.nl.check()
+        u = eng.uint_crd.cpu().numpy().view(np.uint32)
+        got, ref = eng.nl.pairs(), oracle.nl_brute(s, u)
+        say(f"    {len(got)} pairs, status {eng.nl.status()['pairs']}")
+        assert np.array_equal(got, ref)
+        assert eng.nl.status()["pairs"] == len(ref)

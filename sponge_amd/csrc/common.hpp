@@ -58,6 +58,7 @@ __device__ __forceinline__ bool slot_offset(int i, int j, int nsl, int& off) {
 // by the per-slot force loop).
 constexpr int kCoulTab = 1024;
 constexpr int kMaxLjTypes = 64;          // LDS pair table holds kMaxLjTypes^2 (A,B)
+constexpr int kRevCap = 16;              // reverse exclusion row of one atom (batched rebuilds)
 constexpr int kNumXcd = 8;               // MI355X: 8 XCDs, workgroups dealt round-robin
 // Largest PME grid axis: sponge_pme_create rejects larger axes, and the prep
 // kernels' per-x-plane LDS histograms hold this many planes
@@ -198,7 +199,8 @@ struct sponge_nl {
     uint4* pack;                // slot_cap sorted (ux, uy, uz, atom) at the last rebuild
     int* flags;                 // [0] rebuild flag, [1] overflow bits, [2] rebuild count,
                                 // [3] slot count, [4] cluster count, [5] atoms left out
-                                // (column overflow), [7] skin-check vote,
+                                // (column overflow), [6] the rebuild whose per-slot lists
+                                // atom_full holds, [7] skin-check vote,
                                 // [10] fused steps
                                 // completed since the last rebuild
     int device;
@@ -222,7 +224,9 @@ struct sponge_nl {
     // taken modulo the slot count when that is the shorter way (the slot
     // records carry kPkHalo copies on either side, so i + offset is always a
     // readable record). atom_full: every pair of the full list, written by
-    // each rebuild while the inner lists are on, or by the first fused step after a new prune setting (flags[14] holds
+    // each rebuild while the inner lists are on (and by every batched
+    // rebuild; flags[6] is the number of the rebuild that last wrote them),
+    // or by the first fused step after a new prune setting (flags[14] holds
     // that step's number). atom_in: the pairs of atom_full within prune_r2
     // when the prune radius is below the list radius (two levels).
     // flags[11] = 1 once a slot held more than atom_in_cap partners, or a
@@ -242,6 +246,11 @@ struct sponge_nl {
     const int* ex_en;
     int* sym_start;             // n + 1
     int* sym_list;              // 2 x excluded pairs
+    // batched rebuilds read the caller's CSR each time: its reverse rows (the
+    // atoms that name atom a, at most kRevCap of the rev_n[a] kept), rebuilt
+    // with the list; allocated by sponge_batch_create
+    int* rev_n;                 // n
+    int* rev;                   // n * kRevCap
 };
 
 struct sponge_lj {
@@ -357,7 +366,7 @@ struct PruneArgs {
     float r2 = 0.f;
     int* in_n = nullptr;        // cluster-pair inner list (soft-core LJ)
     uint2* in_list = nullptr;
-    int* full_n = nullptr;      // per-slot lists of every listed pair (plain LJ):
+    int* full_n = nullptr;      // per-slot lists of every listed pair (plain LJ; a batch: any):
     unsigned short* full_list = nullptr;  // 16-bit slot offsets
     int* atom_n = nullptr;      // per-slot inner lists, two levels only (else NULL): a prune
     unsigned short* atom_list = nullptr;  // filters the full ones
@@ -412,6 +421,8 @@ float snb_nl_rlm(const sponge_nl* nl);
 float snb_prune_vote_r2(float cutoff, float prune_radius);
 // Two-level per-slot lists: an inner prune radius below the list radius.
 inline bool snb_two_level(const sponge_nl* nl) { return nl->prune_interval > 0 && nl->prune_r2 < nl->rl2; }
+int snb_coulomb_table(PairScratch* ps, float beta, float rc);
+int snb_nl_reverse_rows(sponge_nl* nl);
 int snb_batch_prep(sponge_batch* b, int energy, int from_crd, int overwrite, hipStream_t s);
 int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s);
 int snb_batch_excluded(sponge_batch* b, hipStream_t s);

@@ -263,7 +263,9 @@ __device__ __forceinline__ void nl_sort_body(
     const int* __restrict__ col_atoms, const unsigned int* __restrict__ nl_uint,
     float crx, float cry, float crz, int* __restrict__ s2o, int* __restrict__ o2s,
     uint4* __restrict__ pack, float4* __restrict__ cl_lo, float4* __restrict__ cl_hi,
-    unsigned short* __restrict__ col_z, const int* flags) {
+    unsigned short* __restrict__ col_z, const int* flags, int* __restrict__ rev_n = nullptr,
+    int* __restrict__ rev = nullptr, const int* __restrict__ es = nullptr, const int* __restrict__ en = nullptr,
+    const int* __restrict__ el = nullptr) {
     if (!flags[0]) return;
     __shared__ unsigned long long key[kMaxColumn];
     int cnt = min(col_count[c], col_cap);
@@ -303,6 +305,13 @@ __device__ __forceinline__ void nl_sort_body(
             s2o[slot] = a;
             o2s[a] = slot;
             pack[slot] = make_uint4(nl_uint[3 * a], nl_uint[3 * a + 1], nl_uint[3 * a + 2], (unsigned)a);
+            if (rev) {
+                // this atom into the reverse rows of its exclusion partners
+                for (int q = es[a]; q < es[a] + en[a]; q++) {
+                    const int p = el[q], at = atomicAdd(rev_n + p, 1);
+                    if (at < kRevCap) rev[(size_t)p * kRevCap + at] = a;
+                }
+            }
         } else {
             s2o[slot] = -1;
             pack[slot] = make_uint4(0u, 0u, 0u, 0xffffffffu);
@@ -387,14 +396,16 @@ __device__ __forceinline__ int wrap(int v, int n) { return v < 0 ? v + n : v >= 
 // cluster's first atom with the product from three 4x4x1 MFMAs; a batch with a
 // value closer to (rc + skin)^2 than the expansion's rounding bound, and every
 // batch of a box too small for displacements from one atom (dense_walk.hpp
-// has both conditions), takes the list's own FP32 expression nl_dr2. With
-// symmetric exclusion lists (sym_start) each partner sets its bit in a mask on
-// its cluster among the candidates; without them the CSR is searched for every
-// pair in range.
+// has both conditions), takes the list's own FP32 expression nl_dr2. Each
+// exclusion partner of the i atoms (SYM: from the symmetric lists ex_a, ex_b;
+// else from the CSR's row and the reverse row of the counts ex_a and rows
+// ex_b) sets its bit in a mask on its cluster among the candidates; past kRevCap reverse partners the CSR is searched for
+// every pair in range.
 // Bound: latency of a wave's ~30 record loads and vector issue. Measured, 648 /
 // 4,446 / 10,013 / 23,570 / 96,120 atoms: 12 / 22 / 30 / 46 / 136 us against
 // 24 / 100 / 79 / 128 / 368 us with a box test of the candidates, one pair per
 // lane in the mask stage and one pair counter for all waves.
+template <bool SYM>
 __device__ __forceinline__ void nl_pairs_body(
     int lb, int ncx, int ncy, float bx, float by, float bz, float crx, float cry, float crz, float rl2,
     float rlm, const int* __restrict__ col_start, const unsigned short* __restrict__ col_z,
@@ -402,7 +413,7 @@ __device__ __forceinline__ void nl_pairs_body(
     const int* __restrict__ o2s,
     const int* __restrict__ es, const int* __restrict__ en, const int* __restrict__ el, int list_cap,
     int* __restrict__ list_n, int* __restrict__ list_pairs, uint2* __restrict__ list, int* flags,
-    const int* __restrict__ sym_start = nullptr, const int* __restrict__ sym_list = nullptr) {
+    const int* __restrict__ ex_a, const int* __restrict__ ex_b) {
     if (!flags[0]) return;
     __shared__ uint2 cands[kPairWaves][kCandWindow];  // (j cluster, mask of excluded pairs)
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -429,22 +440,33 @@ __device__ __forceinline__ void nl_pairs_body(
     // of atom i, its slot and cell column
     const int xi = lane >> 4, xk = lane & 15;
     const int xatom = (int)pack[ic * kClusterSize + xi].w;
-    int x0 = 0, x1 = 0;
-    if (sym_start && xatom >= 0) {
-        x0 = sym_start[xatom];
-        x1 = sym_start[xatom + 1];
+    // (its first xown partners in one row, the others in the reverse one)
+    int xrow = 0, xown = 0, xall = 0, back = 0;
+    if (xatom >= 0) {
+        if (SYM) {
+            xrow = ex_a[xatom];
+            xown = xall = ex_a[xatom + 1] - xrow;
+        } else {
+            back = ex_a[xatom];
+            xrow = es[xatom];
+            xown = en[xatom];
+            xall = xown + min(back, kRevCap);
+        }
     }
+    // false: a reverse row overflowed, the CSR is searched
+    const bool marked = SYM || !__any(back > kRevCap);
     auto partner = [&](int k, int& js, int& col) {
         js = -1;
-        if (k >= x1) return;
-        js = o2s[sym_list[k]];
+        if (k >= xall) return;
+        if (SYM) js = o2s[ex_b[xrow + k]];
+        else js = o2s[k < xown ? el[xrow + k] : ex_b[(size_t)xatom * kRevCap + k - xown]];
         if (js < 0) return;
         const uint4 b = pack[js];
         col = (int)(((unsigned long long)b.x * (unsigned)ncx) >> 32) * ncy +
               (int)(((unsigned long long)b.y * (unsigned)ncy) >> 32);
     };
     int xslot, xcol = 0;
-    partner(x0 + xk, xslot, xcol);
+    partner(xk, xslot, xcol);
 
     const float4 li = cl_lo[ic], hi = cl_hi[ic];
     const float cix = 0.5f * (li.x + hi.x), ciy = 0.5f * (li.y + hi.y);
@@ -517,12 +539,12 @@ __device__ __forceinline__ void nl_pairs_body(
             __builtin_amdgcn_wave_barrier();
             // the excluded pairs of each candidate (LDS atomics: two atoms'
             // partners may share a cluster)
-            if (sym_start) {
+            if (marked) {
                 int js = xslot, pc = xcol;
-                for (int kk = x0 + xk; __any(kk < x1); kk += 16) {
-                    if (kk != x0 + xk) partner(kk, js, pc);
+                for (int kk = xk; __any(kk < xall); kk += 16) {
+                    if (kk != xk) partner(kk, js, pc);
                     int src = -1;
-                    if (kk < x1 && js >= 0) {
+                    if (kk < xall && js >= 0) {
                         const int cx = pc / ncy, qx = wrap(cx - ax0, ncx), qy = wrap(pc - cx * ncy - ay0, ncy);
                         if (qx < nxr && qy < nyr) src = qx * nyr + qy - cb;
                     }
@@ -576,7 +598,7 @@ __device__ __forceinline__ void nl_pairs_body(
                         in |= nl_dr2(pack[ic * kClusterSize + i], b, crx, cry, crz) < rl2 ? 1u << i : 0u;
                 }
                 in &= ok;
-                if (!sym_start) {
+                if (!marked) {
 #pragma unroll
                     for (int i = 0; i < kClusterSize; i++)
                         if ((in >> i) & 1u)
@@ -622,7 +644,7 @@ __global__ __launch_bounds__(kPairWaves * 64) __attribute__((amdgpu_waves_per_eu
     const int* __restrict__ es, const int* __restrict__ en, const int* __restrict__ el, int list_cap,
     int* __restrict__ list_n, int* __restrict__ list_pairs, uint2* __restrict__ list, int* flags,
     const int* __restrict__ sym_start, const int* __restrict__ sym_list) {
-    nl_pairs_body(xcd_block(gridDim.x), ncx, ncy, bx, by, bz, crx, cry, crz, rl2, rlm, col_start, col_z, cl_lo, cl_hi,
+    nl_pairs_body<true>(xcd_block(gridDim.x), ncx, ncy, bx, by, bz, crx, cry, crz, rl2, rlm, col_start, col_z, cl_lo, cl_hi,
                   pack, o2s, es, en, el, list_cap, list_n, list_pairs, list, flags, sym_start, sym_list);
 }
 
@@ -635,15 +657,14 @@ __global__ __launch_bounds__(kPairWaves * 64) __attribute__((amdgpu_waves_per_eu
 // writes 64 entries' partners at once. A slot with more partners than cap,
 // or one beyond 16-bit reach, gets the count cap + 1 (its cluster then reads
 // the full list) and raises flags[11].
-__global__ __launch_bounds__(256) void nl_slot_lists_kernel(const int* __restrict__ flags,
-                                                            const int* __restrict__ list_n,
-                                                            const uint2* __restrict__ list, int list_cap,
-                                                            unsigned short* __restrict__ slot_list,
-                                                            int* __restrict__ slot_n, int cap, int* diag) {
+__device__ __forceinline__ void nl_slot_lists_body(int lb, int* __restrict__ flags, const int* __restrict__ list_n,
+                                                   const uint2* __restrict__ list, int list_cap,
+                                                   unsigned short* __restrict__ slot_list, int* __restrict__ slot_n,
+                                                   int cap) {
     if (!flags[0]) return;
     const int lane = threadIdx.x & 63;
-    const int lb = xcd_block(gridDim.x);
     const int ic = lb * 4 + (int)(threadIdx.x >> 6);
+    if (lb == 0 && threadIdx.x == 0) flags[6] = flags[2];  // this rebuild's lists
     if (lb < 0 || ic >= flags[4]) return;
     const int nsl = flags[3];
     const int n = min(list_n[ic], list_cap);
@@ -696,9 +717,16 @@ __global__ __launch_bounds__(256) void nl_slot_lists_kernel(const int* __restric
         if (slot_far) count = cap + 1;
         if (lane == ii) {
             slot_n[ic * kClusterSize + ii] = count;
-            if (count > cap) atomicOr(diag, 1);
+            if (count > cap) atomicOr(flags + 11, 1);
         }
     }
+}
+
+__global__ __launch_bounds__(256) void nl_slot_lists_kernel(int* __restrict__ flags, const int* __restrict__ list_n,
+                                                            const uint2* __restrict__ list, int list_cap,
+                                                            unsigned short* __restrict__ slot_list,
+                                                            int* __restrict__ slot_n, int cap) {
+    nl_slot_lists_body(xcd_block(gridDim.x), flags, list_n, list, list_cap, slot_list, slot_n, cap);
 }
 
 // ---- batched rebuild: one launch per stage over every system --------------
@@ -721,6 +749,9 @@ __global__ void nl_bin_batch(const BatchSys* __restrict__ bs, const int2* __rest
     if (m.x < 0) return;
     const BatchSys& b = bs[m.x];
     const sponge_nl& L = b.nl;
+    // (the reverse exclusion rows start empty; the sort fills them)
+    const int a = m.y * (int)blockDim.x + (int)threadIdx.x;
+    if (L.flags[0] && a < L.n) L.rev_n[a] = 0;
     nl_bin_body(m.y, L.n, b.io.crd, L.old_crd, L.nl_uint, L.box[0], L.box[1], L.box[2], L.cof_q[0], L.cof_q[1],
                 L.cof_q[2], L.ncx, L.ncy, L.col_cap, L.col_count, L.col_atoms, L.flags, L.o2s, L.dropped);
 }
@@ -738,10 +769,11 @@ __global__ __launch_bounds__(kSortThreads) void nl_sort_batch(const BatchSys* __
     if (m.x < 0) return;
     const sponge_nl& L = bs[m.x].nl;
     nl_sort_body(m.y, L.col_cap, L.col_count, L.col_start, L.col_atoms, L.nl_uint, L.cof_dr[0], L.cof_dr[1],
-                 L.cof_dr[2], L.s2o, L.o2s, L.pack, L.cl_lo, L.cl_hi, L.col_z, L.flags);
+                 L.cof_dr[2], L.s2o, L.o2s, L.pack, L.cl_lo, L.cl_hi, L.col_z, L.flags, L.rev_n, L.rev,
+                 bs[m.x].io.excluded_list_start, bs[m.x].io.excluded_numbers, bs[m.x].io.excluded_list);
 }
 
-__global__ __launch_bounds__(kPairWaves * 64) void nl_pairs_batch(const BatchSys* __restrict__ bs,
+__global__ __launch_bounds__(kPairWaves * 64) __attribute__((amdgpu_waves_per_eu(6))) void nl_pairs_batch(const BatchSys* __restrict__ bs,
                                                                   const int2* __restrict__ map, int nmap) {
     const int g = xcd_block(nmap);
     if (g < 0) return;
@@ -749,9 +781,19 @@ __global__ __launch_bounds__(kPairWaves * 64) void nl_pairs_batch(const BatchSys
     if (m.x < 0) return;
     const BatchSys& b = bs[m.x];
     const sponge_nl& L = b.nl;
-    nl_pairs_body(m.y, L.ncx, L.ncy, L.box[0], L.box[1], L.box[2], L.cof_dr[0], L.cof_dr[1], L.cof_dr[2], L.rl2,
+    nl_pairs_body<false>(m.y, L.ncx, L.ncy, L.box[0], L.box[1], L.box[2], L.cof_dr[0], L.cof_dr[1], L.cof_dr[2], L.rl2,
                   b.rlm, L.col_start, L.col_z, L.cl_lo, L.cl_hi, L.pack, L.o2s, b.io.excluded_list_start, b.io.excluded_numbers, b.io.excluded_list,
-                  L.list_cap, L.list_n, L.list_pairs, L.list, L.flags);
+                  L.list_cap, L.list_n, L.list_pairs, L.list, L.flags, L.rev_n, L.rev);
+}
+
+__global__ __launch_bounds__(256) void nl_slot_lists_batch(const BatchSys* __restrict__ bs,
+                                                           const int2* __restrict__ map, int nmap) {
+    const int g = xcd_block(nmap);
+    if (g < 0) return;
+    const int2 m = map[g];
+    if (m.x < 0) return;
+    const sponge_nl& L = bs[m.x].nl;
+    nl_slot_lists_body(m.y, L.flags, L.list_n, L.list, L.list_cap, L.atom_full, L.atom_full_n, L.atom_in_cap);
 }
 
 __global__ void nl_uint_kernel(int n, const float* __restrict__ crd, float cqx, float cqy, float cqz,
@@ -911,10 +953,17 @@ extern "C" void sponge_nl_destroy(sponge_nl* nl) {
     void* ptrs[] = {nl->old_crd, nl->nl_uint, nl->col_count, nl->col_start, nl->col_atoms, nl->s2o,
                     nl->o2s,     nl->cl_lo,   nl->cl_hi,     nl->list_n,    nl->list,      nl->pack,
                     nl->flags,   nl->list_in, nl->list_in_n, nl->sym_start, nl->sym_list, nl->atom_in_n,
-                    nl->atom_in, nl->dropped, nl->prune_ref, nl->atom_full_n, nl->atom_full, nl->col_z, nl->list_pairs};
+                    nl->atom_in, nl->dropped, nl->prune_ref, nl->atom_full_n, nl->atom_full, nl->col_z, nl->list_pairs, nl->rev_n, nl->rev};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     delete nl;
+}
+
+// Buffers of the batched rebuild's reverse exclusion rows.
+int snb_nl_reverse_rows(sponge_nl* nl) {
+    if (!nl->rev_n) SNB_HIP(hipMalloc((void**)&nl->rev_n, nl->n * sizeof(int)));
+    if (!nl->rev) SNB_HIP(hipMalloc((void**)&nl->rev, (size_t)nl->n * kRevCap * sizeof(int)));
+    return SPONGE_NB_OK;
 }
 
 // Squared displacement past which the fused step re-prunes its inner list:
@@ -963,8 +1012,7 @@ static int nl_rebuild(sponge_nl* nl, float* d_crd, const int* es, const int* el,
     SNB_CHECK_LAUNCH();
     if (nl->prune_interval > 0) {
         nl_slot_lists_kernel<<<xcd_grid(ceil_div(nl->ncl_cap, 4)), 256, 0, s>>>(
-            nl->flags, nl->list_n, nl->list, nl->list_cap, nl->atom_full, nl->atom_full_n, nl->atom_in_cap,
-            nl->flags + 11);
+            nl->flags, nl->list_n, nl->list, nl->list_cap, nl->atom_full, nl->atom_full_n, nl->atom_in_cap);
         SNB_CHECK_LAUNCH();
     }
     return SPONGE_NB_OK;
@@ -1193,6 +1241,8 @@ int snb_batch_nl(sponge_batch* b, int forced, hipStream_t s) {
     SNB_CHECK_LAUNCH();
     const int nmap = b->nblk[kStNlPairs];
     nl_pairs_batch<<<xcd_grid(nmap), kPairWaves * 64, 0, s>>>(b->d, b->map[kStNlPairs], nmap);
+    SNB_CHECK_LAUNCH();
+    nl_slot_lists_batch<<<xcd_grid(nmap), 256, 0, s>>>(b->d, b->map[kStNlPairs], nmap);
     SNB_CHECK_LAUNCH();
     return SPONGE_NB_OK;
 }

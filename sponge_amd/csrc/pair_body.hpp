@@ -183,12 +183,15 @@ __device__ __forceinline__ uint4 slot_record(const SlotRecords& r, unsigned w) {
 // factor from its cubic piece in LDS, else from the fitted erfc): the
 // displacement and r^2 to the partner record b, and the factor f of the
 // pair force f (dx, dy, dz) on atom i; 0 unless listed and r < rc. The pair
-// terms are pair_wave's, in FP32.
-template <int TB, bool TABLE>
+// terms are pair_wave's, in FP32. SOFT: scrow holds atom i's soft-core
+// records (s1 at scrow[sc2 + type j]), read by waves that meet a pair type
+// with A < 0.
+template <int TB, bool TABLE, bool SOFT = false>
 __device__ __forceinline__ float slot_pair(const uint4 b, unsigned ax, unsigned ay, unsigned az, float qi,
                                            const float2* srow, const float4* stab, float cx, float cy, float cz,
                                            float rc2, float beta, float mlog2e_b2, float ctab_scale, bool listed,
-                                           float& dx, float& dy, float& dz, float& r2) {
+                                           float& dx, float& dy, float& dz, float& r2,
+                                           const float4* scrow = nullptr, int sc2 = 0) {
     // with at most 4 types the y and z words carry no type bits
     dx = (float)(int)((b.x & ~3u) - ax) * cx;
     dy = (float)(int)((TB == 2 ? b.y : b.y & ~3u) - ay) * cy;
@@ -201,7 +204,7 @@ __device__ __forceinline__ float slot_pair(const uint4 b, unsigned ax, unsigned 
     const float rinv6 = rinv2 * rinv2 * rinv2;
     const int tj = TB == 2 ? (int)(b.x & 3u) : unpack_type(b);
     const float2 AB = srow[tj];
-    const float flj = (AB.y - AB.x * rinv6) * rinv6 * rinv2;
+    float flj = (AB.y - AB.x * rinv6) * rinv6 * rinv2;
     const float qq = qi * __uint_as_float(b.w);
     float fc;
     if (TABLE) {
@@ -218,6 +221,7 @@ __device__ __forceinline__ float slot_pair(const uint4 b, unsigned ax, unsigned 
         const float ecx = erfcx_poly(x);
         fc = qq * ex_ * fmaf(kTwoOverSqrtPi, x, ecx) * rinv * rinv2;
     }
+    if (SOFT && in && AB.x < 0.f) soft_pair(r2, qq, beta, mlog2e_b2, scrow[tj], scrow[sc2 + tj], flj, fc);
     return in ? flj - fc : 0.f;
 }
 
@@ -260,12 +264,12 @@ __device__ __forceinline__ void slot_finish(int islot, int k, const uint4* __res
 // Lanes past the end of a list read a record
 // too (offsets left from earlier prunes, or zero: always inside the records
 // and their copies) and are masked out.
-template <int TB, bool TABLE>
+template <int TB, bool TABLE, bool SOFT = false>
 __device__ __forceinline__ void pair_atoms(int ic, const unsigned short* __restrict__ lists, int n, int nmax,
                                            const uint4* __restrict__ pk, const float2* sab, const float4* stab,
                                            int nt, float cx, float cy, float cz, float rc2, float beta,
                                            const int* __restrict__ s2o, float* __restrict__ frc, int overwrite,
-                                           const PruneArgs& pa, const ExclArgs& ex) {
+                                           const PruneArgs& pa, const ExclArgs& ex, const float4* sc = nullptr) {
     const int lane = threadIdx.x & 63, ii = lane >> 4, k = lane & 15;
     const int islot = ic * kClusterSize + ii;
     const uint4 a = pk[islot];
@@ -275,6 +279,7 @@ __device__ __forceinline__ void pair_atoms(int ic, const unsigned short* __restr
     const float2* srow = sab + ti * nt;
     const float mlog2e_b2 = -1.4426950408889634f * (beta * beta);
     const unsigned* __restrict__ lw = reinterpret_cast<const unsigned*>(lists + (size_t)islot * pa.atom_cap);
+    const float4* scrow = SOFT ? sc + ti * nt : nullptr;
     const int nwords = (nmax + 1) >> 1;  // atom_cap is even: the dword stays inside the slot's list
     float fix = 0.f, fiy = 0.f, fiz = 0.f;
     const SlotRecords rec = slot_records(pk, islot, pa);
@@ -291,8 +296,9 @@ __device__ __forceinline__ void pair_atoms(int ic, const unsigned short* __restr
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             float dx, dy, dz, r2;
-            const float f = slot_pair<TB, TABLE>(h ? b1 : b0_, ax, ay, az, qi, srow, stab, cx, cy, cz, rc2, beta,
-                                                 mlog2e_b2, pa.ctab_scale, t + h < nk, dx, dy, dz, r2);
+            const float f = slot_pair<TB, TABLE, SOFT>(h ? b1 : b0_, ax, ay, az, qi, srow, stab, cx, cy, cz, rc2,
+                                                       beta, mlog2e_b2, pa.ctab_scale, t + h < nk, dx, dy, dz, r2,
+                                                       scrow, nt * nt);
             fix += f * dx;
             fiy += f * dy;
             fiz += f * dz;
@@ -420,15 +426,27 @@ __device__ __forceinline__ int longest(int n) {
 // waves that meet such a pair.
 // TB = 2: every type index is below 4 and sits in the x coordinate's low bits
 // alone (two instructions fewer per pair); TB = 6: the general 6-bit index.
-template <bool SOFT, int TB>
+// BATCH: a batch's step, which writes no lists and has no inner ones: it reads
+// the full per-slot lists, plain and soft-core handles alike, when the last
+// rebuild wrote them (a rebuild of the handle on its own with the inner lists
+// off does not).
+template <bool SOFT, int TB, bool BATCH>
 __device__ __forceinline__ void pair_wave(
     int ic, const float2* sab, const float4* stab, const int* __restrict__ flags, const int* __restrict__ list_n,
     const uint2* __restrict__ list, int list_cap, const uint4* __restrict__ pk, int nt, float cx, float cy, float cz,
     float rc2, float beta, const int* __restrict__ s2o, float* __restrict__ frc, int overwrite,
     const float4* __restrict__ sc, const PruneArgs& pa, const ExclArgs& ex) {
     const int lane = threadIdx.x & 63;
-    const ListStep step = list_step<SOFT>(ic, flags, pk, pa);
-    if (step.slots) {
+    if (BATCH && flags[6] == flags[2]) {
+        const int n = pa.full_n[ic * kClusterSize + (lane >> 4)], nmax = longest(n);
+        if (nmax <= pa.atom_cap) {
+            pair_atoms<TB, true, SOFT>(ic, pa.full_list, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
+                                       overwrite, pa, ex, sc);
+            return;
+        }
+    }
+    const ListStep step = BATCH ? ListStep{false, false, false, false} : list_step<SOFT>(ic, flags, pk, pa);
+    if (!SOFT && !BATCH && step.slots) {
         if (ic == 0 && lane == 0) atomicAdd(pa.diag + 1, 1);
         const bool filter = step.write_inner;
         const bool inner = step.two && !filter;
@@ -459,8 +477,8 @@ __device__ __forceinline__ void pair_wave(
         // and its inner lists follow until the full ones are written again
         if (filter && lane < kClusterSize) pa.atom_n[ic * kClusterSize + lane] = pa.atom_cap + 1;
     }
-    const bool write_cluster = SOFT && step.write_inner;
-    const bool use_inner = SOFT && pa.interval > 0 && !write_cluster;
+    const bool write_cluster = SOFT && !BATCH && step.write_inner;
+    const bool use_inner = SOFT && !BATCH && pa.interval > 0 && !write_cluster;
     const int ii = lane & 3, jj = (lane >> 2) & 3, g = lane >> 4, bit = lane & 15;
     const int islot = ic * kClusterSize + ii;
     const uint4 a = pk[islot];
@@ -559,7 +577,7 @@ __device__ __forceinline__ void pair_wave(
 // One block of the force-only pair kernel: the LJ (A, B) table and, when
 // given, the Coulomb table into LDS, then one i-cluster per wave (logical
 // block lb covers clusters W lb .. W lb + W - 1).
-template <bool SOFT, int TB, int W = kPairWaves>
+template <bool SOFT, int TB, int W = kPairWaves, bool BATCH = false>
 __device__ __forceinline__ void pair_body(
     int lb, const int* __restrict__ flags, const int* __restrict__ list_n, const uint2* __restrict__ list,
     int list_cap, const uint4* __restrict__ pk, const float2* __restrict__ ab, int nt, float cx, float cy, float cz,
@@ -576,7 +594,7 @@ __device__ __forceinline__ void pair_body(
     __syncthreads();
     const int ic = lb * W + (int)(threadIdx.x >> 6);
     if (lb < 0 || ic >= flags[4]) return;
-    pair_wave<SOFT, TB>(ic, sab, stab, flags, list_n, list, list_cap, pk, nt, cx, cy, cz, rc2, beta, s2o, frc,
+    pair_wave<SOFT, TB, BATCH>(ic, sab, stab, flags, list_n, list, list_cap, pk, nt, cx, cy, cz, rc2, beta, s2o, frc,
                         overwrite, sc, pa, ex);
 }
 

@@ -181,3 +181,30 @@ def test_config4_batch_matches_oracle():
             assert abs(p[k] - ref[rk]) <= 1e-6 * abs(ref[rk]), (s.name, k, p[k], ref[rk])
         assert p["pairs_in"] == ref["n_in"], s.name
     print(f"    worst force rel rms {worst:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("n_solute", [12, 40])
+def test_batched_lists_with_long_exclusion_rows(n_solute):
+    """The batched rebuild marks exclusion partners from the CSR's rows and
+    reverse rows; a solute of 40 mutually excluded atoms has reverse rows past
+    their capacity (the CSR is then searched). Lists equal the oracle's, and
+    forces from the per-slot lists equal those of each system's own step."""
+    import torch
+    from sponge_amd import nb
+    systems = [system.fep_system(w, lam, seed=4 + w, n_solute=n_solute, cutoff=7.0, skin=1.0)
+               for w, lam in ((150, 0.0), (420, 0.6))]
+    print("[case] long exclusion rows", [s.n for s in systems], flush=True)
+    engines = [nb.NonbondedEngine(s, refresh_interval=20) for s in systems]
+    batch = nb.BatchedSystems(engines)
+    batch.neighbor_list_update(forced=1)
+    batch.force_step(0, 0)
+    torch.cuda.synchronize()
+    got = [e.frc.cpu().numpy().astype(np.float64) for e in engines]
+    for s, e, f in zip(systems, engines, got):
+        e.nl.check()
+        u = e.uint_crd.cpu().numpy().view(np.uint32)
+        assert np.array_equal(e.nl.pairs(), oracle.nl_brute(s, u)), s.name
+        e.update_neighbor_list(forced=1)
+        e.force_step(0, 0, from_crd=True, overwrite=True)
+        torch.cuda.synchronize()
+        assert rel_rms(f, e.frc.cpu().numpy()) < 1e-6, s.name

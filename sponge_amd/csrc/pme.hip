@@ -63,11 +63,11 @@ constexpr int kGatherThreads = 256;
 // The reciprocal chain's kernels run beside the pair kernel, whose waves hold
 // 64 of a SIMD's 512 VGPRs each: a SIMD with six pair waves has 128 left, so
 // the chain kernels are held to 128 VGPRs (four waves per SIMD) and one of
-// their waves still fits there (radix-8 transforms otherwise take ~132, and
-// wait for pair waves to retire). Held to 64, they spill.
+// their waves still fits there. The plane convolution with all six radices
+// would spill there (its BC values wait in registers) and is held to 168.
 constexpr int kPmeMinWaves = 4;
-// (radix-8 sets only: the others need more registers and would spill)
-#define SNB_PME_CHAIN __attribute__((amdgpu_waves_per_eu(RM == kRadix8 ? kPmeMinWaves : 1)))
+#define SNB_PME_CHAIN __attribute__((amdgpu_waves_per_eu(kPmeMinWaves)))
+#define SNB_PME_PLANE __attribute__((amdgpu_waves_per_eu(RM == kRadixAll ? 3 : kPmeMinWaves)))
 
 __host__ __device__ __forceinline__ int row_blocks(int Ky) { return (Ky + kRowBlock - 1) / kRowBlock; }
 // LDS layout of transform lines. Stockham passes write each line at strides
@@ -132,33 +132,37 @@ __device__ __forceinline__ void dft(float2* v) {
         v[6] = csub(e[2], o2);
         v[3] = cadd(e[3], o3);
         v[7] = csub(e[3], o3);
-    } else if (R == 3) {
-        const float c = -0.5f, s = 0.86602540378443865f;
-        float2 t = cadd(v[1], v[2]);
-        float2 m = make_float2(v[0].x + c * t.x, v[0].y + c * t.y);
-        float2 d = csub(v[1], v[2]);
-        float2 rd = mul_i<SIGN>(make_float2(s * d.x, s * d.y));
-        v[0] = cadd(v[0], t);
-        v[1] = cadd(m, rd);
-        v[2] = csub(m, rd);
     } else {
-        // generic R (5, 7): y_s = sum_q v_q exp(SIGN 2 pi i q s / R)
-        float2 out[R];
+        // odd R: elements q and R - q enter output s through their sum times
+        // cos(2 pi q s / R) and their difference times sin(2 pi q s / R), and
+        // output R - s takes the same two sums (36 operations at R = 5 where
+        // the plain sums take 80)
+        constexpr int h = (R - 1) / 2;
+        float2 t[h + 1], d[h + 1], sum = v[0];
 #pragma unroll
-        for (int s_ = 0; s_ < R; s_++) {
-            float2 acc = v[0];
-#pragma unroll
-            for (int q = 1; q < R; q++) {
-                int m = (q * s_) % R;
-                float ang = (float)(2.0 * M_PI / R) * m;
-                float cs = __builtin_cosf(ang), sn = SIGN * __builtin_sinf(ang);
-                acc.x += v[q].x * cs - v[q].y * sn;
-                acc.y += v[q].x * sn + v[q].y * cs;
-            }
-            out[s_] = acc;
+        for (int q = 1; q <= h; q++) {
+            t[q] = cadd(v[q], v[R - q]);
+            d[q] = csub(v[q], v[R - q]);
+            sum = cadd(sum, t[q]);
         }
+        const float2 v0 = v[0];
+        v[0] = sum;
 #pragma unroll
-        for (int s_ = 0; s_ < R; s_++) v[s_] = out[s_];
+        for (int s = 1; s <= h; s++) {
+            float2 m = v0, u = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int q = 1; q <= h; q++) {
+                const double ang = (2.0 * M_PI / R) * ((q * s) % R);
+                const float c = (float)__builtin_cos(ang), sn = (float)__builtin_sin(ang);
+                m.x += c * t[q].x;
+                m.y += c * t[q].y;
+                u.x += sn * d[q].x;
+                u.y += sn * d[q].y;
+            }
+            const float2 iu = mul_i<SIGN>(u);
+            v[s] = cadd(m, iu);
+            v[R - s] = csub(m, iu);
+        }
     }
 }
 
@@ -167,6 +171,10 @@ __device__ __forceinline__ void dft(float2* v) {
 // 2^-22 (n + 1/2) / d of it, so the truncation is exact. A few VALU
 // operations instead of an integer division.
 __device__ __forceinline__ int div_small(int n, float rd) { return (int)(((float)n + 0.5f) * rd); }
+// 1 / d of a wave-uniform line length for div_small, one instruction instead
+// of an IEEE division's ten; its 1 ulp (2^-23) leaves div_small exact for
+// n < 2^20 (the indices divided are below 2^17).
+__device__ __forceinline__ float rcp_small(int d) { return __builtin_amdgcn_rcpf((float)d); }
 
 // One Stockham radix-R step over nlines lines of length K held in LDS;
 // element (line l, position p) lives at buf[l*ls + p*ks]; tw is the LDS
@@ -178,11 +186,17 @@ __device__ __forceinline__ int div_small(int n, float rd) { return (int)(((float
 template <int R, int SIGN>
 __device__ __forceinline__ void wave_pass(float2* buf, int nlines, int ls, int ks, int K, int Ns, int kons,
                                           const float2* tw, int wid, int nw, int lane) {
+    // Nothing of a pass is computed outside it: the offsets below depend only
+    // on the lane and the line length, and hoisted out of the pass loop they
+    // were computed, and held in registers, for every compiled radix (600
+    // instructions per transform, and 220 instead of 127 VGPRs with all six):
+    // a 20 x 20 plane's kernel took 12.5 us, 9.9 without that.
+    asm volatile("" : "+v"(lane));
     const int per = K / R;
     const int tws = kons / R;
-    const float rns = 1.0f / (float)Ns;
-    if (per <= 64) {
-        const float rper = 1.0f / (float)per;
+    const float rns = rcp_small(Ns);
+    if (64 * R >= kMaxGridAxis || per <= 64) {  // always, for R = 8
+        const float rper = rcp_small(per);
         const int G = div_small(64, rper);
         const int sub = div_small(lane, rper);
         const int j = lane - sub * per;
@@ -292,8 +306,8 @@ __device__ __forceinline__ void wave_pass(float2* buf, int nlines, int ls, int k
 // in. Kernels are instantiated for a few sets (kRadix8: 64- and 512-point
 // axes; kRadix34: e.g. 108 = 4 x 3 x 3 x 3; kRadix248: other powers of two)
 // besides all six radices: without the code of the radices an axis does not
-// use, the kernels need ~120 instead of ~210 VGPRs, so twice the waves fit a
-// SIMD. The host picks the smallest instantiated set that holds every pass.
+// use, the kernels take 60 to 113 VGPRs instead of 114 to 136 and fetch less
+// code. The host picks the smallest instantiated set that holds every pass.
 constexpr int kRadixAll = (1 << 2) | (1 << 3) | (1 << 4) | (1 << 5) | (1 << 7) | (1 << 8);
 constexpr int kRadix8 = 1 << 8;
 constexpr int kRadix34 = (1 << 3) | (1 << 4);
@@ -307,18 +321,23 @@ __device__ __forceinline__ void lds_fft(float2* buf, int nlines, int ls, int ks,
         const int R = (int)((p.code >> (4 * ps)) & 15ull);
         if ((RM & (1 << 8)) && R == 8) {
             wave_pass<8, SIGN>(buf, nlines, ls, ks, p.K, Ns, kons, tw, wid, nw, lane);
+            kons /= 8;
         } else if ((RM & (1 << 4)) && R == 4) {
             wave_pass<4, SIGN>(buf, nlines, ls, ks, p.K, Ns, kons, tw, wid, nw, lane);
+            kons /= 4;
         } else if ((RM & (1 << 2)) && R == 2) {
             wave_pass<2, SIGN>(buf, nlines, ls, ks, p.K, Ns, kons, tw, wid, nw, lane);
+            kons /= 2;
         } else if ((RM & (1 << 3)) && R == 3) {
             wave_pass<3, SIGN>(buf, nlines, ls, ks, p.K, Ns, kons, tw, wid, nw, lane);
+            kons /= 3;
         } else if ((RM & (1 << 5)) && R == 5) {
             wave_pass<5, SIGN>(buf, nlines, ls, ks, p.K, Ns, kons, tw, wid, nw, lane);
+            kons /= 5;
         } else if (RM & (1 << 7)) {
             wave_pass<7, SIGN>(buf, nlines, ls, ks, p.K, Ns, kons, tw, wid, nw, lane);
+            kons /= 7;
         }
-        kons /= R;
         Ns *= R;
     }
 }
@@ -415,7 +434,7 @@ __device__ __forceinline__ void spread_z_body(
     load_twiddles<kZThreads>(tz, twz, Kz);
     if (acc && x == 0 && yb == 0 && threadIdx.x == 0) acc[SPONGE_PART_RECIPROCAL] = 0.0;
     const int npt = nr * Kz;
-    const float rkz = 1.0f / (float)Kz, rnr = 1.0f / (float)nr;
+    const float rkz = rcp_small(Kz), rnr = rcp_small(nr);
     for (int idx = threadIdx.x; idx < npt; idx += kZThreads) {
         if (MODE == 0) {
             qhi[idx] = 0;
@@ -567,7 +586,7 @@ __global__ __launch_bounds__(kZThreads) void spread_z_adjoint_kernel(
 }
 
 // Batched: local block l = x * (row blocks) + row block.
-__global__ __launch_bounds__(kZThreads) void spread_z_batch(const BatchSys* __restrict__ bs,
+__global__ __launch_bounds__(kZThreads) SNB_PME_CHAIN void spread_z_batch(const BatchSys* __restrict__ bs,
                                                             const int2* __restrict__ map, int energy) {
     const int2 m = map[blockIdx.x];
     if (m.x < 0) return;
@@ -600,7 +619,7 @@ __device__ __forceinline__ void conv2d_body(int kz, float2* __restrict__ FQ, con
     float2* plane = FQ + (size_t)kz * Kx * Ky;
     const float* bcp = bc + (size_t)kz * Kx * Ky;
     const int np = Kx * Ky;
-    const float rky = 1.0f / (float)Ky;
+    const float rky = rcp_small(Ky);
     // The plane and its BC values are loaded in one memory round trip when
     // they fit CB points per thread (4,096 points: a 64 x 64 plane with 256
     // or 512 threads; the BC values wait in registers through the forward
@@ -609,62 +628,71 @@ __device__ __forceinline__ void conv2d_body(int kz, float2* __restrict__ FQ, con
     constexpr int CB = kConvBatch * (512 / NT);
     float bv[CB];
     const bool onepass = np <= CB * NT;
-    for (int s0 = threadIdx.x; s0 < np; s0 += CB * NT) {
+    for (int s0 = 0; s0 < np; s0 += CB * NT) {
         float2 v[CB];
 #pragma unroll
         for (int s = 0; s < CB; s++) {
-            const int idx = s0 + s * NT;
+            if (s0 + s * NT >= np) break;  // uniform: a small plane leaves early
+            const int idx = s0 + s * NT + (int)threadIdx.x;
             if (idx < np) {
                 v[s] = plane[idx];
                 if (onepass) bv[s] = bcp[idx];
             }
         }
-        if (s0 == (int)threadIdx.x) {
+        if (s0 == 0) {
             // the twiddle loads join the first round trip
             load_twiddles<NT>(tx, twx, Kx);
             load_twiddles<NT>(ty, twy, Ky);
         }
 #pragma unroll
         for (int s = 0; s < CB; s++) {
-            const int idx = s0 + s * NT;
+            if (s0 + s * NT >= np) break;
+            const int idx = s0 + s * NT + (int)threadIdx.x;
             if (idx < np) {
                 sm[plane_lds(idx, rky, Ky, pitch)] = v[s];
             }
         }
     }
     __syncthreads();
-    lds_fft<-1, NT, RM>(sm, Kx, pitch, 1, py, ty);
-    __syncthreads();
-    lds_fft<-1, NT, RM>(sm, Ky, 1, pitch, px, tx);
-    __syncthreads();
+    // Transforms 0 and 1 are the forward y and x ones; 2 and 3 the inverse x
+    // and y ones, taken as the conjugate of the forward transform of the
+    // conjugate (the same operations with the same roundings), so that all
+    // four run through one copy of the pass code: a plane of a small grid is
+    // one wave per SIMD, and fetching fresh code took as long as running it.
     double e = 0.0;
-    for (int s0 = threadIdx.x; s0 < np; s0 += CB * NT) {
-        if (!onepass) {
+#pragma nounroll
+    for (int t = 0; t < 4; t++) {
+        const bool along_y = t == 0 || t == 3;
+        lds_fft<-1, NT, RM>(sm, along_y ? Kx : Ky, along_y ? pitch : 1, along_y ? 1 : pitch, along_y ? py : px,
+                            along_y ? ty : tx);
+        __syncthreads();
+        if (t != 1) continue;
+        for (int s0 = 0; s0 < np; s0 += CB * NT) {
+            if (!onepass) {
+#pragma unroll
+                for (int s = 0; s < CB; s++) {
+                    const int idx = s0 + s * NT + (int)threadIdx.x;
+                    if (idx < np) bv[s] = bcp[idx];
+                }
+            }
 #pragma unroll
             for (int s = 0; s < CB; s++) {
-                const int idx = s0 + s * NT;
-                if (idx < np) bv[s] = bcp[idx];
+                if (s0 + s * NT >= np) break;
+                const int idx = s0 + s * NT + (int)threadIdx.x;
+                if (idx < np) {
+                    const int o = plane_lds(idx, rky, Ky, pitch);
+                    const float b = bv[s];
+                    const float2 w = sm[o];
+                    if (energy) e += (double)b * ((double)w.x * w.x + (double)w.y * w.y);
+                    sm[o] = make_float2(w.x * b, -(w.y * b));
+                }
             }
         }
-#pragma unroll
-        for (int s = 0; s < CB; s++) {
-            const int idx = s0 + s * NT;
-            if (idx < np) {
-                const int o = plane_lds(idx, rky, Ky, pitch);
-                const float b = bv[s];
-                const float2 w = sm[o];
-                if (energy) e += (double)b * ((double)w.x * w.x + (double)w.y * w.y);
-                sm[o] = make_float2(w.x * b, w.y * b);
-            }
-        }
+        __syncthreads();
     }
-    __syncthreads();
-    lds_fft<1, NT, RM>(sm, Ky, 1, pitch, px, tx);
-    __syncthreads();
-    lds_fft<1, NT, RM>(sm, Kx, pitch, 1, py, ty);
-    __syncthreads();
     for (int idx = threadIdx.x; idx < np; idx += NT) {
-        plane[idx] = sm[plane_lds(idx, rky, Ky, pitch)];
+        const float2 w = sm[plane_lds(idx, rky, Ky, pitch)];
+        plane[idx] = make_float2(w.x, -w.y);
     }
     if (energy) {
         const double t = block_sum<NT>(e, red);
@@ -674,7 +702,7 @@ __device__ __forceinline__ void conv2d_body(int kz, float2* __restrict__ FQ, con
 }
 
 template <int RM>
-__global__ __launch_bounds__(kConvThreads) SNB_PME_CHAIN void conv2d_kernel(float2* __restrict__ FQ, const float* __restrict__ bc,
+__global__ __launch_bounds__(kConvThreads) SNB_PME_PLANE void conv2d_kernel(float2* __restrict__ FQ, const float* __restrict__ bc,
                                                               int Kx, int Ky, int Kz, FftPlan px, FftPlan py,
                                                               const float2* __restrict__ twx,
                                                               const float2* __restrict__ twy, int energy,
@@ -685,14 +713,14 @@ __global__ __launch_bounds__(kConvThreads) SNB_PME_CHAIN void conv2d_kernel(floa
 // The same with 512 threads (8 waves) per plane: more waves to hide the LDS
 // latency of the transform passes, where the CUs are free to hold them.
 template <int RM>
-__global__ __launch_bounds__(2 * kConvThreads) SNB_PME_CHAIN void conv2d_wide_kernel(
+__global__ __launch_bounds__(2 * kConvThreads) SNB_PME_PLANE void conv2d_wide_kernel(
     float2* __restrict__ FQ, const float* __restrict__ bc, int Kx, int Ky, int Kz, FftPlan px, FftPlan py,
     const float2* __restrict__ twx, const float2* __restrict__ twy, int energy, double* __restrict__ acc,
     int* __restrict__ bin_count) {
     conv2d_body<RM, 2 * kConvThreads>(blockIdx.x, FQ, bc, Kx, Ky, Kz, px, py, twx, twy, energy, acc, bin_count);
 }
 
-__global__ __launch_bounds__(kConvThreads) void conv2d_batch(const BatchSys* __restrict__ bs,
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(3))) void conv2d_batch(const BatchSys* __restrict__ bs,
                                                              const int2* __restrict__ map, int energy) {
     const int2 m = map[blockIdx.x];
     if (m.x < 0) return;
@@ -724,7 +752,7 @@ __device__ __forceinline__ void conv_y_body(int bx, int kz, float2* __restrict__
     const int x0 = bx * kLines, nl = min(kLines, Kx - x0);
     float2* rows = FQ + ((size_t)kz * Kx + x0) * Ky;
     const int np = nl * Ky;
-    const float rky = 1.0f / (float)Ky;
+    const float rky = rcp_small(Ky);
     // kConvBatch loads per thread in flight at a time; the twiddle loads
     // join the first round
     for (int s0 = threadIdx.x; s0 < np; s0 += kConvBatch * kLineThreads) {
@@ -865,10 +893,11 @@ __device__ __forceinline__ void inv_z_body(int x, int yb, const float2* __restri
     float2* rows = sm;                      // nr x H
     float2* pk = sm + kRowBlock * H;        // nrp lines at pitch zp
     float2* tz = pk + (kRowBlock / 2) * zp;
-    const float rkz = 1.0f / (float)Kz, rnr = 1.0f / (float)nr;
+    const float rkz = rcp_small(Kz), rnr = rcp_small(nr);
     float2 v[kZPer];
 #pragma unroll
     for (int s = 0; s < kZPer; s++) {
+        if (s * kZThreads >= nr * H) break;  // uniform
         const int idx = threadIdx.x + s * kZThreads;
         if (idx < nr * H) {
             const int k = div_small(idx, rnr), r = idx - k * nr;
@@ -879,6 +908,7 @@ __device__ __forceinline__ void inv_z_body(int x, int yb, const float2* __restri
     load_twiddles<kZThreads>(tz, twz, Kz);
 #pragma unroll
     for (int s = 0; s < kZPer; s++) {
+        if (s * kZThreads >= nr * H) break;  // uniform
         const int idx = threadIdx.x + s * kZThreads;
         if (idx < nr * H) {
             const int k = div_small(idx, rnr), r = idx - k * nr;
@@ -923,7 +953,7 @@ __global__ __launch_bounds__(kZThreads) SNB_PME_CHAIN void inv_z_kernel(const fl
     inv_z_body<RM>(x, blockIdx.x - x * nyb, FQ, R, Kx, Ky, Kz, pz, twz);
 }
 
-__global__ __launch_bounds__(kZThreads) void inv_z_batch(const BatchSys* __restrict__ bs,
+__global__ __launch_bounds__(kZThreads) SNB_PME_CHAIN void inv_z_batch(const BatchSys* __restrict__ bs,
                                                          const int2* __restrict__ map) {
     const int2 m = map[blockIdx.x];
     if (m.x < 0) return;
@@ -1053,7 +1083,7 @@ __device__ __forceinline__ void spread_yz_body(int x, const unsigned* __restrict
     __syncthreads();
     // rows (2p, 2p + 1) -> the real and imaginary parts of z-line p
     float* pkf = reinterpret_cast<float*>(pk);
-    const float rkz = 1.0f / (float)Kz, rky = 1.0f / (float)Ky;
+    const float rkz = rcp_small(Kz), rky = rcp_small(Ky);
     for (int idx = threadIdx.x; idx < npt; idx += NT) {
         const int r = div_small(idx, rkz), z = idx - r * Kz;
         const long long q = (long long)qhi[idx] * 65536ll + (long long)qlo[idx];
@@ -1103,7 +1133,7 @@ __device__ __forceinline__ void inv_yz_body(int x, const float2* __restrict__ FQ
     float2* pk = sm + yz_tile(Ky, Kz); // nrp lines at pitch zp
     float2* tz = pk + yz_lines(Ky, Kz);
     float2* ty = tz + Kz;
-    const float rky = 1.0f / (float)Ky, rkz = 1.0f / (float)Kz;
+    const float rky = rcp_small(Ky), rkz = rcp_small(Kz);
     const int np = Ky * H;
     // kConvBatch loads per thread in flight at a time; the twiddle loads
     // join the first round

@@ -43,6 +43,7 @@ namespace {
 constexpr int kRowBlock = 16;
 constexpr int kZThreads = 256;
 constexpr int kSpreadPerThread = 8;
+constexpr int kSpreadRing = 128;  // a wave's queue: at most 63 left over + 64 pushed
 // Fixed-point unit of the spread grid: one contribution q*Mx*My*Mz must stay
 // below 2^31 units, i.e. |q| < 128 / (2/3)^3 = 432 (18.2223 x 23.7 e).
 constexpr float kSpreadScale = 16777216.0f;
@@ -80,6 +81,10 @@ __host__ __device__ __forceinline__ int padded_len(int K) { return pd(K - 1) + 1
 __host__ __device__ __forceinline__ int pitch16(int n) { return ((n + 14) / 16) * 16 + 1; }
 // pitch of the packed z-lines and of the y direction of the convolution plane
 __host__ __device__ __forceinline__ int line_pitch(int K) { return pitch16(padded_len(K)); }
+// offset of the spread's queues: after its sums, packed lines and twiddles
+__host__ __device__ __forceinline__ int spread_queue_at(int Kz) {
+    return (kRowBlock * Kz + (kRowBlock / 2) * line_pitch(Kz) + Kz + 1) & ~1;
+}
 // LDS offset of point idx = x Ky + y of a padded plane (row pitch `pitch`);
 // rky = 1 / Ky. 24-bit multiplies (full rate; every index here < 2^24).
 __device__ __forceinline__ int plane_lds(int idx, float rky, int Ky, int pitch) {
@@ -387,6 +392,41 @@ __device__ __forceinline__ float bsp_dw(float f, int k) {
     }
 }
 
+// Orders a wave's LDS writes before its later reads by other lanes (LDS
+// operations of one wave execute in order: no instruction, only no reordering).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One queued record per lane: its four rows of four points added to the
+// block's sums.
+__device__ __forceinline__ void spread_wave(float4 f, int nr, int Ky, int Kz, int* qhi, unsigned* qlo) {
+    const int d = (int)(__float_as_uint(f.w) & 0xffffu), bz = (int)(__float_as_uint(f.w) >> 16);
+    float wz[4];
+    int gz[4];
+#pragma unroll
+    for (int kz = 0; kz < 4; kz++) {
+        wz[kz] = bsp_w(f.y, kz);
+        const int tt = bz - kz;
+        gz[kz] = tt + (tt < 0 ? Kz : 0);
+    }
+#pragma unroll
+    for (int ky = 0; ky < 4; ky++) {
+        int rr = d - ky;
+        rr += rr < 0 ? Ky : 0;
+        if (rr >= nr) continue;
+        const float wy = f.z * bsp_w(f.x, ky);
+        const int row = (int)__umul24((unsigned)rr, (unsigned)Kz);
+#pragma unroll
+        for (int kz = 0; kz < 4; kz++) {
+            const int c = __float2int_rn(wy * wz[kz]);
+            atomicAdd(qhi + row + gz[kz], c >> 16);
+            atomicAdd(qlo + row + gz[kz], (unsigned)c & 0xffffu);
+        }
+    }
+}
+
 // PME_Q_Spread (PME_force.cu:428-471) fused with the forward z transform of
 // one block of kRowBlock y rows of one x plane: grid point (base - k) gets
 // q M4(fx+kx) M4(fy+ky) M4(fz+kz); plane x receives the atoms filed under
@@ -397,6 +437,12 @@ __device__ __forceinline__ float bsp_dw(float f, int k) {
 // in which atoms arrive), converted, paired into complex z-lines (row r is
 // the real (r even) or imaginary (r odd) part of line r/2), transformed, and
 // unpacked (R2C) straight into the spectrum, stored [kz][x][y].
+//
+// About 30 % of the four planes' atoms (64 rows in blocks of 16) have a row in
+// the block: each wave queues those in a ring in LDS and adds 64 of them at a
+// time, so the weights and atomics run on full waves (12.8 -> 11.4 us at
+// 23,570 atoms on 64^3, 27.3 -> 23.9 at 96,120 on 108^3, beside the pair
+// kernel).
 //
 // MODE 1 spreads, instead of the charge, the adjoint source of the
 // force-matching gradient, q_i w_i . grad M_i(g): wv[i] = (w_x Kx/Lx,
@@ -431,6 +477,12 @@ __device__ __forceinline__ void spread_z_body(
     unsigned* qlo = reinterpret_cast<unsigned*>(sm) + kRowBlock * Kz;       //         nr x Kz
     float2* pk = sm + kRowBlock * Kz;                                       // nrp lines at pitch zp
     float2* tz = pk + (kRowBlock / 2) * zp;
+    // the wave's queue of records whose stencil meets the block's rows: ring
+    // of 128 x (fy, fz, q unit ax, row offset | bz << 16)
+    float4* const ring =
+        reinterpret_cast<float4*>(sm + spread_queue_at(Kz)) + kSpreadRing * (int)(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    int rhead = 0, rcount = 0;
     load_twiddles<kZThreads>(tz, twz, Kz);
     if (acc && x == 0 && yb == 0 && threadIdx.x == 0) acc[SPONGE_PART_RECIPROCAL] = 0.0;
     const int npt = nr * Kz;
@@ -480,20 +532,39 @@ __device__ __forceinline__ void spread_z_body(
                 ff[r] = rec_frac[sl[r]];
                 if (MODE) ai[r] = bin_atoms[sl[r]];
             }
+        if (MODE == 0) {
+#pragma unroll
+            for (int r = 0; r < kSpreadPerThread; r++) {
+                if (t0 + r * kZThreads >= total) break;  // uniform
+                // stencil rows by - ky, ky = 0..3, relative to the block: one
+                // of them is a row of it when d < nr + 3
+                int d = (int)((bb[r] >> 10) & 1023u) - y0;
+                d += d < 0 ? Ky : 0;
+                const bool inside = sl[r] >= 0 && d < nr + 3;
+                const unsigned long long in = __ballot(inside);
+                if (inside) {
+                    const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(in >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((unsigned)in, 0u));
+                    ring[(rhead + rcount + rank) & (kSpreadRing - 1)] =
+                        make_float4(ff[r].y, ff[r].z, ff[r].w * unit * bsp_w(ff[r].x, akx[r]),
+                                    __uint_as_float((unsigned)d | (bb[r] >> 20) << 16));
+                }
+                rcount += __popcll(in);
+                if (rcount >= 64) {
+                    wave_lds_sync();
+                    spread_wave(ring[(rhead + lane) & (kSpreadRing - 1)], nr, Ky, Kz, qhi, qlo);
+                    rhead += 64;
+                    rcount -= 64;
+                }
+            }
+            continue;
+        }
 #pragma unroll
         for (int r = 0; r < kSpreadPerThread; r++) {
             if (sl[r] < 0) continue;
-            // stencil rows by - ky, ky = 0..3, relative to the block
             int d = (int)((bb[r] >> 10) & 1023u) - y0;
             d += d < 0 ? Ky : 0;
-            bool inside = false;
-#pragma unroll
-            for (int ky = 0; ky < 4; ky++) {
-                int rr = d - ky;
-                rr += rr < 0 ? Ky : 0;
-                inside |= rr < nr;
-            }
-            if (!inside) continue;
+            if (d >= nr + 3) continue;
             const float4 f = ff[r];
             const int bz = (int)(bb[r] >> 20);
             float wz[4], dz[4];
@@ -501,44 +572,33 @@ __device__ __forceinline__ void spread_z_body(
 #pragma unroll
             for (int kz = 0; kz < 4; kz++) {
                 wz[kz] = bsp_w(f.z, kz);
-                if (MODE) dz[kz] = bsp_dw(f.z, kz);
+                dz[kz] = bsp_dw(f.z, kz);
                 int tt = bz - kz;
                 gz[kz] = tt + (tt < 0 ? Kz : 0);
             }
-            float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (MODE) w = wv[ai[r]];
+            const float4 w = wv[ai[r]];
             const float qs = f.w * unit;
             const float ax = bsp_w(f.x, akx[r]);
-            const float dax = MODE ? bsp_dw(f.x, akx[r]) : 0.f;
+            const float dax = bsp_dw(f.x, akx[r]);
 #pragma unroll
             for (int ky = 0; ky < 4; ky++) {
                 int rr = d - ky;
                 rr += rr < 0 ? Ky : 0;
                 if (rr >= nr) continue;
-                const float ay = bsp_w(f.y, ky);
+                const float ay = bsp_w(f.y, ky), day = bsp_dw(f.y, ky);
                 unsigned long long* row = qacc + rr * Kz;
-                if (MODE == 0) {
-                    const float wy = qs * ax * ay;
-                    int* rhi = qhi + rr * Kz;
-                    unsigned* rlo = qlo + rr * Kz;
+                const float c1 = qs * (w.x * dax * ay + w.y * ax * day);
+                const float c2 = qs * w.z * ax * ay;
 #pragma unroll
-                    for (int kz = 0; kz < 4; kz++) {
-                        const int c = __float2int_rn(wy * wz[kz]);
-                        atomicAdd(rhi + gz[kz], c >> 16);
-                        atomicAdd(rlo + gz[kz], (unsigned)c & 0xffffu);
-                    }
-                } else {
-                    const float day = bsp_dw(f.y, ky);
-                    const float c1 = qs * (w.x * dax * ay + w.y * ax * day);
-                    const float c2 = qs * w.z * ax * ay;
-#pragma unroll
-                    for (int kz = 0; kz < 4; kz++)
-                        atomicAdd(row + gz[kz],
-                                  (unsigned long long)(long long)__float2int_rn(fmaf(c1, wz[kz], c2 * dz[kz])));
-                }
+                for (int kz = 0; kz < 4; kz++)
+                    atomicAdd(row + gz[kz],
+                              (unsigned long long)(long long)__float2int_rn(fmaf(c1, wz[kz], c2 * dz[kz])));
             }
         }
     }
+    wave_lds_sync();
+    if (MODE == 0 && lane < rcount)
+        spread_wave(ring[(rhead + lane) & (kSpreadRing - 1)], nr, Ky, Kz, qhi, qlo);
     __syncthreads();
     float* pkf = reinterpret_cast<float*>(pk);
     for (int idx = threadIdx.x; idx < npt; idx += kZThreads) {
@@ -1414,7 +1474,7 @@ int plan_axis(int K, FftPlan* p) {
 
 // Dynamic LDS of the three transform kernels (bytes).
 size_t spread_z_lds(int Kz) {
-    return (size_t)(kRowBlock * Kz + (kRowBlock / 2) * line_pitch(Kz) + Kz) * sizeof(float2);
+    return (size_t)spread_queue_at(Kz) * sizeof(float2) + (kZThreads / 64) * kSpreadRing * sizeof(float4);
 }
 size_t inv_z_lds(int Kz) {
     return (size_t)(kRowBlock * (Kz / 2 + 1) + (kRowBlock / 2) * line_pitch(Kz) + Kz) * sizeof(float2);

@@ -196,10 +196,15 @@ __global__ __launch_bounds__(1024) void pressure_kernel(int n, const float* __re
                                                         float* __restrict__ pressure, float* __restrict__ ek_out) {
     __shared__ double red[16];
     double ek = 0.0, av = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    // one block: the loads of four (eight) atoms in flight per thread
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += 1024) {
         const double vx = vel[3 * i], vy = vel[3 * i + 1], vz = vel[3 * i + 2];
         ek += 0.5 * (vx * vx + vy * vy + vz * vz) * (double)mass[i];
-        if (atom_virial) av += atom_virial[i];
+    }
+    if (atom_virial) {
+#pragma unroll 8
+        for (int i = threadIdx.x; i < n; i += 1024) av += atom_virial[i];
     }
     ek = block_sum<1024>(ek, red);
     av = block_sum<1024>(av, red);

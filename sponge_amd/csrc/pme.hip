@@ -1389,16 +1389,19 @@ __global__ __launch_bounds__(kGatherThreads) void pme_gather_batch(const BatchSy
 // Energy / virial bookkeeping of PME_Reciprocal_Force_With_Energy_And_Virial
 // (PME_force.cu:753-771) with FP64 sums: potential += corr + self + rec,
 // virial += direct + corr + self + rec.
-__global__ void pme_finalize_kernel(int n, const float* __restrict__ dir_atom, const float* __restrict__ corr_atom,
+__global__ __launch_bounds__(1024) void pme_finalize_kernel(int n, const float* __restrict__ dir_atom, const float* __restrict__ corr_atom,
                                     double beta, double nf, int need_energy, int need_virial,
                                     float* __restrict__ d_potential, float* __restrict__ d_virial,
                                     double* __restrict__ acc) {
     __shared__ double red[16];
     double sd = 0.0, sc = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        if (dir_atom) sd += dir_atom[i];
-        sc += corr_atom[i];
+    // one block: eight loads in flight per thread, added in order
+    if (dir_atom) {
+#pragma unroll 8
+        for (int i = threadIdx.x; i < n; i += 1024) sd += dir_atom[i];
     }
+#pragma unroll 8
+    for (int i = threadIdx.x; i < n; i += 1024) sc += corr_atom[i];
     double tsd = block_sum<1024>(sd, red);
     double tsc = block_sum<1024>(sc, red);
     if (threadIdx.x == 0) {

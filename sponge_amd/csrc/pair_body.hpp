@@ -440,8 +440,8 @@ __device__ __forceinline__ void pair_wave(
     if (BATCH && flags[6] == flags[2]) {
         const int n = pa.full_n[ic * kClusterSize + (lane >> 4)], nmax = longest(n);
         if (nmax <= pa.atom_cap) {
-            pair_atoms<TB, true, SOFT>(ic, pa.full_list, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
-                                       overwrite, pa, ex, sc);
+            pair_atoms<TB, false, SOFT>(ic, pa.full_list, n, nmax, pk, sab, stab, nt, cx, cy, cz, rc2, beta, s2o, frc,
+                                        overwrite, pa, ex, sc);
             return;
         }
     }

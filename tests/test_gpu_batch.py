@@ -208,3 +208,45 @@ def test_batched_lists_with_long_exclusion_rows(n_solute):
         e.force_step(0, 0, from_crd=True, overwrite=True)
         torch.cuda.synchronize()
         assert rel_rms(f, e.frc.cpu().numpy()) < 1e-6, s.name
+
+
+@pytest.mark.parametrize("between", ["other_beta", "larger_scratch"])
+def test_batch_forces_are_its_own_pme_beta(between):
+    """A batch's forces belong to its own PME handles: fused steps of its LJ
+    handles with PME handles of another tolerance (another beta), or calls with
+    lists of more slots (which replace the handles' scratch; sponge_batch_sync
+    follows), change nothing. The order of the exclusion stage's float atomics
+    is the only difference between the two steps: 1e-7, as above."""
+    import torch
+    from sponge_amd import nb
+    systems = [system.config(0), system.fep_system(150, 0.3, seed=5, cutoff=7.0, skin=1.0)]
+    print("[case] batch beta", between, [s.n for s in systems], flush=True)
+    engines = [nb.NonbondedEngine(s, refresh_interval=20) for s in systems]
+    batch = nb.BatchedSystems(engines)
+    batch.neighbor_list_update(forced=1)
+    batch.force_step(0, 0)
+    torch.cuda.synchronize()
+    before = [e.frc.cpu().numpy().copy() for e in engines]
+    for s, e in zip(systems, engines):
+        if between == "other_beta":
+            own = e.pme
+            e.pme = nb.Particle_Mesh_Ewald(s.n, e.box, s.cutoff, 1e-2, *s.fft)
+            assert abs(e.pme.beta - own.beta) > 0.05
+            e.force_step(0, 0, from_crd=True, overwrite=True)
+            torch.cuda.synchronize()
+            assert rel_rms(e.frc.cpu().numpy(), before[engines.index(e)]) > 1e-6
+            e.pme = own
+        else:
+            # the same volume as a flat box: 20 times the cell columns, each
+            # with room for padding slots (never rebuilt: no slot in use)
+            x, y, z = e.box
+            flat = nb.NEIGHBOR_LIST(s.n, [4.0 * x, 4.0 * y, z / 16.0], s.cutoff, s.skin)
+            e.lj.LJ_Force_With_PME_Direct_Force(e.uint_crd, e.charge, e.frc, flat, e.pme.beta)
+            torch.cuda.synchronize()
+    batch.sync()
+    batch.force_step(0, 0)
+    torch.cuda.synchronize()
+    for s, e, f in zip(systems, engines, before):
+        err = rel_rms(e.frc.cpu().numpy(), f)
+        print(f"    {s.name}: {err:.2e}", flush=True)
+        assert err < 1e-7, s.name

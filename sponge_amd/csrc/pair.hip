@@ -215,7 +215,7 @@ __global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(!SOFT ? 
 // their per-atom sums up in wave order, so these repeat bit for bit.
 // Bound: vector issue (scan ~130 instructions per 256 listed pairs, terms
 // ~110 per 64 pairs inside the cutoff) at 4 waves per SIMD. Energies and
-// forces measured, 23,570 / 96,120 atoms at 10 A: 89 + 27 and 306 + 168 us,
+// forces measured, 23,570 / 96,120 atoms at 10 A: 89 + 32 and 300 + 169 us,
 // against 369 and 1,362 us with both on 16 lanes per listed cluster pair and
 // the device library's erfc; 10,013 atoms without per-slot lists 55 + 37
 // against 191 us.
@@ -813,14 +813,16 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
         if (!d_frc) return SPONGE_NB_OK;
     }
     // the per-slot force loop of force-only plain steps reads the Coulomb
-    // force factor from a table in LDS; every fused step makes sure it
-    // exists (built by the first one, so that a prune schedule turned on
-    // later allocates nothing inside a graph capture)
-    if (fused && !sc && ps->pk_alloc) {
+    // force factor from a table in LDS; every such step makes sure it exists
+    // (built by the first one, so that a prune schedule turned on later
+    // allocates nothing inside a graph capture). Energy steps take the fitted
+    // erfc, the more exact of the two (the table's is 1.6e-5 of the force of
+    // two charges 0.15 A apart, the erfc's 7e-7), and build nothing.
+    if (fused && !energy && !sc && ps->pk_alloc) {
         rc = coulomb_table(ps, beta, cutoff);
         if (rc) return rc;
     }
-    if (inner && !sc) {
+    if (inner && !energy && !sc) {
         pa.ctab = ps->ctab;
         pa.ctab_scale = (float)kCoulTab / (cutoff * 1.0001f);
         lds = ((lds + 15) & ~(size_t)15) + kCoulTab * sizeof(float4);

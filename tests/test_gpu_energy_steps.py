@@ -1,0 +1,99 @@
+"""Energy steps beside force-only ones: the same pair terms to the same
+precision, and nothing allocated or built that the step does not read."""
+import dataclasses
+import sys
+
+import numpy as np
+import pytest
+
+import oracle
+from sponge_amd import system
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def rel_rms(a, b):
+    a = np.asarray(a, np.float64)
+    b = np.asarray(b, np.float64)
+    return float(np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum()))
+
+
+def dimers():
+    """216 pairs of opposite charges 0.15 to 0.3 A apart, 6.7 A from each
+    other, without LJ terms or exclusions: each atom's force is one pair's
+    direct Coulomb term but for ~1 %."""
+    rng = np.random.default_rng(12)
+    g = np.stack(np.meshgrid(*[np.arange(6)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    at = (g + 0.5) * (40.0 / 6.0)
+    d = rng.normal(0.0, 1.0, at.shape)
+    d *= rng.uniform(0.15, 0.3, (len(at), 1)) / np.linalg.norm(d, axis=1, keepdims=True)
+    crd = np.stack([at, at + d], 1).reshape(-1, 3).astype(np.float32)
+    base = system.small_random(len(crd), (40.0, 40.0, 40.0), seed=2, cutoff=10.0, skin=1.0, excl_frac=0.0,
+                               fft=(40, 40, 40))
+    q = np.repeat(rng.uniform(0.2, 0.8, len(at)), 2) * np.tile([1.0, -1.0], len(at)) * system.CHARGE_SCALE
+    return dataclasses.replace(base, crd=crd, charge=q.astype(np.float32), lj_A=np.zeros_like(base.lj_A),
+                               lj_B=np.zeros_like(base.lj_B))
+
+
+@pytest.mark.parametrize("kind", ["energy step", "batched step", "batched energy step"])
+def test_close_pairs(kind):
+    """The Coulomb factor of energy steps and of batched steps is the fitted
+    erfc (5.2e-7 at most): with the displacement's and the products' roundings
+    (rsq cubed 3.6e-7, four products 2.4e-7, three coordinates' sum 1.8e-7)
+    1.5e-6 of each atom's force at most, and 5e-7 in the mean square."""
+    import torch
+    from sponge_amd import nb
+    s = dimers()
+    say(f"[case] close pairs, {kind}")
+    eng = nb.NonbondedEngine(s, refresh_interval=20)
+    assert eng.shapes().as_dict()["prune_interval"] > 0
+    energy = 1 if "energy" in kind else 0
+    if "batched" in kind:
+        batch = nb.BatchedSystems([eng])
+        batch.neighbor_list_update(forced=1)
+        batch.force_step(energy, energy)
+    else:
+        eng.update_neighbor_list(forced=1)
+        eng.force_step(energy, energy, from_crd=True, overwrite=True)
+    torch.cuda.synchronize()
+    eng.nl.check()
+    ref = oracle.full_reference(s, crd=eng.crd.cpu().numpy(), beta=eng.pme.beta,
+                                K=(eng.pme.fftx, eng.pme.ffty, eng.pme.fftz))["frc"]
+    f = eng.frc.cpu().numpy().astype(np.float64)
+    err = np.linalg.norm(f - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    say(f"    worst {err.max():.2e}, mean square {np.sqrt((err ** 2).mean()):.2e}")
+    assert err.max() < 1.5e-6 and np.sqrt((err ** 2).mean()) < 5e-7
+
+
+def test_first_energy_step_inside_a_capture():
+    """A list update and one direct-force call prepare a handle for a captured
+    energy step: the step allocates nothing of its own."""
+    import torch
+    from sponge_amd import nb
+    s = system.config(0)
+    say("[case] first fused step an energy step, captured")
+    eng = nb.NonbondedEngine(s, refresh_interval=20)
+    eng.update_neighbor_list(forced=1)
+    eng.crd_to_uint()
+    eng.lj.LJ_Force_With_PME_Direct_Force(eng.uint_crd, eng.charge, eng.frc, eng.nl, eng.pme.beta)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        eng.force_step(1, 1, from_crd=True, overwrite=True, stream=torch.cuda.current_stream())
+    got = []
+    for _ in range(3):
+        eng.frc.fill_(float("nan"))
+        g.replay()
+        p = eng.energy_parts()
+        got.append((eng.frc.cpu().numpy().copy(), p))
+    eng.force_step(1, 1, from_crd=True, overwrite=True)
+    p = eng.energy_parts()
+    for f, q in got:
+        assert rel_rms(f, eng.frc.cpu().numpy()) < 1e-6
+        for k in ("lj", "direct", "correction", "reciprocal"):
+            assert abs(q[k] - p[k]) <= 1e-9 * max(1.0, abs(p[k])), k

@@ -756,6 +756,18 @@ static void launch(K kernel, int grid, int threads, size_t lds, hipStream_t s, h
     else kernel<<<grid, threads, lds, s>>>(args...);
 }
 
+// Asks for the dynamic LDS of an energy kernel whose blocks pass 64 KB with
+// their static LDS (24 KB at most): the LJ table of 60 types and more at a
+// usual beta, 97 KB with 64 types and every erfc row. The attribute is the
+// kernel's, the call host work: fine inside a capture.
+constexpr size_t kEnergyStaticLds = 24 * 1024;
+template <class K>
+static int energy_lds(K kernel, size_t bytes) {
+    if (bytes + kEnergyStaticLds > 64 * 1024)
+        SNB_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return SPONGE_NB_OK;
+}
+
 // Gather + pair kernel: forces added to d_frc (original order, may be NULL),
 // per-atom energies to the given arrays, FP64 totals to ps->acc.
 int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, float cutoff, const float* cof,
@@ -803,13 +815,18 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
         const int rows = erfc_rows(beta, cutoff);
         const EnergyOut out{atom_e, atom_v, atom_d};
         auto go = [&](auto kernel) {
-            kernel<<<dense_blocks(nl->ncl_cap), kDenseWaves * 64, lds + erfc_lds(rows), s>>>(
+            const size_t bytes = lds + erfc_lds(rows);
+            const int err = energy_lds(kernel, bytes);
+            if (err) return err;
+            kernel<<<dense_blocks(nl->ncl_cap), kDenseWaves * 64, bytes, s>>>(
                 nl->flags, nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0], cof[1], cof[2], rc2, beta, rows,
                 nl->s2o, out, ps->acc, sc);
+            SNB_CHECK_LAUNCH();
+            return SPONGE_NB_OK;
         };
-        if (nt <= 4) sc ? go(pair_energy_kernel<true, 2>) : go(pair_energy_kernel<false, 2>);
-        else sc ? go(pair_energy_kernel<true, 6>) : go(pair_energy_kernel<false, 6>);
-        SNB_CHECK_LAUNCH();
+        rc = nt <= 4 ? (sc ? go(pair_energy_kernel<true, 2>) : go(pair_energy_kernel<false, 2>))
+                     : (sc ? go(pair_energy_kernel<true, 6>) : go(pair_energy_kernel<false, 6>));
+        if (rc) return rc;
         if (!d_frc) return SPONGE_NB_OK;
     }
     // the per-slot force loop of force-only plain steps reads the Coulomb
@@ -988,11 +1005,17 @@ int snb_batch_pairs(sponge_batch* b, int energy, int overwrite, hipStream_t s) {
         for (int k = 0; k < b->nsys; k++) x = std::max(x, (double)b->h[k].pme.beta * b->h[k].lj.cutoff);
         const int rows = erfc_rows(x, 1.0);
         auto go = [&](auto kernel) {
-            kernel<<<grid, kPairWaves * 64, b->lds_pair + erfc_lds(rows), s>>>(b->d, b->map[kStPair], nmap, rows);
+            const size_t bytes = b->lds_pair + erfc_lds(rows);
+            const int err = energy_lds(kernel, bytes);
+            if (err) return err;
+            kernel<<<grid, kPairWaves * 64, bytes, s>>>(b->d, b->map[kStPair], nmap, rows);
+            SNB_CHECK_LAUNCH();
+            return SPONGE_NB_OK;
         };
-        if (b->max_nt <= 4) b->soft ? go(pair_energy_batch<true, 2>) : go(pair_energy_batch<false, 2>);
-        else b->soft ? go(pair_energy_batch<true, 6>) : go(pair_energy_batch<false, 6>);
-        SNB_CHECK_LAUNCH();
+        const int rc = b->max_nt <= 4
+                           ? (b->soft ? go(pair_energy_batch<true, 2>) : go(pair_energy_batch<false, 2>))
+                           : (b->soft ? go(pair_energy_batch<true, 6>) : go(pair_energy_batch<false, 6>));
+        if (rc) return rc;
     }
     auto go = [&](auto kernel) {
         kernel<<<grid, kPairWaves * 64, b->lds_pair, s>>>(b->d, b->map[kStPair], nmap, overwrite);

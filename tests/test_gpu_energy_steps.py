@@ -97,3 +97,52 @@ def test_first_energy_step_inside_a_capture():
         assert rel_rms(f, eng.frc.cpu().numpy()) < 1e-6
         for k in ("lj", "direct", "correction", "reciprocal"):
             assert abs(q[k] - p[k]) <= 1e-9 * max(1.0, abs(p[k])), k
+
+
+@pytest.mark.parametrize("tolerance", [1e-5, 1e-30])
+@pytest.mark.parametrize("batched", [False, True])
+def test_energies_of_64_types(tolerance, batched):
+    """The most LJ types a handle takes, with the erfc table of a usual beta
+    and with all its rows (beta * cutoff past 8): 75 and 97 KB of LDS a block
+    of the energy kernel. Totals are FP64 sums of FP64 terms: 1e-9 of the
+    terms' scale."""
+    import torch
+    from sponge_amd import nb
+    s = system.small_random(900, (20.0, 21.0, 22.0), seed=9, cutoff=6.0, skin=1.0, n_types=64, fft=(20, 20, 24))
+    # on a jittered lattice: no pair so close that it hides the others' terms
+    g = np.stack(np.meshgrid(np.arange(9), np.arange(10), np.arange(10), indexing="ij"), -1).reshape(-1, 3)
+    x = (g + 0.5) / (9.0, 10.0, 10.0) * s.box + np.random.default_rng(3).uniform(-0.3, 0.3, (900, 3))
+    s.crd = x.astype(np.float32)
+    s.pme_tolerance = tolerance
+    say(f"[case] 64 types, tolerance {tolerance}, batched {batched}")
+    eng = nb.NonbondedEngine(s, refresh_interval=0)
+    if batched:
+        batch = nb.BatchedSystems([eng])
+        batch.neighbor_list_update(forced=1)
+        batch.force_step(1, 1)
+    else:
+        eng.update_neighbor_list(forced=1)
+        eng.force_step(1, 1, from_crd=True, overwrite=True)
+    torch.cuda.synchronize()
+    eng.nl.check()
+    u = eng.uint_crd.cpu().numpy().view(np.uint32)
+    ref = oracle.direct(s, u, oracle.nl_brute(s, u), eng.pme.beta)
+    p = eng.energy_parts()
+    assert p["pairs_in"] == ref["n_in"]
+    direct = np.abs(ref["atom_direct"]).sum()
+    lj = np.abs(ref["atom_energy"] - ref["atom_direct"]).sum()
+    for k, v, scale in (("lj", ref["e_lj"], lj), ("direct", ref["e_direct"], direct)):
+        say(f"    beta * cutoff {eng.pme.beta * s.cutoff:.2f} {k} {v:.3e}: {abs(p[k] - v) / scale:.2e}")
+        assert abs(p[k] - v) <= 1e-9 * scale, (k, p[k], v)
+    if batched:
+        return
+    assert abs(eng.lj.Get_Energy(eng.nl, eng.uint_crd) - p["lrc"] - ref["e_lj"]) <= 1e-9 * lj
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        eng.force_step(1, 1, from_crd=True, overwrite=True, stream=torch.cuda.current_stream())
+    for _ in range(2):
+        eng.parts.zero_()
+        g.replay()
+        q = eng.energy_parts()
+        assert abs(q["lj"] - ref["e_lj"]) <= 1e-9 * lj and abs(q["direct"] - ref["e_direct"]) <= 1e-9 * direct
+        eng.force_step(0, 0, from_crd=True, overwrite=True)

@@ -251,7 +251,8 @@ int sponge_lj_soft_create(int atom_numbers, int atom_type_numbers_A, int atom_ty
  * pair-kernel launch of this module records the two hipEvent_t as its start
  * and end (hipExtLaunchKernel on the launch stream: the kernel's own times,
  * without the latency of marker packets around it), so a caller can time the
- * dominant kernel inside a timed region. Both events or neither; NULL events
+ * dominant kernel inside a timed region. A call with energies and forces is
+ * two launches: the start of the first and the end of the second. Both events or neither; NULL events
  * switch the hook off. Not for graph capture. */
 int sponge_lj_set_pair_events(sponge_lj* lj, void* start_event, void* stop_event);
 

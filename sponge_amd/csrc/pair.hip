@@ -748,11 +748,11 @@ void snb_scratch_free(PairScratch* ps) {
     ps->waves = waves;  // a setting, not storage
 }
 
-// A launch that records its own start and end times in two events when given.
+// A launch that records its own start and end times in the events given.
 template <class K, class... A>
 static void launch(K kernel, int grid, int threads, size_t lds, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
                    A... args) {
-    if (e0) hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), (std::uint32_t)lds, s, e0, e1, 0u, args...);
+    if (e0 || e1) hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), (std::uint32_t)lds, s, e0, e1, 0u, args...);
     else kernel<<<grid, threads, lds, s>>>(args...);
 }
 
@@ -805,9 +805,11 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
     }
     const float rc2 = cutoff * cutoff;
     size_t lds = (size_t)nt * nt * sizeof(float2);
-    // With timing events set, the launch itself records them (hipExtLaunchKernel
-    // takes the kernel's own start and end times; events recorded around a
-    // launch add the marker packets' latency, ~8 us per launch here)
+    // With timing events set, the launches themselves record them
+    // (hipExtLaunchKernel takes the kernel's own start and end times; events
+    // recorded around a launch add the marker packets' latency, ~8 us per
+    // launch here): the start of the call's first pair kernel and the end of
+    // its last one (energies first, then forces where asked for)
     const bool timed = ps->ev_start && ps->ev_stop;
     const hipEvent_t e0 = timed ? ps->ev_start : nullptr, e1 = timed ? ps->ev_stop : nullptr;
     const uint4* pk = ps->pk;
@@ -818,9 +820,9 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
             const size_t bytes = lds + erfc_lds(rows);
             const int err = energy_lds(kernel, bytes);
             if (err) return err;
-            kernel<<<dense_blocks(nl->ncl_cap), kDenseWaves * 64, bytes, s>>>(
-                nl->flags, nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0], cof[1], cof[2], rc2, beta, rows,
-                nl->s2o, out, ps->acc, sc);
+            launch(kernel, dense_blocks(nl->ncl_cap), kDenseWaves * 64, bytes, s, e0, d_frc ? nullptr : e1, nl->flags,
+                   nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0], cof[1], cof[2], rc2, beta, rows, nl->s2o,
+                   out, ps->acc, sc);
             SNB_CHECK_LAUNCH();
             return SPONGE_NB_OK;
         };
@@ -847,7 +849,7 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
     const int W = (!sc && (ps->waves == 2 || ps->waves == 8)) ? ps->waves : kPairWaves;
     const int grid = xcd_grid(ceil_div(nl->ncl_cap, W));
     auto go = [&](auto kernel) {
-        launch(kernel, grid, W * 64, lds, s, e0, e1, nl->flags, nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0],
+        launch(kernel, grid, W * 64, lds, s, energy ? nullptr : e0, e1, nl->flags, nl->list_n, nl->list, nl->list_cap, pk, ab, nt, cof[0],
                cof[1], cof[2], rc2, beta, nl->s2o, d_frc, overwrite, sc, pa, ex);
     };
     if (sc) nt <= 4 ? go(pair_kernel<true, 2>) : go(pair_kernel<true, 6>);

@@ -146,3 +146,38 @@ def test_energies_of_64_types(tolerance, batched):
         q = eng.energy_parts()
         assert abs(q["lj"] - ref["e_lj"]) <= 1e-9 * lj and abs(q["direct"] - ref["e_direct"]) <= 1e-9 * direct
         eng.force_step(0, 0, from_crd=True, overwrite=True)
+
+
+def test_pair_events_of_energy_calls():
+    """The pair events bracket every pair launch of a call: both kernels of an
+    energy step, the energy kernel alone where no forces are asked for. The
+    energy kernel takes longer than the force kernel (27 against 12 us for
+    6,591 atoms), so a step with both takes over 1.5 times a force-only one."""
+    import torch
+    from sponge_amd import nb
+    length = (2197 * system.WATER_VOLUME) ** (1.0 / 3.0)
+    s = system.water_box(2197, round(length, 3), seed=3, cutoff=9.0, skin=1.0, fft=(48, 48, 48))
+    say("[case] pair events", s.n)
+    eng = nb.NonbondedEngine(s, refresh_interval=20)
+    eng.update_neighbor_list(forced=1)
+
+    def timed(call):
+        call()
+        best = np.inf
+        for _ in range(5):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            for x in e:
+                x.record()
+            torch.cuda.synchronize()
+            eng.lj.set_pair_events(*e)
+            call()
+            eng.lj.set_pair_events()
+            torch.cuda.synchronize()
+            best = min(best, e[0].elapsed_time(e[1]) * 1e3)
+        return best
+
+    force = timed(lambda: eng.force_step(0, 0, from_crd=True, overwrite=True, serial=True))
+    both = timed(lambda: eng.force_step(1, 1, from_crd=True, overwrite=True, serial=True))
+    alone = timed(lambda: eng.lj.Get_Energy(eng.nl, eng.uint_crd))
+    say(f"    force {force:.1f} us, energies and forces {both:.1f}, energies alone {alone:.1f}")
+    assert both > 1.5 * force and alone > 0.6 * (both - force)

@@ -369,12 +369,13 @@ __device__ __forceinline__ float nl_dr2(uint4 a, uint4 b, float cx, float cy, fl
     return dr2_exact(dx, dy, dz);
 }
 
+// Whether the row of either atom names the other.
 __device__ __forceinline__ bool excluded_pair(int a, int b, const int* __restrict__ es,
                                               const int* __restrict__ en, const int* __restrict__ el) {
-    int lo = min(a, b), hi = max(a, b);
-    int s = es[lo], e = s + en[lo];
-    for (int k = s; k < e; k++)
-        if (el[k] == hi) return true;
+    for (int k = es[a], e = k + en[a]; k < e; k++)
+        if (el[k] == b) return true;
+    for (int k = es[b], e = k + en[b]; k < e; k++)
+        if (el[k] == a) return true;
     return false;
 }
 
@@ -399,8 +400,9 @@ __device__ __forceinline__ int wrap(int v, int n) { return v < 0 ? v + n : v >= 
 // has both conditions), takes the list's own FP32 expression nl_dr2. Each
 // exclusion partner of the i atoms (SYM: from the symmetric lists ex_a, ex_b;
 // else from the CSR's row and the reverse row of the counts ex_a and rows
-// ex_b) sets its bit in a mask on its cluster among the candidates; past kRevCap reverse partners the CSR is searched for
-// every pair in range.
+// ex_b) sets its bit in a mask on its cluster among the candidates; past
+// kRevCap reverse partners the CSR rows of both atoms are searched for every
+// pair in range.
 // Bound: latency of a wave's ~30 record loads and vector issue. Measured, 648 /
 // 4,446 / 10,013 / 23,570 / 96,120 atoms: 12 / 22 / 30 / 46 / 136 us against
 // 24 / 100 / 79 / 128 / 368 us with a box test of the candidates, one pair per

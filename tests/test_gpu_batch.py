@@ -250,3 +250,34 @@ def test_batch_forces_are_its_own_pme_beta(between):
         err = rel_rms(e.frc.cpu().numpy(), f)
         print(f"    {s.name}: {err:.2e}", flush=True)
         assert err < 1e-7, s.name
+
+
+def test_batched_exclusions_in_rows_of_the_higher_atom():
+    """The single-system list takes an excluded pair from the row of either of
+    its atoms; so does the batched one, by marks and (a solute of 40 mutually
+    excluded atoms: past the reverse rows' capacity) by searching the rows."""
+    import dataclasses
+    import torch
+    from sponge_amd import nb
+    s = system.fep_system(150, 0.3, seed=4, n_solute=40, cutoff=7.0, skin=1.0)
+    rows = [[] for _ in range(s.n)]
+    for a in range(s.n):
+        for p in s.excl_list[s.excl_start[a]:s.excl_start[a] + s.excl_numbers[a]]:
+            rows[int(p)].append(a)
+    numbers = np.array([len(r) for r in rows], np.int32)
+    t = dataclasses.replace(s, excl_numbers=numbers,
+                            excl_start=np.concatenate(([0], np.cumsum(numbers)[:-1])).astype(np.int32),
+                            excl_list=np.array([a for r in rows for a in r], np.int32))
+    print("[case] exclusions in the higher atom's row", t.n, flush=True)
+    got = []
+    for v in (s, t):
+        eng = nb.NonbondedEngine(v, refresh_interval=20)
+        batch = nb.BatchedSystems([eng])
+        batch.neighbor_list_update(forced=1)
+        batch.force_step(0, 0)
+        torch.cuda.synchronize()
+        eng.nl.check()
+        u = eng.uint_crd.cpu().numpy().view(np.uint32)
+        assert np.array_equal(eng.nl.pairs(), oracle.nl_brute(s, u))
+        got.append(eng.frc.cpu().numpy())
+    assert rel_rms(got[1], got[0]) < 1e-6

@@ -263,7 +263,7 @@ __device__ __forceinline__ void nl_sort_body(
     const int* __restrict__ col_atoms, const unsigned int* __restrict__ nl_uint,
     float crx, float cry, float crz, int* __restrict__ s2o, int* __restrict__ o2s,
     uint4* __restrict__ pack, float4* __restrict__ cl_lo, float4* __restrict__ cl_hi,
-    unsigned short* __restrict__ col_z, const int* flags, int* __restrict__ rev_n = nullptr,
+    unsigned short* __restrict__ col_z, const int* flags, int n = 0, int* __restrict__ rev_n = nullptr,
     int* __restrict__ rev = nullptr, const int* __restrict__ es = nullptr, const int* __restrict__ en = nullptr,
     const int* __restrict__ el = nullptr) {
     if (!flags[0]) return;
@@ -307,8 +307,11 @@ __device__ __forceinline__ void nl_sort_body(
             pack[slot] = make_uint4(nl_uint[3 * a], nl_uint[3 * a + 1], nl_uint[3 * a + 2], (unsigned)a);
             if (rev) {
                 // this atom into the reverse rows of its exclusion partners
+                // (an entry that names no atom, such as padding, is skipped)
                 for (int q = es[a]; q < es[a] + en[a]; q++) {
-                    const int p = el[q], at = atomicAdd(rev_n + p, 1);
+                    const int p = el[q];
+                    if ((unsigned)p >= (unsigned)n) continue;
+                    const int at = atomicAdd(rev_n + p, 1);
                     if (at < kRevCap) rev[(size_t)p * kRevCap + at] = a;
                 }
             }
@@ -415,7 +418,7 @@ __device__ __forceinline__ void nl_pairs_body(
     const int* __restrict__ o2s,
     const int* __restrict__ es, const int* __restrict__ en, const int* __restrict__ el, int list_cap,
     int* __restrict__ list_n, int* __restrict__ list_pairs, uint2* __restrict__ list, int* flags,
-    const int* __restrict__ ex_a, const int* __restrict__ ex_b) {
+    const int* __restrict__ ex_a, const int* __restrict__ ex_b, int natoms = 0) {
     if (!flags[0]) return;
     __shared__ uint2 cands[kPairWaves][kCandWindow];  // (j cluster, mask of excluded pairs)
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -451,7 +454,7 @@ __device__ __forceinline__ void nl_pairs_body(
         } else {
             back = ex_a[xatom];
             xrow = es[xatom];
-            xown = en[xatom];
+            xown = max(en[xatom], 0);
             xall = xown + min(back, kRevCap);
         }
     }
@@ -460,8 +463,12 @@ __device__ __forceinline__ void nl_pairs_body(
     auto partner = [&](int k, int& js, int& col) {
         js = -1;
         if (k >= xall) return;
-        if (SYM) js = o2s[ex_b[xrow + k]];
-        else js = o2s[k < xown ? el[xrow + k] : ex_b[(size_t)xatom * kRevCap + k - xown]];
+        if (SYM) {
+            js = o2s[ex_b[xrow + k]];
+        } else {
+            const int p = k < xown ? el[xrow + k] : ex_b[(size_t)xatom * kRevCap + k - xown];
+            if ((unsigned)p < (unsigned)natoms) js = o2s[p];
+        }
         if (js < 0) return;
         const uint4 b = pack[js];
         col = (int)(((unsigned long long)b.x * (unsigned)ncx) >> 32) * ncy +
@@ -771,7 +778,7 @@ __global__ __launch_bounds__(kSortThreads) void nl_sort_batch(const BatchSys* __
     if (m.x < 0) return;
     const sponge_nl& L = bs[m.x].nl;
     nl_sort_body(m.y, L.col_cap, L.col_count, L.col_start, L.col_atoms, L.nl_uint, L.cof_dr[0], L.cof_dr[1],
-                 L.cof_dr[2], L.s2o, L.o2s, L.pack, L.cl_lo, L.cl_hi, L.col_z, L.flags, L.rev_n, L.rev,
+                 L.cof_dr[2], L.s2o, L.o2s, L.pack, L.cl_lo, L.cl_hi, L.col_z, L.flags, L.n, L.rev_n, L.rev,
                  bs[m.x].io.excluded_list_start, bs[m.x].io.excluded_numbers, bs[m.x].io.excluded_list);
 }
 
@@ -785,7 +792,7 @@ __global__ __launch_bounds__(kPairWaves * 64) __attribute__((amdgpu_waves_per_eu
     const sponge_nl& L = b.nl;
     nl_pairs_body<false>(m.y, L.ncx, L.ncy, L.box[0], L.box[1], L.box[2], L.cof_dr[0], L.cof_dr[1], L.cof_dr[2], L.rl2,
                   b.rlm, L.col_start, L.col_z, L.cl_lo, L.cl_hi, L.pack, L.o2s, b.io.excluded_list_start, b.io.excluded_numbers, b.io.excluded_list,
-                  L.list_cap, L.list_n, L.list_pairs, L.list, L.flags, L.rev_n, L.rev);
+                  L.list_cap, L.list_n, L.list_pairs, L.list, L.flags, L.rev_n, L.rev, L.n);
 }
 
 __global__ __launch_bounds__(256) void nl_slot_lists_batch(const BatchSys* __restrict__ bs,

@@ -281,3 +281,35 @@ def test_batched_exclusions_in_rows_of_the_higher_atom():
         assert np.array_equal(eng.nl.pairs(), oracle.nl_brute(s, u))
         got.append(eng.frc.cpu().numpy())
     assert rel_rms(got[1], got[0]) < 1e-6
+
+
+def test_batched_rebuild_skips_partners_out_of_range():
+    """Entries of the exclusion list that name no atom (padding values) are
+    skipped by the batched rebuild: no pair is excluded by them, and nothing
+    is read or written for them. (Lists only: the force step's correction
+    needs a valid list.)"""
+    import dataclasses
+    import torch
+    from sponge_amd import nb
+    s = system.fep_system(150, 0.3, seed=4, n_solute=12, cutoff=7.0, skin=1.0)
+    eng = nb.NonbondedEngine(s, refresh_interval=20)
+    gone = np.arange(5, len(s.excl_list), 7)
+    bad = s.excl_list.copy()
+    bad[gone] = np.where(np.arange(len(gone)) % 2 == 0, -1, s.n + 7)
+    eng.excl_list.copy_(torch.as_tensor(bad, dtype=torch.int32))
+    print("[case] partners out of range", s.n, len(gone), flush=True)
+    batch = nb.BatchedSystems([eng])
+    batch.neighbor_list_update(forced=1)
+    eng.crd_to_uint()
+    torch.cuda.synchronize()
+    eng.nl.check()
+    u = eng.uint_crd.cpu().numpy().view(np.uint32)
+    keep = np.ones(len(bad), bool)
+    keep[gone] = False
+    owner = np.repeat(np.arange(s.n), s.excl_numbers)[keep]
+    numbers = np.bincount(owner, minlength=s.n).astype(np.int32)
+    t = dataclasses.replace(s, excl_numbers=numbers,
+                            excl_start=np.concatenate(([0], np.cumsum(numbers)[:-1])).astype(np.int32),
+                            excl_list=s.excl_list[keep])
+    assert np.array_equal(eng.nl.pairs(), oracle.nl_brute(t, u))
+    assert len(oracle.nl_brute(t, u)) > len(oracle.nl_brute(s, u))

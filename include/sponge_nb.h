@@ -98,15 +98,16 @@ int sponge_nl_set_exclusions(sponge_nl* nl, const int* d_excluded_list_start, co
                              const int* d_excluded_numbers);
 
 /* Inner list of the fused step (no counterpart in the reference);
- * prune_interval 0 turns it off (the cluster-pair list every step). Plain LJ
- * (force-only steps): each rebuild also writes the list's pairs per atom
- * (every pair within cutoff + skin at the rebuild, the reference's own
- * list) and the fused steps read them; with
+ * prune_interval 0 turns it off (the cluster-pair list every step). Plain LJ:
+ * each rebuild also writes the list's pairs per atom (every pair within
+ * cutoff + skin at the rebuild, the reference's own list) and the fused steps
+ * take their forces from them (energies come from the cluster-pair list); with
  * prune_radius >= cutoff + skin nothing else is pruned. With a smaller
  * prune_radius (>= cutoff) those per-atom lists are the outer ones: every
  * prune_interval fused steps an inner list keeps their pairs within
  * prune_radius of the current coordinates. Soft-core LJ prunes its
- * cluster-pair list to prune_radius on the same schedule. Between
+ * cluster-pair list to a prune_radius below cutoff + skin on the same
+ * schedule (with a larger one it reads the full list). Between
  * scheduled prunes of a distance-pruned list, a step at which some atom has
  * moved more than (prune_radius - cutoff) / 2 since the last prune prunes at
  * once (decided on the device), so the inner list never misses a pair
@@ -131,10 +132,10 @@ int sponge_nl_update_volume(sponge_nl* nl, const float box_length[3]);
 int sponge_nl_status(sponge_nl* nl, long* pair_count, int* overflow_flags, int* rebuilds);
 
 /* Synchronises. Diagnostics of the fused step's inner list (no counterpart in
- * the reference): with plain LJ, force-only fused steps read per-slot partner
- * lists pruned to the inner radius; `slot_overflow` = 1 when a slot had more
- * partners than those lists hold at a prune since the last rebuild (its
- * cluster then reads the full list), and `slot_launches` counts the
+ * the reference): with plain LJ, the forces of fused steps come from per-slot
+ * partner lists (pruned to the inner radius where that is below the list's);
+ * `slot_overflow` = 1 when a slot had more partners than those lists hold
+ * since the last rebuild (its cluster then reads the full list), and `slot_launches` counts the
  * pair-kernel launches that read the per-slot form since the list was
  * created. */
 int sponge_nl_inner_status(sponge_nl* nl, int* slot_overflow, int* slot_launches);

@@ -777,7 +777,7 @@ int snb_pairs(const sponge_nl* nl, const float2* ab, int nt, const int* d_type, 
     // the per-slot inner lists address records through 16-bit offsets,
     // which needs the record halo of an owned scratch
     const bool fused = inner != 0;
-    inner = inner && nl->prune_interval > 0 && ps->pk_alloc != nullptr;
+    inner = inner && nl->prune_interval > 0 && ps->pk_alloc != nullptr && (!sc || snb_two_level(nl));
     PruneArgs pa{};
     if (inner) {
         pa.interval = nl->prune_interval;
@@ -868,10 +868,7 @@ int snb_step_prep(const sponge_nl* nl, sponge_lj* lj, sponge_pme* pme, const flo
     for (int d = 0; d < 3; d++) cq[d] = 0.25f * (4294967296.0f / lj->box[d]);
     const int cap = lj->ps.cap;
     const bool prune = nl->prune_interval > 0;
-    // displacement votes: the per-slot lists of plain LJ prune by distance
-    // only in the two-level form (else they hold every pair of the full
-    // list); soft-core LJ prunes its cluster-pair inner list by distance
-    const bool vote = prune && (lj->d_sc != nullptr || snb_two_level(nl));
+    const bool vote = snb_two_level(nl);  // displacement votes
     step_prep_kernel<<<ceil_div(cap, 256), 256, 0, s>>>(nl->flags, nl->s2o, d_crd, cq[0], cq[1], cq[2], d_uint_crd,
                                                         d_charge, lj->d_type, lj->ps.pk, pme_prep_args(pme), energy,
                                                         lj->ps.acc, prune ? nl->flags + 10 : nullptr, nl->dropped,

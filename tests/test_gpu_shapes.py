@@ -135,3 +135,33 @@ def test_rebuild_lists_equal_the_pair_kernels(name):
         torch.cuda.synchronize()
         say(f"    radius {radius}: max |diff| {np.abs(f_rebuild - f_pair).max():.3e}")
         assert np.array_equal(f_rebuild, f_pair), radius
+
+
+def test_soft_core_lists_pruned_only_below_the_list_radius():
+    """With a prune radius of cutoff + skin (the tuned table's) the cluster
+    list of a soft-core handle holds the same pairs before and after a prune:
+    no step prunes, and an atom that moves half the skin and more votes for
+    nothing. A smaller radius prunes as asked."""
+    import torch
+    from sponge_amd import nb
+    s = system.fep_system(150, 0.3, seed=4, cutoff=7.0, skin=2.0)
+    eng = nb.NonbondedEngine(s, refresh_interval=20)
+    sh = eng.shapes().as_dict()
+    assert sh["prune_interval"] > 0 and sh["prune_radius"] == s.cutoff + s.skin
+    say(f"[case] soft-core prune rule n={s.n}")
+    got = {}
+    for radius in (float(s.cutoff + s.skin), float(s.cutoff) + 0.5 * float(s.skin), None):
+        eng.crd.copy_(torch.as_tensor(s.crd))
+        if radius is None:
+            eng.nl.set_prune(0)
+        else:
+            eng.nl.set_prune(20, radius)
+        eng.update_neighbor_list(forced=1)
+        steps(eng, 2)
+        v0 = eng.nl.prune_votes()
+        eng.crd[0, 0] += 0.6 * s.skin
+        got[radius] = steps(eng, 1).astype(np.float64)
+        assert eng.nl.prune_votes() - v0 == (1 if radius and radius < s.cutoff + s.skin else 0), radius
+    ref = got.pop(None)
+    for f in got.values():
+        np.testing.assert_allclose(f, ref, rtol=0, atol=1e-5 * float(np.abs(ref).max()))

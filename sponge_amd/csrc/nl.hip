@@ -7,7 +7,7 @@
 // Here atoms are counting-sorted into xy columns, z-sorted inside each column
 // and cut into clusters of 4; the list holds, per i-cluster, every j-cluster
 // (both directions, so each unordered cluster pair appears twice and the pair
-// kernel needs no atomics) whose bounding box comes within rc+skin, each with
+// kernel needs no atomics) with an atom pair within rc+skin, each with
 // a 16-bit mask whose bit (jj*4+ii) is set exactly when the reference would
 // list that atom pair: the same FP32 dr2 expression, the same strict
 // comparison, minus exclusions and padding. The set of listed unordered atom
@@ -607,7 +607,7 @@ __device__ __forceinline__ void nl_pairs_body(
                         in |= nl_dr2(pack[ic * kClusterSize + i], b, crx, cry, crz) < rl2 ? 1u << i : 0u;
                 }
                 in &= ok;
-                if (!marked) {
+                if (!SYM && !marked) {
 #pragma unroll
                     for (int i = 0; i < kClusterSize; i++)
                         if ((in >> i) & 1u)
@@ -649,12 +649,11 @@ __global__ __launch_bounds__(kPairWaves * 64) __attribute__((amdgpu_waves_per_eu
     int ncx, int ncy, float bx, float by, float bz, float crx, float cry, float crz, float rl2,
     float rlm, const int* __restrict__ col_start, const unsigned short* __restrict__ col_z,
     const float4* __restrict__ cl_lo, const float4* __restrict__ cl_hi, const uint4* __restrict__ pack,
-    const int* __restrict__ o2s,
-    const int* __restrict__ es, const int* __restrict__ en, const int* __restrict__ el, int list_cap,
-    int* __restrict__ list_n, int* __restrict__ list_pairs, uint2* __restrict__ list, int* flags,
-    const int* __restrict__ sym_start, const int* __restrict__ sym_list) {
-    nl_pairs_body<true>(xcd_block(gridDim.x), ncx, ncy, bx, by, bz, crx, cry, crz, rl2, rlm, col_start, col_z, cl_lo, cl_hi,
-                  pack, o2s, es, en, el, list_cap, list_n, list_pairs, list, flags, sym_start, sym_list);
+    const int* __restrict__ o2s, int list_cap, int* __restrict__ list_n, int* __restrict__ list_pairs,
+    uint2* __restrict__ list, int* flags, const int* __restrict__ sym_start, const int* __restrict__ sym_list) {
+    nl_pairs_body<true>(xcd_block(gridDim.x), ncx, ncy, bx, by, bz, crx, cry, crz, rl2, rlm, col_start, col_z, cl_lo,
+                        cl_hi, pack, o2s, nullptr, nullptr, nullptr, list_cap, list_n, list_pairs, list, flags,
+                        sym_start, sym_list);
 }
 
 // Per-slot lists of the fused step from the stored list (plain LJ, inner list
@@ -989,8 +988,7 @@ float snb_nl_rlm(const sponge_nl* nl) { return std::sqrt(nl->rl2) + 1.0e-3f * (1
 
 // Launches the rebuild pipeline; `forced` latches the decision on the host,
 // otherwise the device flag written by nl_check_kernel decides.
-static int nl_rebuild(sponge_nl* nl, float* d_crd, const int* es, const int* el, const int* en, int forced,
-                      hipStream_t s) {
+static int nl_rebuild(sponge_nl* nl, float* d_crd, int forced, hipStream_t s) {
     const int n = nl->n;
     nl_begin_kernel<<<1, 256, 0, s>>>(forced, nl->flags, nl->col_count, nl->ncol);
     SNB_CHECK_LAUNCH();
@@ -1016,7 +1014,7 @@ static int nl_rebuild(sponge_nl* nl, float* d_crd, const int* es, const int* el,
     int nblk = xcd_grid(ceil_div(nl->ncl_cap, kPairWaves));
     nl_pairs_kernel<<<nblk, kPairWaves * 64, 0, s>>>(
         nl->ncx, nl->ncy, nl->box[0], nl->box[1], nl->box[2], nl->cof_dr[0], nl->cof_dr[1], nl->cof_dr[2], nl->rl2,
-        rlm, nl->col_start, nl->col_z, nl->cl_lo, nl->cl_hi, nl->pack, nl->o2s, es, en, el, nl->list_cap, nl->list_n,
+        rlm, nl->col_start, nl->col_z, nl->cl_lo, nl->cl_hi, nl->pack, nl->o2s, nl->list_cap, nl->list_n,
         nl->list_pairs, nl->list, nl->flags, nl->sym_start, nl->sym_list);
     SNB_CHECK_LAUNCH();
     if (nl->prune_interval > 0) {
@@ -1095,12 +1093,12 @@ extern "C" int sponge_nl_update(sponge_nl* nl, float* d_crd, const int* d_exclud
         if (rc) return rc;
     }
     if (forced_update) {
-        return nl_rebuild(nl, d_crd, d_excluded_list_start, d_excluded_list, d_excluded_numbers, 1, s);
+        return nl_rebuild(nl, d_crd, 1, s);
     }
     if (nl->refresh_interval > 0 && !forced_check) {
         int rc = SPONGE_NB_OK;
         if (nl->refresh_count % nl->refresh_interval == 0)
-            rc = nl_rebuild(nl, d_crd, d_excluded_list_start, d_excluded_list, d_excluded_numbers, 1, s);
+            rc = nl_rebuild(nl, d_crd, 1, s);
         nl->refresh_count += 1;
         return rc;
     }
@@ -1108,7 +1106,7 @@ extern "C" int sponge_nl_update(sponge_nl* nl, float* d_crd, const int* d_exclud
     nl_check_kernel<<<ceil_div(nl->n, 256), 256, 0, s>>>(nl->n, d_crd, nl->old_crd, nl->box[0], nl->box[1],
                                                          nl->box[2], thresh, nl->flags);
     SNB_CHECK_LAUNCH();
-    return nl_rebuild(nl, d_crd, d_excluded_list_start, d_excluded_list, d_excluded_numbers, 0, s);
+    return nl_rebuild(nl, d_crd, 0, s);
 }
 
 extern "C" int sponge_nl_set_exclusions(sponge_nl* nl, const int* d_excluded_list_start, const int* d_excluded_list,

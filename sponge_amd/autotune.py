@@ -181,8 +181,7 @@ def write_table(winners, path=TABLE_PATH):
     txt = open(TABLE_PATH).read()
     head = txt[:txt.index("constexpr TuneRow kTuneTable[] = {")]
     tail = txt[txt.index("// clang-format on"):]
-    new = head + "constexpr TuneRow kTuneTable[] = {\n    // generated by sponge_amd/autotune.py\n" + \
-        "\n".join(lines) + "\n};\n" + tail
+    new = head + "constexpr TuneRow kTuneTable[] = {\n" + "\n".join(lines) + "\n};\n" + tail
     with open(path, "w") as f:
         f.write(new)
 

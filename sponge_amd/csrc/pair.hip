@@ -194,8 +194,8 @@ __global__ __launch_bounds__(256) void step_prep_batch(const BatchSys* __restric
 
 
 
-// Force-only steps. W: i-clusters (waves) per block; the plain-LJ launch
-// takes the handle's tuned value (2, 4 or 8), every other launch 4. The
+// Forces (of energy steps too). W: i-clusters (waves) per block; the plain-LJ
+// launch takes the handle's tuned value (2, 4 or 8), every other launch 4. The
 // plain kernels are held to 64 VGPRs (8 waves per SIMD): the per-slot force
 // loops wait on gathered slot records, which the other waves cover; the
 // filtering loop of the two-level lists would take 66 (two registers are

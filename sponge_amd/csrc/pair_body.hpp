@@ -254,16 +254,16 @@ __device__ __forceinline__ void slot_finish(int islot, int k, const uint4* __res
     }
 }
 
-// Force-only steps of plain LJ from the per-slot lists: lane (i, k),
-// i = lane >> 4, takes partners 2k and 2k + 1 of every 32 of atom i of the
-// wave's cluster (n of them; nmax the longest of the four lists) from one
-// dword of two 16-bit slot offsets, so every lane holds listed pairs (the
-// cluster form evaluates all 16 pairs of each listed cluster pair, in cutoff
-// or not). A dword of offsets is fetched two rounds ahead and the first
-// record of a round one round ahead.
-// Lanes past the end of a list read a record
-// too (offsets left from earlier prunes, or zero: always inside the records
-// and their copies) and are masked out.
+// Forces from the per-slot lists (plain LJ, and any handle in a batch; TABLE on
+// force-only steps of single systems): lane (i, k), i = lane >> 4, takes
+// partners 2k and 2k + 1 of every 32 of atom i of the wave's cluster (n of
+// them; nmax the longest of the four lists) from one dword of two 16-bit slot
+// offsets, so every lane holds listed pairs (the cluster form evaluates all 16
+// pairs of each listed cluster pair, in cutoff or not). A dword of offsets is
+// fetched two rounds ahead and the first record of a round one round ahead.
+// Lanes past the end of a list read a record too (offsets left from earlier
+// prunes, or zero: always inside the records and their copies) and are masked
+// out.
 template <int TB, bool TABLE, bool SOFT = false>
 __device__ __forceinline__ void pair_atoms(int ic, const unsigned short* __restrict__ lists, int n, int nmax,
                                            const uint4* __restrict__ pk, const float2* sab, const float4* stab,
@@ -414,7 +414,7 @@ __device__ __forceinline__ int longest(int n) {
     return max(max(__shfl(n, 0), __shfl(n, 16)), max(__shfl(n, 32), __shfl(n, 48)));
 }
 
-// Force-only steps: one i-cluster per wave.
+// Forces of a step: one i-cluster per wave.
 // Cutoff test shared with the oracle: FP32 dr2 = (dx*dx + dy*dy) + dz*dz with
 // every operation rounded (the neighbor list's expression) against rc*rc in
 // FP32, so both sides agree on every pair, including those within one ulp of
@@ -574,7 +574,7 @@ __device__ __forceinline__ void pair_wave(
     }
 }
 
-// One block of the force-only pair kernel: the LJ (A, B) table and, when
+// One block of the force kernel: the LJ (A, B) table and, when
 // given, the Coulomb table into LDS, then one i-cluster per wave (logical
 // block lb covers clusters W lb .. W lb + W - 1).
 template <bool SOFT, int TB, int W = kPairWaves, bool BATCH = false>
@@ -599,7 +599,7 @@ __device__ __forceinline__ void pair_body(
 }
 
 // ---- energy steps -----------------------------------------------------------
-// Forces come from the force-only kernel (with the lists it reads or writes);
+// Forces come from the force kernel (with the lists it reads or writes);
 // the energies of every pair of the full list from energy_wave.
 
 // Sums of an energy step: the FP32 per-atom energies of lane (i, k)'s pairs

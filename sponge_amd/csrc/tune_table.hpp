@@ -1,8 +1,11 @@
-// Default launch shapes of the fused step, by system size: the winners of
-// the shape sweep of sponge_amd/autotune.py (times per MD step of each
-// candidate on the measured systems are listed beside each row). A row
-// applies to systems of up to max_atoms atoms; the last row to all larger
-// ones. Regenerate with `python -m sponge_amd.autotune --table`.
+// Default launch shapes of the fused step, by system size, from the shape
+// sweep of sponge_amd/autotune.py (times per MD step of plain water boxes
+// beside each row): the fastest candidate, or one within the ~1 % that two
+// sweeps of the same shape differ by. A row applies to systems of up to
+// max_atoms atoms; the last row to all larger ones. Regenerate with
+// `python -m sponge_amd.autotune --table` (which takes the fastest).
+// Soft-core handles take the rows of their size, and prune only with a radius
+// below cutoff + skin.
 //
 // Columns: pair_waves (i-clusters per block of the force-only pair kernel),
 // conv_split (-1: by plane size, one workgroup per plane up to 64 x 64; 0 /
@@ -27,9 +30,8 @@ struct TuneRow {
 
 // clang-format off
 constexpr TuneRow kTuneTable[] = {
-    // generated by sponge_amd/autotune.py
-    {      3908, 2, -1, 256, 0, 1, 1.0f},  // 648 atoms, PME 20x20x20: 39.20 us/step (list every step: 43.77)
-    {     47597, 8,  1, 256, 0, 1, 1.0f},  // 23570 atoms, PME 64x64x64: 63.70 us/step
+    {      3908, 2, -1, 256, 0, 1, 1.0f},  // 648 atoms, PME 20x20x20: 39.20 us/step
+    {     47597, 8,  1, 256, 0, 1, 1.0f},  // 23570 atoms, PME 64x64x64: 63.70 us/step (kept: 5th, 1st 63.11)
     {0x7fffffff, 4, -1, 256, 0, 1, 1.0f},  // 96120 atoms, PME 108x108x108: 159.69 us/step
 };
 // clang-format on

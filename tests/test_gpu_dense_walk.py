@@ -27,7 +27,8 @@ CASES = [
     (216, 8.0, 1.0, None),    # 18.6 A box: cutoff + a cluster's extent passes half of it
     (216, 9.2, 0.1, None),    # cutoff at half the box
     (343, 5.0, 0.5, 1.7),     # beta * cutoff 8.5: past the table's end
-    (343, 5.0, 0.5, 0.02),    # one or two rows
+    (343, 5.0, 0.5, 0.02),    # 8 rows
+    (343, 5.0, 0.5, 0.002),   # the fewest: 2 rows
     (2197, 9.0, 2.0, None),
 ]
 

@@ -759,12 +759,14 @@ static void launch(K kernel, int grid, int threads, size_t lds, hipStream_t s, h
 // Asks for the dynamic LDS of an energy kernel whose blocks pass 64 KB with
 // their static LDS (24 KB at most): the LJ table of 60 types and more at a
 // usual beta, 97 KB with 64 types and every erfc row. The attribute is the
-// kernel's, the call host work: fine inside a capture.
+// kernel's, so it is always set to the most a call can need: calls of several
+// threads agree. Host work, fine inside a capture.
 constexpr size_t kEnergyStaticLds = 24 * 1024;
 template <class K>
 static int energy_lds(K kernel, size_t bytes) {
+    const size_t most = erfc_lds(kErfcMaxRows) + (size_t)kMaxLjTypes * kMaxLjTypes * sizeof(float2);
     if (bytes + kEnergyStaticLds > 64 * 1024)
-        SNB_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+        SNB_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
     return SPONGE_NB_OK;
 }
 
